@@ -27,31 +27,52 @@ __device__ __forceinline__ float frame_value(float I, int m, bool has_mask, floa
     return v;
 }
 
+// Frames a thread reads ahead of its chain of adds.
+constexpr uint32_t kAhead = 8;
+
 // One thread per pixel, frames in order: adds to the float sum (ParAdd with
 // threshold) or to the long photon tally; calls over consecutive frame stacks
-// continue the same per-pixel sequence.
+// continue the same per-pixel sequence.  avg != null: the stack is the whole run, the
+// sequence starts at zero and ends as finish_kernel ends it (no accumulator in memory).
+// HBM bound; kAhead loads are in flight per thread, since a stack of few pixels holds few
+// waves per SIMD (200 frames of 517 x 512, 212 MB: 84 us one
+// load at a time, 32 us this way, the frames partly still in the last-level cache).
+template <bool kPhotons>
 __global__ void __launch_bounds__(256)
     accumulate_pixels_kernel(const float *__restrict__ frames, uint32_t nframes, uint32_t npix,
                              const int *__restrict__ mask, float T, float S, float *__restrict__ sum,
-                             long long *__restrict__ tally)
+                             long long *__restrict__ tally, float *__restrict__ avg)
 {
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= npix) return;
     const int m = mask ? mask[j] : 1;
-    if (S > 0) {
-        long long acc = tally[j];
-        for (uint32_t f = 0; f < nframes; f++) {
-            const float v = frame_value(frames[(size_t)f * npix + j], m, mask != nullptr, T, S);
-            if (v != 0.0f) acc += (long long)floor((double)v + 0.5);
+    long long n = 0;
+    float s = 0.0f;
+    if (!avg) {
+        if (kPhotons) n = tally[j]; else s = sum[j];
+    }
+    auto add = [&](float I) {
+        const float v = frame_value(I, m, mask != nullptr, T, kPhotons ? S : 0.0f);
+        if (kPhotons) {
+            if (v != 0.0f) n += (long long)floor((double)v + 0.5);
+        } else {
+            if (v >= T) s += v;
         }
-        tally[j] = acc;
+    };
+    const float *p = frames + j;
+    uint32_t f = 0;
+    for (; f + kAhead <= nframes; f += kAhead) {
+        float I[kAhead];
+#pragma unroll
+        for (uint32_t k = 0; k < kAhead; k++) I[k] = p[(size_t)(f + k) * npix];
+#pragma unroll
+        for (uint32_t k = 0; k < kAhead; k++) add(I[k]);
+    }
+    for (; f < nframes; f++) add(p[(size_t)f * npix]);
+    if (avg) {
+        avg[j] = (kPhotons ? (float)n : s) * (1.0f / (float)nframes);
     } else {
-        float acc = sum[j];
-        for (uint32_t f = 0; f < nframes; f++) {
-            const float v = frame_value(frames[(size_t)f * npix + j], m, mask != nullptr, T, S);
-            if (v >= T) acc += v;
-        }
-        sum[j] = acc;
+        if (kPhotons) tally[j] = n; else sum[j] = s;
     }
 }
 
@@ -65,20 +86,42 @@ __global__ void finish_kernel(uint32_t npix, uint32_t ntotal, float S, const flo
     avg[j] = v * (1.0f / (float)ntotal);
 }
 
-// One wave per frame: ArrayOperators::Sum<float> (IAC/ArrayOperators.h:260-268) of the frame's
+// One block per frame: ArrayOperators::Sum<float> (IAC/ArrayOperators.h:260-268) of the frame's
 // values, a serial float sum in pixel order; MeanIntensity = sum / P and, with photon
 // discretisation, PhotonCount = (int) sum.
-__global__ void __launch_bounds__(iac::kSumWave)
+template <bool kMask, bool kPhotons>
+__global__ void __launch_bounds__(iac::kSumThreads)
     frame_sums_kernel(const float *__restrict__ frames, uint32_t npix, const int *__restrict__ mask, float T, float S,
                       float *__restrict__ mean_intensity, int *__restrict__ photon_count)
 {
+    __shared__ iac::SerialSumShared sh;
     const uint32_t f = blockIdx.x;
-    const float s = iac::serial_sum_wave(frames + (size_t)f * npix, npix, [=](uint32_t j, float v) {
-        return frame_value(v, mask ? mask[j] : 1, mask != nullptr, T, S);
-    });
+    const float s = iac::serial_sum_block<kMask>(
+        frames + (size_t)f * npix, mask, npix, sh,
+        [=](float v, int m) { return frame_value(v, m, kMask, T, kPhotons ? S : 0.0f); });
     if (threadIdx.x != 0) return;
     if (mean_intensity) mean_intensity[f] = s / (float)npix;
-    if (photon_count && S > 0) photon_count[f] = iac::cvtt_i32(s);
+    if (photon_count && kPhotons) photon_count[f] = iac::cvtt_i32(s);
+}
+
+// A stack's frame sums, then its pixel sequences (into d_avg, or the accumulators).
+int accumulate_stack(iac_ctx *ctx, const float *d_frames, uint32_t nframes, uint32_t npix, const int *d_mask, float T,
+                     float S, float *d_sum, int64_t *d_tally, float *d_avg, float *d_mean_intensity,
+                     int *d_photon_count)
+{
+    if (d_mean_intensity || d_photon_count) {
+        if (nframes > 0x7fffffffu) return iac::fail(IAC_ERR_LIMIT, "too many frames in one stack");
+        auto sums = S > 0 ? (d_mask ? frame_sums_kernel<true, true> : frame_sums_kernel<false, true>)
+                          : (d_mask ? frame_sums_kernel<true, false> : frame_sums_kernel<false, false>);
+        hipLaunchKernelGGL(sums, dim3(nframes), dim3(iac::kSumThreads), 0, ctx->stream, d_frames, npix,
+                           d_mask, T, S, d_mean_intensity, d_photon_count);
+        IAC_HIP(hipGetLastError());
+    }
+    auto kern = S > 0 ? accumulate_pixels_kernel<true> : accumulate_pixels_kernel<false>;
+    hipLaunchKernelGGL(kern, dim3((npix + 255) / 256), dim3(256), 0, ctx->stream, d_frames, nframes, npix, d_mask, T, S,
+                       d_sum, reinterpret_cast<long long *>(d_tally), d_avg);
+    IAC_HIP(hipGetLastError());
+    return IAC_OK;
 }
 
 }  // namespace
@@ -93,16 +136,8 @@ int iac_intensity_accumulate(iac_ctx *ctx, const float *d_frames, uint32_t nfram
     if (!d_frames || npix == 0) return iac::fail(IAC_ERR_INVALID_ARG, "bad averaging request");
     if (step > 0 ? !d_tally : !d_sum) return iac::fail(IAC_ERR_INVALID_ARG, "missing accumulator");
     if (nframes == 0) return IAC_OK;
-    hipLaunchKernelGGL(accumulate_pixels_kernel, dim3((npix + 255) / 256), dim3(256), 0, ctx->stream, d_frames,
-                       nframes, npix, d_mask, threshold, step, d_sum, reinterpret_cast<long long *>(d_tally));
-    IAC_HIP(hipGetLastError());
-    if (d_mean_intensity || d_photon_count) {
-        if (nframes > 0x7fffffffu) return iac::fail(IAC_ERR_LIMIT, "too many frames in one stack");
-        hipLaunchKernelGGL(frame_sums_kernel, dim3(nframes), dim3(iac::kSumWave), 0, ctx->stream, d_frames, npix,
-                           d_mask, threshold, step, d_mean_intensity, d_photon_count);
-        IAC_HIP(hipGetLastError());
-    }
-    return IAC_OK;
+    return accumulate_stack(ctx, d_frames, nframes, npix, d_mask, threshold, step, d_sum, d_tally, nullptr,
+                            d_mean_intensity, d_photon_count);
 }
 
 int iac_intensity_finish(iac_ctx *ctx, uint32_t npix, uint32_t ntotal_frames, float step, const float *d_sum,
@@ -124,14 +159,8 @@ int iac_average_intensity(iac_ctx *ctx, const float *d_frames, uint32_t nframes,
     IAC_TRY(iac::bind(ctx));
     if (!d_frames || !d_avg || npix == 0) return iac::fail(IAC_ERR_INVALID_ARG, "bad averaging request");
     if (nframes == 0) return iac::fail(IAC_ERR_PRECONDITION, "event list is empty, nothing to average");
-    void *acc = nullptr;
-    IAC_TRY(iac::scratch(ctx, 0, (size_t)npix * 8, &acc));
-    IAC_HIP(hipMemsetAsync(acc, 0, (size_t)npix * 8, ctx->stream));
-    float *sum = step > 0 ? nullptr : static_cast<float *>(acc);
-    int64_t *tally = step > 0 ? static_cast<int64_t *>(acc) : nullptr;
-    IAC_TRY(iac_intensity_accumulate(ctx, d_frames, nframes, npix, d_mask, threshold, step, sum, tally,
-                                     d_mean_intensity, d_photon_count));
-    return iac_intensity_finish(ctx, npix, nframes, step, sum, tally, d_avg);
+    return accumulate_stack(ctx, d_frames, nframes, npix, d_mask, threshold, step, nullptr, nullptr, d_avg,
+                            d_mean_intensity, d_photon_count);
 }
 
 }  // extern "C"

@@ -368,15 +368,17 @@ __global__ void zero_acc_kernel(FrameAcc *acc, uint32_t n)
 
 // Pass 2: PhotonCount = (int) of the frame sum and MeanIntensity = (float)PhotonCount /
 // (float)npix (IAC/PPP.cpp:490-491); the exact integer sum where it holds, else the serial float
-// sum.  One wave per frame.
-__global__ void __launch_bounds__(iac::kSumWave)
+// sum.  One block per frame.
+__global__ void __launch_bounds__(iac::kSumThreads)
     photon_count_kernel(const float *__restrict__ frames, uint32_t npix, const FrameAcc *__restrict__ acc,
                         int *__restrict__ count, float *__restrict__ mean)
 {
     const uint32_t f = blockIdx.x;
     const bool exact = !acc[f].bad && acc[f].mag <= (1ull << 24);
+    __shared__ iac::SerialSumShared sh;
     const float s = exact ? (float)acc[f].sum
-                          : iac::serial_sum_wave(frames + (size_t)f * npix, npix, [](uint32_t, float v) { return v; });
+                          : iac::serial_sum_block<false>(frames + (size_t)f * npix, nullptr, npix, sh,
+                                                         [](float v, int) { return v; });
     if (threadIdx.x != 0) return;
     const int pc = iac::cvtt_i32(s);
     if (count) count[f] = pc;
@@ -489,7 +491,7 @@ int iac_ppp_lap(iac_ctx *ctx, const float *d_in, float *d_out, uint32_t nframes,
     }
     IAC_TRY(iac::timer_end(ctx));
     if (acc) {
-        hipLaunchKernelGGL(photon_count_kernel, dim3(nframes), dim3(iac::kSumWave), 0, ctx->stream, d_out, npix, acc,
+        hipLaunchKernelGGL(photon_count_kernel, dim3(nframes), dim3(iac::kSumThreads), 0, ctx->stream, d_out, npix, acc,
                            d_photon_count, d_mean_intensity);
         IAC_HIP(hipGetLastError());
     }
