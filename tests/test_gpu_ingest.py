@@ -72,3 +72,27 @@ def test_average_over_frame_counts(ctx, dev, nframes, thr, step):
     assert np.array_equal(g_mi.cpu().numpy().view(np.int32), mi.view(np.int32))
     if step > 0:
         assert np.array_equal(g_pc.cpu().numpy(), pc)
+
+
+@pytest.mark.parametrize("npix,nframes", [(1, 3), (63, 2), (65, 5), (2048, 3), (2049, 2), (33000, 2), (16385, 300)])
+@pytest.mark.parametrize("fill", [0.0, 0.02, 1.0])
+def test_hit_lists_at_slice_edges(ctx, dev, npix, nframes, fill):
+    import torch
+
+    rng = np.random.default_rng(npix + nframes)
+    fr = np.where(rng.random((nframes, npix)) < fill, rng.random((nframes, npix)) * 5 + 0.6, -1).astype(np.float32)
+    if fill > 0:
+        fr[:, -1] = 2.5  # the last pixel
+        fr[-1, 0] = 0.5  # the threshold itself
+    km = rng.normal(size=(npix, 3)).astype(np.float32)
+    mask = (rng.random(npix) > 0.1).astype(np.int32)
+    rec = torch.zeros((nframes * npix, 4), device=dev)
+    off = torch.zeros(nframes + 1, dtype=torch.int64, device=dev)
+    for m in (None, mask):
+        n = ctx.sparse_hit_list(torch.from_numpy(km).to(dev), torch.from_numpy(fr).to(dev),
+                                None if m is None else torch.from_numpy(m).to(dev), 0.5, 0.7, rec, off)
+        ref = [O.sparse_hit_list(f, km, 0.5, 0.7, np.ones(npix, np.int32) if m is None else m) for f in fr]
+        assert n == sum(len(r) for r in ref)
+        assert np.array_equal(off.cpu().numpy(), np.cumsum([0] + [len(r) for r in ref]))
+        want = np.concatenate([np.asarray(r, np.float32).reshape(-1, 4) for r in ref])
+        assert np.array_equal(rec[:n].cpu().numpy().view(np.int32), want.view(np.int32))
