@@ -39,62 +39,285 @@ __global__ void u64_to_f64_kernel(const unsigned long long *__restrict__ in, siz
         out[i] = (double)in[i] / mult;
 }
 
-// Merge_CQ: small voxel `ind` (blockIdx.x * blockDim.x + threadIdx.x) rotated
-// by the events [e0, e1) of this block row.  Row-major rotation, nearest or
-// linear binning into the cubic big mesh whose slow-scan index also uses the
-// AB centre (kernel.cl:287).
-__global__ void merge_cq_kernel(const double *__restrict__ small, size_t small_stride, int sab, int sc, int ka,
-                                int kb, int kc, const float *__restrict__ rw, uint32_t nev, uint32_t ev_per_row,
-                                int interp, double mult, unsigned long long *__restrict__ big,
-                                unsigned long long *__restrict__ dropped)
+// ---- Merge_CQ ------------------------------------------------------------------------
+// Every small-mesh voxel, rotated by every event, adds to the cubic big mesh (its slow-scan index
+// uses size_ab's centre too).  A scattered add is one L2 atomic request (2.4e10/s, 1,656 us for
+// 1,000 events of a 129 x 129 x 3 mesh), so the big mesh is cut into bricks held in LDS: a block
+// takes a brick and a slice of the events, finds per event the small voxels that can reach the
+// brick (the brick turned back by the transposed matrix), bins exactly those and flushes the
+// brick with contiguous adds: 284 us and 42 us for the rest.  Bound: VALU issue, most of it for
+// the rows of candidates, whose 54 updates per brick and event lie in about 50 rows.  Other bricks
+// and events per block measured (whole call, 315 us): 16 x 8 x 8 with 32, 128 or 256 events 340,
+// 326, 378 us; 16 x 16 x 16 with 128 events 358; 16 x 8 x 4 459; the z rows of a y row in one
+// thread 353 (rows of unequal length side by side).
+// The transposed matrix is the inverse only of a rotation.  Events whose matrix is not
+// orthonormal to kOrtho, and the count of updates that leave the mesh (voxels near or beyond its
+// inscribed sphere), go through merge_rest_kernel.
+
+constexpr float kOrtho = 1e-4f;               // largest |(R^T R - 1)_ij| the bricks take
+constexpr int kBrX = 16, kBrY = 8, kBrZ = 8;  // 8 KB: 16 voxels are two 64-byte segments to flush
+constexpr int kBrick = kBrX * kBrY * kBrZ;
+constexpr uint32_t kBrickEvents = 64;        // events that reach a brick, per block (about)
+
+__device__ __forceinline__ bool orthonormal(const float *R)
 {
+    float worst = 0.0f;
+    bool finite = true;
+    for (int i = 0; i < 3; i++)
+        for (int j = i; j < 3; j++) {
+            const float d = (R[i] * R[j] + R[3 + i] * R[3 + j]) + R[6 + i] * R[6 + j] - (i == j ? 1.0f : 0.0f);
+            worst = fmaxf(worst, fabsf(d));
+            finite = finite && fabsf(d) < 1.0f;  // false for NaN
+        }
+    return finite && worst <= kOrtho;
+}
+
+constexpr int kRowAhead = 4;  // small voxels of a row read at once
+
+// (unsigned long long)x, the usual values below 2^32 in one instruction
+__device__ __forceinline__ unsigned long long fixed_u64(double x)
+{
+    if (__builtin_amdgcn_ballot_w64(!(x >= 0.0 && x < 4294967296.0)) != 0) {
+        asm volatile("");
+        return (unsigned long long)x;
+    }
+    return (uint32_t)x;
+}
+
+// What one small voxel of value val_in at the rotated (q0, q1, q2) adds (kernel.cl:262-341):
+// add(fs, ms, ss, value) once, or per corner.
+template <bool kLinear, class Add>
+__device__ __forceinline__ void merge_voxel(float q0, float q1, float q2, double val_in, double w, double mult,
+                                            int cab, Add add)
+{
+    if (!kLinear) {
+        // roundf(q) for |q| < 2^22: half away from zero is x + copysign(0.49999997f, x), truncated
+        auto round_away = [](float x) { return (int)(x + copysignf(0.49999997f, x)); };
+        add(round_away(q0) + cab, round_away(q1) + cab, round_away(q2) + cab, fixed_u64((val_in * w) * mult));
+        return;
+    }
+    const double sfs = (double)(1.0f - (q0 - floorf(q0)));
+    const double sms = (double)(1.0f - (q1 - floorf(q1)));
+    const double sss = (double)(1.0f - (q2 - floorf(q2)));
+    const int fs = (int)(floorf(q0) + (float)cab);
+    const int ms = (int)(floorf(q1) + (float)cab);
+    const int ss = (int)(floorf(q2) + (float)cab);
+    const double vmw = (val_in * mult) * w;
+#pragma unroll
+    for (int c = 0; c < 8; c++) {
+        const int ex = (c >> 1) & 1, ey = c >> 2, ez = c & 1;
+        add(fs + ex, ms + ey, ss + ez,
+            fixed_u64(vmw * (((ex ? 1 - sfs : sfs) * (ey ? 1 - sms : sms)) * (ez ? 1 - sss : sss))));
+    }
+}
+
+// The event's candidates for a brick: rows (y, z) of small voxels along k_a, y of ny from y0
+// (k_b), z of nz from z0 (k_c); row0 is the number of rows of the events listed before it.
+struct BrickEvent {
+    uint32_t event, row0;
+    int16_t y0, ny, z0, nz;
+};
+
+// Grid: x bricks, y slices of the events; a brick takes as many slices as events reach it.
+template <bool kLinear>
+__global__ void __launch_bounds__(256)
+    merge_brick_kernel(const double *__restrict__ small, size_t small_stride, int sab, int sc, int ka, int kb, int kc,
+                       const float *__restrict__ rw, uint32_t nev, double mult, int nbx, int nby,
+                       unsigned long long *__restrict__ big)
+{
+    __shared__ unsigned long long box[kBrick];
+    __shared__ BrickEvent list[256];
+    __shared__ uint32_t wev[4], wrow[4];
+    const int cab = (sab - 1) / 2, cc = (sc - 1) / 2;
+    const int bi = (int)blockIdx.x, b0 = (bi % nbx) * kBrX, b1 = (bi / nbx % nby) * kBrY, b2 = bi / (nbx * nby) * kBrZ;
+    const int e0_ = min(kBrX, sab - b0), e1_ = min(kBrY, sab - b1), e2_ = min(kBrZ, sab - b2);
+    // the q that reach the brick: its voxels' range (nearest: half a voxel more, linear: one),
+    // with a margin for the float arithmetic of either side
+    const float reach = (kLinear ? 1.0f : 0.5f) + 0.01f;
+    const float lo[3] = {(float)(b0 - cab) - reach, (float)(b1 - cab) - reach, (float)(b2 - cab) - reach};
+    const float hi[3] = {(float)(b0 + e0_ - 1 - cab) + reach, (float)(b1 + e1_ - 1 - cab) + reach,
+                         (float)(b2 + e2_ - 1 - cab) + reach};
+    const float mid[3] = {0.5f * (lo[0] + hi[0]), 0.5f * (lo[1] + hi[1]), 0.5f * (lo[2] + hi[2])};
+    const float half[3] = {0.5f * (hi[0] - lo[0]), 0.5f * (hi[1] - lo[1]), 0.5f * (hi[2] - lo[2])};
+    // events whose slab (cc planes each side) reaches a brick at distance r: about the share
+    // (its half diagonal + cc) / r
+    const float r = sqrtf(mid[0] * mid[0] + mid[1] * mid[1] + mid[2] * mid[2]);
+    const float share = fminf(1.0f, (11.0f + (float)cc) / fmaxf(r, 1.0f));
+    const uint32_t slices = min(gridDim.y, (uint32_t)((float)nev * share) / kBrickEvents + 1);
+    if (blockIdx.y >= slices) return;
+    const uint32_t ev0 = (uint32_t)((uint64_t)nev * blockIdx.y / slices);
+    const uint32_t ev1 = (uint32_t)((uint64_t)nev * (blockIdx.y + 1) / slices);
+    const float qmax = sqrtf(2.0f * (float)cab * (float)cab + (float)cc * (float)cc);
+    const float margin = 0.02f + 3.0f * kOrtho * qmax;  // |R^T q - q_in| of a small voxel
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    bool any = false;
+    for (uint32_t first = ev0; first < ev1; first += 256) {
+        const uint32_t e = first + threadIdx.x;
+        int l[3] = {0, 0, 0}, n[3] = {0, 0, 0};
+        if (e < ev1) {
+            float R[9];
+            for (int i = 0; i < 9; i++) R[i] = rw[10 * (size_t)e + i];
+            if (orthonormal(R)) {
+                const int c[3] = {ka, kb, kc}, ext[3] = {cab, cab, cc};
+#pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    const float r0 = c[j] == 0 ? R[0] : (c[j] == 1 ? R[1] : R[2]);
+                    const float r1 = c[j] == 0 ? R[3] : (c[j] == 1 ? R[4] : R[5]);
+                    const float r2 = c[j] == 0 ? R[6] : (c[j] == 1 ? R[7] : R[8]);
+                    const float p = r0 * mid[0] + r1 * mid[1] + r2 * mid[2];
+                    const float h = fabsf(r0) * half[0] + fabsf(r1) * half[1] + fabsf(r2) * half[2] + margin;
+                    l[j] = max(-ext[j], (int)ceilf(p - h));
+                    n[j] = min(ext[j], (int)floorf(p + h)) - l[j] + 1;
+                }
+            }
+        }
+        const bool hit = n[0] > 0 && n[1] > 0 && n[2] > 0;
+        const uint32_t rows = hit ? (uint32_t)(n[1] * n[2]) : 0u;
+        const uint64_t hits = __ballot(hit);
+        uint32_t x = rows;  // inclusive scan
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o, 64);
+            if (lane >= (uint32_t)o) x += y;
+        }
+        if (lane == 63) {
+            wev[wave] = (uint32_t)__popcll(hits);
+            wrow[wave] = x;
+        }
+        __syncthreads();
+        uint32_t at = (uint32_t)__popcll(hits & ((1ull << lane) - 1)), row = x - rows, nlist = 0, total = 0;
+        for (uint32_t w = 0; w < 4; w++) {
+            if (w < wave) {
+                at += wev[w];
+                row += wrow[w];
+            }
+            nlist += wev[w];
+            total += wrow[w];
+        }
+        if (hit)
+            list[at] = BrickEvent{e, row, (int16_t)l[1], (int16_t)n[1], (int16_t)l[2], (int16_t)n[2]};
+        if (total && !any) {
+            any = true;
+            for (int v = threadIdx.x; v < kBrick; v += 256) box[v] = 0ull;
+        }
+        __syncthreads();
+        for (uint32_t t = threadIdx.x; t < total; t += 256) {
+            uint32_t a = 0, end = nlist;  // the event of row t
+            while (end - a > 1) {
+                const uint32_t m = (a + end) / 2;
+                if (list[m].row0 <= t) a = m; else end = m;
+            }
+            const BrickEvent E = list[a];
+            const uint32_t k = t - E.row0, iz = k / (uint32_t)E.ny;
+            const int y = E.y0 + (int)(k - iz * (uint32_t)E.ny), z = E.z0 + (int)iz;
+            const float *Re = rw + 10 * (size_t)E.event;
+            const double w = (double)Re[9];
+            // q_i = (slope x + u) + v in the order of the components, x the voxel along k_a
+            float slope[3], u[3], v[3], x0 = (float)-cab, x1 = (float)cab;
+#pragma unroll
+            for (int i = 0; i < 3; i++) {
+                slope[i] = Re[3 * i + ka];
+                const float py = Re[3 * i + kb] * (float)y, pz = Re[3 * i + kc] * (float)z;
+                const float first_p = kb < kc ? py : pz, second_p = kb < kc ? pz : py;
+                u[i] = ka == 2 ? first_p + second_p : first_p;
+                v[i] = ka == 2 ? 0.0f : second_p;
+                const float s = py + pz;
+                if (fabsf(slope[i]) > 1e-6f) {
+                    const float inv = __builtin_amdgcn_rcpf(slope[i]), xa = (lo[i] - s) * inv, xb = (hi[i] - s) * inv;
+                    x0 = fmaxf(x0, fminf(xa, xb));
+                    x1 = fminf(x1, fmaxf(xa, xb));
+                } else if (s < lo[i] - 0.01f || s > hi[i] + 0.01f) {
+                    x1 = x0 - 1.0f;
+                }
+            }
+            const int i0 = max((int)ceilf(x0 - 0.02f), -cab), i1 = min((int)floorf(x1 + 0.02f), cab);
+            const double *src = small + small_stride * E.event + ((size_t)(z + cc) * sab + (size_t)(y + cab)) * sab + cab;
+            for (int i = i0; i <= i1; i += kRowAhead) {
+                double val[kRowAhead];
+#pragma unroll
+                for (int j = 0; j < kRowAhead; j++) val[j] = i + j <= i1 ? src[i + j] : 0.0;
+#pragma unroll
+                for (int j = 0; j < kRowAhead; j++) {
+                    if (val[j] < (double)1e-37f) continue;
+                    const float xf = (float)(i + j);
+                    const float q0 = (slope[0] * xf + u[0]) + v[0];
+                    const float q1 = (slope[1] * xf + u[1]) + v[1];
+                    const float q2 = (slope[2] * xf + u[2]) + v[2];
+                    merge_voxel<kLinear>(q0, q1, q2, val[j], w, mult, cab,
+                                         [&](int fs, int ms, int ss, unsigned long long x) {
+                                             const int lx = fs - b0, ly = ms - b1, lz = ss - b2;
+                                             if ((unsigned)lx < (unsigned)e0_ && (unsigned)ly < (unsigned)e1_ &&
+                                                 (unsigned)lz < (unsigned)e2_)
+                                                 atomicAdd(&box[lx + kBrX * (ly + kBrY * lz)], x);
+                                         });
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (!any) return;
+    for (int v = threadIdx.x; v < kBrick; v += 256) {
+        const unsigned long long x = box[v];
+        if (x) {
+            const size_t fs = b0 + v % kBrX, ms = b1 + v / kBrX % kBrY, ss = b2 + v / (kBrX * kBrY);
+            atomicAdd(big + fs + ms * sab + ss * sab * sab, x);
+        }
+    }
+}
+
+constexpr uint32_t kRestEvents = 16;  // at most 64
+
+// Small voxel `ind` under the events of this block row: every update of an event the bricks
+// do not take (all events where bricks is 0), of the others only the count of updates outside
+// the mesh, which voxels well inside its inscribed sphere do not have.
+template <bool kLinear>
+__global__ void __launch_bounds__(256)
+    merge_rest_kernel(const double *__restrict__ small, size_t small_stride, int sab, int sc, int ka, int kb, int kc,
+                      const float *__restrict__ rw, uint32_t nev, double mult, int bricks,
+                      unsigned long long *__restrict__ big, unsigned long long *__restrict__ dropped)
+{
+    __shared__ uint64_t taken;  // bit k: the bricks take event e0 + k
     const size_t nsmall = (size_t)sab * sab * sc;
     const size_t ind = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
+    const uint32_t e0 = blockIdx.y * kRestEvents, e1 = min(nev, e0 + kRestEvents);
+    if (threadIdx.x < 64) {
+        const uint32_t e = e0 + threadIdx.x;
+        const uint64_t b = __ballot(bricks && e < e1 && orthonormal(rw + 10 * (size_t)e));
+        if (threadIdx.x == 0) taken = b;
+    }
+    __syncthreads();
     if (ind >= nsmall) return;
-    const uint32_t e0 = blockIdx.y * ev_per_row, e1 = min(nev, e0 + ev_per_row);
     const int cab = (sab - 1) / 2, cc = (sc - 1) / 2;
     const int ss_in = (int)(ind / ((size_t)sab * sab));
     const int ms_in = (int)((ind - (size_t)ss_in * sab * sab) / sab);
     const int fs_in = (int)(ind - (size_t)ss_in * sab * sab - (size_t)ms_in * sab);
-    float q_in[3];
-    q_in[ka] = (float)(fs_in - cab);
-    q_in[kb] = (float)(ms_in - cab);
-    q_in[kc] = (float)(ss_in - cc);
-    auto add = [&](int fs, int ms, int ss, unsigned long long v) {
-        if ((unsigned)fs < (unsigned)sab && (unsigned)ms < (unsigned)sab && (unsigned)ss < (unsigned)sab) {
-            if (v) atomicAdd(big + (size_t)fs + (size_t)ms * sab + (size_t)ss * sab * sab, v);
-        } else {
-            atomicAdd(dropped, 1ull);
-        }
-    };
+    const float qa = (float)(fs_in - cab), qb = (float)(ms_in - cab), qc = (float)(ss_in - cc);
+    const float qi0 = ka == 0 ? qa : (kb == 0 ? qb : qc), qi1 = ka == 1 ? qa : (kb == 1 ? qb : qc);
+    const float qi2 = ka == 2 ? qa : (kb == 2 ? qb : qc);
+    // |R q| <= |q| sqrt(1 + 3 kOrtho); the farthest corner is within one voxel of it per axis
+    const float inner = (float)cab - 1.5f;
+    const bool inside = inner > 0.0f && (qa * qa + qb * qb + qc * qc) * (1.0f + 4.0f * kOrtho) < inner * inner;
+    const uint64_t skip = taken;
+    const uint32_t n = e1 - e0;
+    if (inside && skip == (n < 64 ? (1ull << n) - 1 : ~0ull)) return;
     for (uint32_t i = e0; i < e1; i++) {
+        const float *R = rw + 10 * (size_t)i;
+        const bool in_bricks = (skip >> (i - e0)) & 1;
+        if (in_bricks && inside) continue;
         const double val_in = small[small_stride * i + ind];  // stride 0: one mesh for all events
         if (val_in < (double)1e-37f) continue;
-        const float *R = rw + 10 * (size_t)i;
-        const float q0 = R[0] * q_in[0] + R[1] * q_in[1] + R[2] * q_in[2];
-        const float q1 = R[3] * q_in[0] + R[4] * q_in[1] + R[5] * q_in[2];
-        const float q2 = R[6] * q_in[0] + R[7] * q_in[1] + R[8] * q_in[2];
-        const double w = (double)R[9];
-        if (interp == 0) {
-            add((int)(roundf(q0) + (float)cab), (int)(roundf(q1) + (float)cab), (int)(roundf(q2) + (float)cab),
-                (unsigned long long)((val_in * w) * mult));
-        } else {
-            const double sfs = (double)(1.0f - (q0 - floorf(q0)));
-            const double sms = (double)(1.0f - (q1 - floorf(q1)));
-            const double sss = (double)(1.0f - (q2 - floorf(q2)));
-            const int fs = (int)(floorf(q0) + (float)cab);
-            const int ms = (int)(floorf(q1) + (float)cab);
-            const int ss = (int)(floorf(q2) + (float)cab);
-            const double vmw = (val_in * mult) * w;
-            add(fs + 0, ms + 0, ss + 0, (unsigned long long)(vmw * ((sfs * sms) * sss)));
-            add(fs + 0, ms + 0, ss + 1, (unsigned long long)(vmw * ((sfs * sms) * (1 - sss))));
-            add(fs + 1, ms + 0, ss + 0, (unsigned long long)(vmw * (((1 - sfs) * sms) * sss)));
-            add(fs + 1, ms + 0, ss + 1, (unsigned long long)(vmw * (((1 - sfs) * sms) * (1 - sss))));
-            add(fs + 0, ms + 1, ss + 0, (unsigned long long)(vmw * ((sfs * (1 - sms)) * sss)));
-            add(fs + 0, ms + 1, ss + 1, (unsigned long long)(vmw * ((sfs * (1 - sms)) * (1 - sss))));
-            add(fs + 1, ms + 1, ss + 0, (unsigned long long)(vmw * (((1 - sfs) * (1 - sms)) * sss)));
-            add(fs + 1, ms + 1, ss + 1, (unsigned long long)(vmw * (((1 - sfs) * (1 - sms)) * (1 - sss))));
-        }
+        const float q0 = R[0] * qi0 + R[1] * qi1 + R[2] * qi2;
+        const float q1 = R[3] * qi0 + R[4] * qi1 + R[5] * qi2;
+        const float q2 = R[6] * qi0 + R[7] * qi1 + R[8] * qi2;
+        merge_voxel<kLinear>(q0, q1, q2, val_in, (double)R[9], mult, cab,
+                             [&](int fs, int ms, int ss, unsigned long long v) {
+                                 if ((unsigned)fs < (unsigned)sab && (unsigned)ms < (unsigned)sab &&
+                                     (unsigned)ss < (unsigned)sab) {
+                                     if (v && !in_bricks)
+                                         atomicAdd(big + (size_t)fs + (size_t)ms * sab + (size_t)ss * sab * sab, v);
+                                 } else {
+                                     atomicAdd(dropped, 1ull);
+                                 }
+                             });
     }
 }
 
@@ -264,14 +487,31 @@ static int merge_launch(iac_ctx *ctx, const double *d_small_cq, bool per_event, 
     if (interp != IAC_NEAREST && interp != IAC_LINEAR) return iac::fail(IAC_ERR_INVALID_ARG, "bad interpolation");
     if (nev == 0) return IAC_OK;
     const size_t nsmall = (size_t)small_shape->size_ab * small_shape->size_ab * small_shape->size_c;
-    const uint32_t per_row = 16;
-    const dim3 grid((unsigned)((nsmall + 255) / 256), (nev + per_row - 1) / per_row);
+    const size_t stride = per_event ? nsmall : (size_t)0;
+    const int sab = (int)small_shape->size_ab, sc = (int)small_shape->size_c;
+    const int ka = (int)small_shape->k_a, kb = (int)small_shape->k_b, kc = (int)small_shape->k_c;
+    auto *big = reinterpret_cast<unsigned long long *>(d_big);
+    // Bricks cost about 20 us and 3 ns each before their first candidate, a scattered add costs
+    // 0.04 ns: measured break-even (nearest / linear) at 63 / 8 events of 65 x 65 x 3 (405 bricks),
+    // 11 / 1 of 129 x 129 x 3 (2,601) and 10 / 1 of 257 x 257 x 3 (18,513).  100 linear events of
+    // those meshes take 441, 1,451 and 4,938 us scattered, 150, 214 and 603 us in bricks.  The
+    // candidate ranges are 16 bits.
+    const uint64_t nbx = (sab + kBrX - 1) / kBrX, nby = (sab + kBrY - 1) / kBrY, nbz = (sab + kBrZ - 1) / kBrZ;
+    const uint64_t nbricks = nbx * nby * nbz;
+    const bool bricks = (uint64_t)nev * nsmall * (interp ? 8 : 1) >= 600000 + 75 * nbricks && sab < 32768 &&
+                        sc < 32768 && nbricks < (1u << 31);
+    const dim3 rest((unsigned)((nsmall + 255) / 256), (nev + kRestEvents - 1) / kRestEvents);
     IAC_TRY(iac::timer_begin(ctx));
-    hipLaunchKernelGGL(merge_cq_kernel, grid, dim3(256), 0, ctx->stream, d_small_cq, per_event ? nsmall : (size_t)0,
-                       (int)small_shape->size_ab,
-                       (int)small_shape->size_c, (int)small_shape->k_a, (int)small_shape->k_b,
-                       (int)small_shape->k_c, d_rw10, nev, per_row, interp, mult,
-                       reinterpret_cast<unsigned long long *>(d_big), ctx->d_counters);
+    if (bricks) {
+        const dim3 grid((unsigned)nbricks, std::min<uint32_t>(65535, nev / kBrickEvents + 1));
+        hipLaunchKernelGGL(interp ? merge_brick_kernel<true> : merge_brick_kernel<false>, grid, dim3(256), 0,
+                           ctx->stream, d_small_cq, stride, sab, sc, ka, kb, kc, d_rw10, nev, mult, (int)nbx, (int)nby,
+                           big);
+        IAC_HIP(hipGetLastError());
+    }
+    hipLaunchKernelGGL(interp ? merge_rest_kernel<true> : merge_rest_kernel<false>, rest, dim3(256), 0, ctx->stream,
+                       d_small_cq, stride, sab, sc, ka, kb, kc, d_rw10, nev, mult, bricks ? 1 : 0, big,
+                       ctx->d_counters);
     IAC_HIP(hipGetLastError());
     IAC_TRY(iac::timer_end(ctx));
     return IAC_OK;

@@ -329,3 +329,47 @@ def test_cfg3_full_size_halves_and_symmetry(ctx, dev):
     assert np.array_equal(sm, sm[:, ::-1])
     assert np.array_equal(got_big, got_big[::-1])
     assert got_big.sum() > 0
+
+
+@pytest.mark.parametrize("axes", [(0, 1, 2), (1, 0, 2), (2, 0, 1), (0, 2, 1)])
+@pytest.mark.parametrize("sab,sc,nev", [(5, 5, 1), (17, 3, 2), (31, 15, 5), (33, 3, 260), (49, 7, 70), (65, 3, 9)])
+@pytest.mark.parametrize("interp", [0, 1])
+def test_merge_bricks_vs_oracle(ctx, dev, axes, sab, sc, nev, interp):
+    """The merge's brick and rest kernels: every axis order, meshes that are no multiple of a
+    brick, few and many events, rotations beside matrices that are none (scaled, sheared,
+    mirrored, zero), values up to the mesh's corners: the mesh and the count of updates that
+    leave it."""
+    import torch
+
+    import incohautocorrelate_amd as iac
+
+    rng = np.random.default_rng(sab * 7 + nev + interp)
+    s = iac.MeshShape(k_a=axes[0], k_b=axes[1], k_c=axes[2], size_ab=sab, size_c=sc)
+    s.voxel_per_dq, s.max_q = 1, 1.0
+    rots = W.random_rotations(nev, nev)
+    rots[0] = np.eye(3, dtype=np.float32).reshape(9)
+    if nev > 4:
+        rots[1] *= np.float32(1.00002)  # still taken by the bricks
+        rots[2] *= np.float32(1.2)
+        rots[3] = rng.normal(0, 0.5, 9)
+        rots[4] = 0
+    if nev > 60:
+        rots[5::9, :3] *= -1
+    rw = np.concatenate([rots, rng.random((nev, 1)).astype(np.float32)], 1).astype(np.float32)
+    small = rng.random((nev, sc * sab * sab)) * (rng.random(sc * sab * sab) < 0.8)
+    mult = 1e4 if interp else 1e11  # nearest: values past 2^32
+    for multi in (False, True)[: 2 if nev < 100 else 1]:
+        ref, drop = np.zeros(sab ** 3, np.uint64), 0
+        if multi:
+            for i in range(nev):
+                r, d = O.merge_cq(small[i], s, rw[i:i + 1], interp, mult)
+                ref += r
+                drop += d
+        else:
+            ref, drop = O.merge_cq(small[0], s, rw, interp, mult)
+        big = _zeros(sab ** 3, dev)
+        before = ctx.dropped()
+        call = ctx.merge_cq_multi if multi else ctx.merge_cq
+        call(torch.from_numpy(small if multi else small[0]).to(dev), s, to_dev(rw, dev), interp, mult, big)
+        assert np.array_equal(mesh_np(big), ref)
+        assert ctx.dropped() - before == drop
