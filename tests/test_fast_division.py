@@ -86,3 +86,29 @@ def test_fixed_point_step():
         t = fast(np.array([p], f32), step)[0] + f32(0.5)
         short = int(np.floor(t).astype(np.int64)) & 0xFFFFFFFF
         assert L.ora_pair_val(float(p)) == short, p
+
+
+def test_nearest_bin_from_raw_root():
+    """The nearest-neighbour C(q) bin from a square root off by up to one ulp, a float 1 / dq and
+    one multiply-add: wherever its fraction is accepted, it is the bin of the exact q."""
+    rng = np.random.default_rng(5)
+    accepted = total = 0
+    for size in (64, 500, 4096, 6144):
+        for _ in range(6):
+            dq = f32(2.0 ** rng.uniform(-30, 2))
+            near = (rng.integers(0, size - 2, 200_000) + 0.5) * (1 + rng.normal(0, 1e-6, 200_000))
+            b = np.concatenate([rng.uniform(0, size - 1.5, 200_000), near])
+            x = ((b * f64(dq)) ** 2).astype(f32)
+            root = np.sqrt(x)
+            want = np.floor((root / dq).astype(f32).astype(f64) + 0.5)
+            inv = f32(f64(1.0) / f64(dq))
+            for ulp in (-1, 0, 1):
+                s = (root.view(np.int32) + ulp).astype(np.int32).view(f32)
+                s = np.where(x > 0, s, f32(0))
+                u = (s.astype(f64) * f64(inv) + 0.5).astype(f32)  # exact product, one rounding (53 >= 48 bits)
+                fr = u - np.floor(u)
+                ok = np.abs(fr - f32(0.5)) < (u.astype(f64) * f64(f32(-5e-7)) + 0.5).astype(f32)
+                assert np.array_equal(np.floor(u[ok]).astype(f64), want[ok])
+                accepted += int(ok[:200_000].sum())
+                total += 200_000
+    assert accepted > 0.99 * total

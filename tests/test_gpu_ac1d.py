@@ -221,3 +221,62 @@ def test_ac1d_acuw_sparse_1024_4096_bins(ctx, dev, interp):
         assert np.array_equal(got, ref)
     else:
         assert np.allclose(got, ref, rtol=1e-12, atol=1e-9)
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 1), (1, 2), (3, 5), (1, 63), (8, 8), (5, 13), (9, 9), (1, 129), (31, 37)])
+@pytest.mark.parametrize("interp", [0, 1])
+@pytest.mark.parametrize("kind", ["plain", "masked", "negative", "cut", "coarse", "huge_mult"])
+def test_ac1d_cq_units_and_plain_images(ctx, dev, rows, cols, interp, kind):
+    """The C(q) kernel at the edges of its units (64 x 16 pairs), with images that take the plain
+    loop and ones that must not: negative values, a Max_Q that cuts pairs, bins too coarse for
+    its range, values past 2^32."""
+    import torch
+
+    import incohautocorrelate_amd as iac
+
+    rng = np.random.default_rng(rows * 100 + cols)
+    pm = iac.generate_pixel_map(rows, cols, 75.0, [0, 0, 2e4], [1, 0, 0], [0, 1, 0])
+    km, _, _, mq = iac.calc_kmap(pm)
+    size = 64
+    max_q, dq = iac.ac1d_shape(mq, size) if rows * cols > 1 else (0.1, 0.01)
+    I = rng.gamma(1.0, 0.5, rows * cols).astype(np.float32)
+    mult = 1e6
+    if kind == "masked":
+        I *= rng.random(I.size) > 0.4
+    elif kind == "negative":
+        I -= np.float32(0.3)
+    elif kind == "cut":
+        max_q *= 0.6
+    elif kind == "coarse":
+        dq *= 0.7
+    elif kind == "huge_mult":
+        mult = 1e13
+    ref, dref = O.ac1d_cq(I, km, size, max_q, dq, interp, mult)
+    h = torch.zeros(size, dtype=torch.int64, device=dev)
+    before = ctx.dropped()
+    ctx.ac1d_cq(to_dev(km, dev), to_dev(I, dev), size, max_q, dq, interp, mult, h)
+    assert np.array_equal(mesh_np(h), ref)
+    assert ctx.dropped() - before == dref
+
+
+@pytest.mark.parametrize("interp", [0, 1])
+def test_ac1d_acuw_frame_edges(ctx, dev, interp):
+    """AC_uw over frames of 0, 1 and sizes about the units' 16 and 64 records, in one call; the
+    double sums to 1e-12 (their order differs), each bin's weights being up to 2 n^2."""
+    import torch
+
+    import incohautocorrelate_amd as iac
+
+    sizes = [0, 1, 2, 0, 15, 16, 17, 63, 64, 65, 127, 128, 129, 0, 300, 1, 0]
+    _, km, mq = W.detector(48)
+    max_q, dq = iac.ac1d_shape(mq, 200)
+    rng = np.random.default_rng(3)
+    hl = [np.concatenate([km[np.sort(rng.choice(48 * 48, n, False))], rng.integers(1, 4, (n, 1))], 1).astype(np.float32)
+          for n in sizes]
+    ref = np.zeros(200)
+    for x in hl:
+        ref, _ = O.ac1d_acuw(x, 200, max_q, dq, interp, 2, ac=ref)
+    off = np.cumsum([0] + sizes).astype(np.int64)
+    h = torch.zeros(200, dtype=torch.float64, device=dev)
+    ctx.ac1d_acuw_records(to_dev(np.concatenate(hl), dev), to_dev(off, dev), int(off[-1]), 200, max_q, dq, interp, h)
+    assert np.allclose(h.cpu().numpy(), ref, rtol=1e-12, atol=0)
