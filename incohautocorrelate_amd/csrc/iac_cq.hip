@@ -358,13 +358,6 @@ int cq_frames(iac_ctx *ctx, const float *d_kmap, uint32_t npix, const float *d_f
     if (!(mult > 0)) return iac::fail(IAC_ERR_INVALID_ARG, "multiplicator must be > 0");
     if (nframes == 0) return IAC_OK;
     const uint64_t n = (uint64_t)npix * nframes;
-    // records, then the frame offsets, in scratch slot 0
-    void *rec = nullptr;
-    IAC_TRY(iac::scratch(ctx, 0, n * sizeof(float4) + (nframes + 1) * sizeof(uint64_t), &rec));
-    void *off = static_cast<char *>(rec) + n * sizeof(float4);
-    hipLaunchKernelGGL(gather_dense_kernel, dim3(blocks_for(n)), dim3(256), 0, ctx->stream, d_kmap, d_frames,
-                       npix, nframes, static_cast<float4 *>(rec), static_cast<uint64_t *>(off));
-    IAC_HIP(hipGetLastError());
     iac::PairRun R;
     std::memset(&R.spec, 0, sizeof(R.spec));
     R.spec.kind = iac::kKindCq;
@@ -384,13 +377,25 @@ int cq_frames(iac_ctx *ctx, const float *d_kmap, uint32_t npix, const float *d_f
     R.ordered = interp == IAC_LINEAR;
     R.d_kmap = d_kmap;
     R.npix = npix;
-    R.rec = static_cast<const float4 *>(rec);
-    R.d_frame_off = static_cast<const uint64_t *>(off);
+    R.rec = nullptr;
+    R.d_frame_off = nullptr;
     R.nframes = nframes;
     R.n_total = n;
     R.h_group_off = h_group_off;
     R.ngroups = ngroups;
     R.d_mesh = d_meshes;
+    bool done = false;
+    IAC_TRY(iac::cq_tiles_run(ctx, R, d_frames, &done));
+    if (done) return IAC_OK;
+    // records, then the frame offsets, in scratch slot 0
+    void *rec = nullptr;
+    IAC_TRY(iac::scratch(ctx, 0, n * sizeof(float4) + (nframes + 1) * sizeof(uint64_t), &rec));
+    void *off = static_cast<char *>(rec) + n * sizeof(float4);
+    hipLaunchKernelGGL(gather_dense_kernel, dim3(blocks_for(n)), dim3(256), 0, ctx->stream, d_kmap, d_frames,
+                       npix, nframes, static_cast<float4 *>(rec), static_cast<uint64_t *>(off));
+    IAC_HIP(hipGetLastError());
+    R.rec = static_cast<const float4 *>(rec);
+    R.d_frame_off = static_cast<const uint64_t *>(off);
     return iac::pairs_run(ctx, R);
 }
 

@@ -45,6 +45,11 @@ struct PairRun {
 
 int pairs_run(iac_ctx *ctx, const PairRun &run);
 
+// C(q) of dense frames d_frames ([nframes][npix]) by region tiles (run.rec and run.d_frame_off are
+// not read).  *done is false where the frames are too sparse or the geometry does not suit them:
+// nothing was added, and pairs_run takes the run.
+int cq_tiles_run(iac_ctx *ctx, const PairRun &run, const float *d_frames, bool *done);
+
 // Prepared runs: the plan, the frame chunks and every buffer made once (run.rec,
 // run.d_frame_off and the kmap are kept by pointer; their contents may change
 // between launches as long as sizes and the frame count stay); pairs_enqueue

@@ -1239,6 +1239,468 @@ __global__ void __launch_bounds__(kBlock, (Occupancy<FAST, BOX>::blocks))
     }
 }
 
+// ---- dense C(q): region tiles -----------------------------------------------------
+//
+// Dense images hold many records per voxel, so the cell-offset tasks above spend their time on
+// index work and on neighbouring pairs adding to one LDS word (20.6 ms for the 9.6e9 pairs of a
+// 384 x 360 image into 129 x 129 x 3).  Here a task is a pair of regions (I, J) of the detector,
+// up to 12 x 12 voxels each, whose whole range of q fits the LDS box: a wave owns 64 records of
+// I, one per lane, spread evenly over the region so that they fall on different voxels, and takes
+// J's records one by one from the scalar unit.  A pair is then its binning and nothing else:
+// about 24 VALU instructions nearest, 67 linear.  Measured: the image above 20.6 -> 5.6 ms
+// (nearest: VALU issue), 191 x 173 into 97 x 97 x 3 linear 14.6 -> 5.4 ms (bound by its eight LDS
+// adds per pair, 23 clocks each: two or three of the 64 lanes share a voxel).
+
+struct TileTask {
+    int ci, cj;         // the regions of the a and b records; nearest neighbour: ci <= cj
+    int bx0, by0, bz0;  // LDS box origin (voxel indices) and extent, as in Task
+    int bx, by, bz;
+    int inbox;  // every voxel the task's pairs add to lies in the box
+    int allin;  // no pair fails the cut
+    int sa, sb;  // the sign of q along the mesh's first two axes: 1 or -1, 0 where it varies
+};
+
+constexpr int kTileB = 16;  // b records per unit of work
+constexpr int kTileParts = 144;  // voxel-sized parts of a region, at most
+// b records per scalar load batch, unrolled: a linear pair's eight corners are work enough for the
+// scheduler, and more of them spill
+template <bool LINEAR>
+struct TileBatch {
+    static constexpr int n = LINEAR ? 2 : 8;
+};
+
+typedef float f4v __attribute__((ext_vector_type(4)));
+typedef const __attribute__((address_space(4))) f4v *scalar_rec_t;
+
+// The sort key of a k: its region, then its voxel-sized part of the region (side x side parts,
+// so records of one region that lie far apart in its order lie on different voxels).
+__device__ __forceinline__ uint32_t tile_key(const CellGeom &g, int side, float ku, float kv)
+{
+    const float xu = (ku - g.u0) * g.inv_wu, xv = (kv - g.v0) * g.inv_wv;
+    const int cu = min(max((int)floorf(xu), 0), g.ncu - 1), cv = min(max((int)floorf(xv), 0), g.ncv - 1);
+    const int su = min(max((int)((xu - (float)cu) * (float)side), 0), side - 1);
+    const int sv = min(max((int)((xv - (float)cv) * (float)side), 0), side - 1);
+    return (uint32_t)((cv * g.ncu + cu) * side + sv) * (uint32_t)side + (uint32_t)su;
+}
+
+// Counts of the frames' nonzero pixels per key (cs, zeroed by the caller), the groups' self
+// values (symmetric modes), the number of kept records, and the run's flag, cleared by any record
+// that could make a pair negative, NaN or 2^32 or more (then the pairs take the general value).
+// Grid: ns blocks per frame.
+template <bool ORD>
+__global__ void __launch_bounds__(kBlock)
+    tile_count_kernel(const float *__restrict__ kmap, const float *__restrict__ frames, uint32_t npix, uint32_t ns,
+                      CellGeom g, int side, PairSpec S, const uint32_t *__restrict__ group_off, uint32_t ngroups,
+                      uint32_t *__restrict__ cs, unsigned long long *__restrict__ self,
+                      uint32_t *__restrict__ plain, unsigned long long *__restrict__ kept)
+{
+    __shared__ unsigned long long sred[kBlock / 64], kred[kBlock / 64];
+    const uint32_t f = blockIdx.x / ns;
+    const size_t nkey = (size_t)g.ncu * g.ncv * side * side;
+    uint32_t *csf = cs + f * (nkey + 1);
+    unsigned long long sv = 0, n = 0;
+    bool ok = 1e-37 * S.mult < 0.99;  // a product below 1e-37 adds nothing either way
+    for (uint32_t p = (blockIdx.x - f * ns) * kBlock + threadIdx.x; p < npix; p += ns * kBlock) {
+        const float I = frames[(size_t)f * npix + p];
+        if (I == 0.0f) continue;
+        atomicAdd(csf + tile_key(g, side, kmap[3 * (size_t)p + g.au], kmap[3 * (size_t)p + g.av]), 1u);
+        n++;
+        if (!ORD) sv += self_value<kKindCq>(S, I);
+        ok = ok && I > 0.0f && (double)(I * I) * S.mult < 4294967296.0;
+    }
+    if (!ok) plain[0] = 0u;
+    for (int o = 32; o > 0; o >>= 1) {
+        sv += __shfl_down(sv, o, 64);
+        n += __shfl_down(n, o, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        sred[threadIdx.x >> 6] = sv;
+        kred[threadIdx.x >> 6] = n;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        sv = n = 0;
+        for (int w = 0; w < kBlock / 64; w++) {
+            sv += sred[w];
+            n += kred[w];
+        }
+        if (n) atomicAdd(kept, n);
+        if (sv) {
+            uint32_t lo = 0, hi = ngroups;  // group of f: largest gi with group_off[gi] <= f
+            while (hi - lo > 1) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (group_off[mid] <= f) lo = mid; else hi = mid;
+            }
+            atomicAdd(self + lo, sv);
+        }
+    }
+}
+
+// One block per frame: the key counts become first positions (cs[nkey] the frame's records), and
+// the scatter's cursors.
+__global__ void __launch_bounds__(1024) tile_scan_kernel(uint32_t *__restrict__ cs, uint32_t *__restrict__ cursor,
+                                                         uint32_t nkey)
+{
+    __shared__ uint32_t part[16];
+    uint32_t *csf = cs + (size_t)blockIdx.x * (nkey + 1);
+    uint32_t *cur = cursor + (size_t)blockIdx.x * nkey;
+    const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+    uint32_t base = 0;
+    for (uint32_t k0 = 0; k0 < nkey; k0 += 4096) {  // four keys per thread and step
+        uint32_t v[4], s = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            v[i] = k0 + 4 * t + i < nkey ? csf[k0 + 4 * t + i] : 0u;
+            s += v[i];
+        }
+        uint32_t x = s;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o, 64);
+            if (lane >= (uint32_t)o) x += y;
+        }
+        if (lane == 63) part[wave] = x;
+        __syncthreads();
+        uint32_t run = base + x - s;
+        for (uint32_t w = 0; w < 16; w++) {
+            if (w < wave) run += part[w];
+            base += part[w];
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < 4; i++) {
+            if (k0 + 4 * t + i < nkey) csf[k0 + 4 * t + i] = cur[k0 + 4 * t + i] = run;
+            run += v[i];
+        }
+        __syncthreads();
+    }
+    if (t == 0) csf[nkey] = base;
+}
+
+// The nonzero pixels as records {k[ka], k[kb], k[kc], I} in key order, frame f from f npix.
+__global__ void __launch_bounds__(kBlock)
+    tile_scatter_kernel(const float *__restrict__ kmap, const float *__restrict__ frames, uint32_t npix, uint32_t ns,
+                        CellGeom g, int side, int ka, int kb, int kc, uint32_t *__restrict__ cursor,
+                        float4 *__restrict__ srec)
+{
+    const uint32_t f = blockIdx.x / ns;
+    uint32_t *cur = cursor + f * ((size_t)g.ncu * g.ncv * side * side);
+    for (uint32_t p = (blockIdx.x - f * ns) * kBlock + threadIdx.x; p < npix; p += ns * kBlock) {
+        const float I = frames[(size_t)f * npix + p];
+        if (I == 0.0f) continue;
+        const float *k = kmap + 3 * (size_t)p;
+        srec[(size_t)f * npix + atomicAdd(cur + tile_key(g, side, k[g.au], k[g.av]), 1u)] =
+            make_float4(k[ka], k[kb], k[kc], I);
+    }
+}
+
+constexpr uint32_t kPartBatch = 4;  // b records per scalar load batch
+
+// A nearest-neighbour task of an image with many records per voxel.  For one a record the records
+// of one part of J -- a voxel across -- fall on at most two voxels per axis, so a lane keeps the
+// sums of its a with the part in registers and adds them to the box once per part: two compares in
+// place of the rounding and the address, and no LDS add per pair.  Exact: subtraction, scaling and
+// rounding are monotone, so the part's k extents give its first and last voxel; x rounds to n + 1
+// or more where x >= n + 1/2 (n >= 0) or x > n + 1/2 (n < 0, half away from zero); the values are
+// whole numbers below 2^32, whose sums a double holds.  A part that spans more voxels for some
+// lane is binned pair by pair.
+__device__ __forceinline__ void tile_by_parts(const float4 *__restrict__ rec, const uint32_t *__restrict__ csf,
+                                              size_t parts, uint32_t a0, uint32_t na, const TileTask &T, float vox,
+                                              double mult, int bx8, int bxby8, int c8, char *boxb,
+                                              float (*ext)[kTileParts], uint32_t share, uint32_t shares)
+{
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t *pj = csf + T.cj * parts;
+    __syncthreads();  // the frame before may still be read
+    for (uint32_t s = wave; s < parts; s += kBlock / 64) {
+        const uint32_t s0 = pj[s], s1 = pj[s + 1];
+        float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
+        for (uint32_t i = s0 + lane; i < s1; i += 64) {
+            const float4 r = rec[i];
+            lo[0] = fminf(lo[0], r.x);
+            lo[1] = fminf(lo[1], r.y);
+            lo[2] = fminf(lo[2], r.z);
+            hi[0] = fmaxf(hi[0], r.x);
+            hi[1] = fmaxf(hi[1], r.y);
+            hi[2] = fmaxf(hi[2], r.z);
+        }
+        for (int o = 32; o > 0; o >>= 1)
+            for (int d = 0; d < 3; d++) {
+                lo[d] = fminf(lo[d], __shfl_xor(lo[d], o, 64));
+                hi[d] = fmaxf(hi[d], __shfl_xor(hi[d], o, 64));
+            }
+        if (lane == 0)
+            for (int d = 0; d < 3; d++) {
+                ext[d][s] = lo[d];
+                ext[3 + d][s] = hi[d];
+            }
+    }
+    __syncthreads();
+    const uint32_t groups = (na + 63) / 64, np = (uint32_t)parts;
+    const uint64_t units = (uint64_t)groups * np;
+    const uint64_t u0 = units * share / shares, u1 = units * (share + 1) / shares;
+    uint32_t gr = (uint32_t)(u0 / np), s = (uint32_t)(u0 - (uint64_t)gr * np);
+    float4 a = rec[a0 + min(gr * 64 + lane, na - 1)];
+    // the float above n + 1/2 that the first x of voxel n + 1 reaches
+    auto edge_of = [](int n) {
+        const float t = (float)n + 0.5f;
+        return n < 0 ? __uint_as_float(__float_as_uint(t) - 1u) : t;
+    };
+    // v, or next to nothing: only the high word is selected, and what the low word leaves (below
+    // 2^-1021) vanishes in a sum of whole numbers or truncates to 0
+    auto v_if = [](bool m, double v) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        const uint32_t h = m ? (uint32_t)(u >> 32) : 0u;
+        return __builtin_bit_cast(double, ((uint64_t)h << 32) | (uint32_t)u);
+    };
+    auto add = [&](int o, double x) {
+        if (x >= 1.0) atomicAdd(reinterpret_cast<unsigned long long *>(boxb + o), (unsigned long long)x);
+    };
+    for (uint64_t u = u0; u < u1; u++) {
+        const uint32_t s0 = pj[s], s1 = pj[s + 1];
+        if (s0 < s1 && gr * 64 + lane < na) {
+            const scalar_rec_t b = (scalar_rec_t)(uintptr_t)(rec + s0);
+            const uint32_t n = s1 - s0;
+            const int a_n0 = round_away((a.x - ext[3][s]) * vox), a_n1 = round_away((a.x - ext[0][s]) * vox);
+            const int b_n0 = round_away((a.y - ext[4][s]) * vox), b_n1 = round_away((a.y - ext[1][s]) * vox);
+            const int c_n0 = round_away((a.z - ext[5][s]) * vox), c_n1 = round_away((a.z - ext[2][s]) * vox);
+            const int o = __mul24(c_n0, bxby8) + (__mul24(b_n0, bx8) + (a_n0 * 8 + c8));
+            const bool wide = a_n1 - a_n0 > 1 || b_n1 - b_n0 > 1 || c_n1 - c_n0 > 1;
+            if (__ballot(wide) != 0 || n >= (1u << 20)) {
+                for (uint32_t j = 0; j < n; j++) {
+                    const f4v r = b[j];
+                    const double v = (double)(a.w * r.w) * mult;
+                    const int q = __mul24(round_away((a.z - r.z) * vox), bxby8) +
+                                  (__mul24(round_away((a.y - r.y) * vox), bx8) + (round_away((a.x - r.x) * vox) * 8 + c8));
+                    atomicAdd(reinterpret_cast<unsigned long long *>(boxb + q), (unsigned long long)(uint32_t)v);
+                }
+            } else {
+                const float ta = edge_of(a_n0), tb = edge_of(b_n0), tc = edge_of(c_n0);
+                // sums over the pairs beyond no, one or both edges: s00 all, s10 beyond a's, s01 b's, s11 both
+                auto sums = [&](auto deep_c) {
+                    constexpr bool kDeep = decltype(deep_c)::value;
+                    double s00 = 0, s10 = 0, s01 = 0, s11 = 0, d00 = 0, d10 = 0, d01 = 0, d11 = 0;
+                    for (uint32_t j0 = 0; j0 < n; j0 += kPartBatch) {
+                        f4v r[kPartBatch];
+#pragma unroll
+                        for (uint32_t k = 0; k < kPartBatch; k++) {
+                            r[k] = b[min(j0 + k, n - 1)];
+                            if (j0 + k >= n) r[k].w = 0.0f;  // past the part: adds nothing
+                        }
+#pragma unroll
+                        for (uint32_t k = 0; k < kPartBatch; k++) {
+                            const bool ma = (a.x - r[k].x) * vox >= ta, mb = (a.y - r[k].y) * vox >= tb;
+                            const double v = trunc((double)(a.w * r[k].w) * mult);
+                            s00 += v;
+                            s10 += v_if(ma, v);
+                            s01 += v_if(mb, v);
+                            s11 += v_if(ma && mb, v);
+                            if (kDeep) {
+                                const bool mc = (a.z - r[k].z) * vox >= tc;
+                                d00 += v_if(mc, v);
+                                d10 += v_if(mc && ma, v);
+                                d01 += v_if(mc && mb, v);
+                                d11 += v_if(mc && ma && mb, v);
+                            }
+                        }
+                    }
+                    auto plane = [&](int at, double p00, double p10, double p01, double p11) {
+                        add(at, (p00 - p10) - (p01 - p11));
+                        add(at + 8, p10 - p11);
+                        add(at + bx8, p01 - p11);
+                        add(at + bx8 + 8, p11);
+                    };
+                    if (kDeep) {
+                        plane(o, s00 - d00, s10 - d10, s01 - d01, s11 - d11);
+                        plane(o + bxby8, d00, d10, d01, d11);
+                    } else {
+                        plane(o, s00, s10, s01, s11);
+                    }
+                };
+                if (__ballot(c_n1 != c_n0) != 0) sums(std::true_type{}); else sums(std::false_type{});
+            }
+        }
+        if (++s == np) {
+            s = 0;
+            gr++;
+            a = rec[a0 + min(gr * 64 + lane, na - 1)];
+        }
+    }
+}
+
+// Grid: ntasks per chunk of frames of one group.  Symmetric (nearest) runs bin each unordered pair
+// once into the half mesh, linear ones every ordered pair, self pairs too, into the mesh.
+template <bool LINEAR>
+__global__ void __launch_bounds__(kBlock, LINEAR ? 4 : 8)
+    cq_tile_kernel(const float4 *__restrict__ srec, uint32_t npix, const uint32_t *__restrict__ cs, int ncell, int side,
+                   const Chunk *__restrict__ chunks, const TileTask *__restrict__ tasks, uint32_t ntasks, PairSpec S,
+                   unsigned long long *__restrict__ target, size_t nvox, unsigned long long *__restrict__ dropped,
+                   const uint32_t *__restrict__ plain_flag, int by_parts, uint32_t splits)
+{
+    __shared__ float part_ext[LINEAR ? 1 : 6][LINEAR ? 1 : kTileParts];  // by parts: min a b c, max a b c
+    extern __shared__ unsigned long long box[];  // the plan's largest box
+    const uint32_t split = blockIdx.x % splits, ti = blockIdx.x / splits;
+    const TileTask T = tasks[ti % ntasks];
+    const Chunk CH = chunks[ti / ntasks];
+    const int vbox = T.bx * T.by * T.bz;
+    for (int v = threadIdx.x; v < vbox; v += kBlock) box[v] = 0ull;
+    __syncthreads();
+    // the wave's share of a task's units: contiguous, first by block, then by wave
+    const uint32_t share = split * (kBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t shares = splits * (kBlock / 64);
+    const bool tri = !LINEAR && T.ci == T.cj;
+    const bool fast = T.inbox && plain_flag[0] != 0u, is_signed = T.sa != 0 && T.sb != 0;
+    unsigned long long *const out = target + (size_t)CH.group * nvox;
+    BoxSink sink{box, out, dropped, T.bx0, T.by0, T.bz0, T.bx, T.by, T.bz, S.P.sab, S.P.sc, LINEAR ? 1ull : 2ull,
+                 nullptr, 0, 0, 0};
+    // byte strides of the box, and the centre's byte offset in it
+    const int bx8 = 8 * T.bx, bxby8 = 8 * T.bx * T.by;
+    const int c8 = 8 * (S.P.c0 - T.bx0) + bx8 * (S.P.c1 - T.by0) + bxby8 * (S.P.c2 - T.bz0);
+    const int cab8 = 8 * (S.P.c0 - T.bx0) + bx8 * (S.P.c1 - T.by0);  // in a plane of the box
+    char *const boxb = reinterpret_cast<char *>(box);
+    const float vox = S.P.vox, cut_sq = S.P.cut_sq;
+    const uint32_t lane = threadIdx.x & 63u;
+
+    // the pair's |q|^2 in the order of the k components (records hold them as the mesh's axes)
+    auto norm2 = [&](float qa, float qb, float qc) {
+        const float a2 = qa * qa, b2 = qb * qb, c2 = qc * qc;
+        const float z = S.kc == 2 ? c2 : (S.kb == 2 ? b2 : a2);
+        return ((S.kc == 2 ? a2 : (S.kb == 2 ? a2 : b2)) + (S.kc == 2 ? b2 : c2)) + z;
+    };
+    auto add8 = [&](int o, double x) {
+        atomicAdd(reinterpret_cast<unsigned long long *>(boxb + o), (unsigned long long)(uint32_t)x);
+    };
+    // signed voxel scale and byte stride of the first two axes: q times the first is not negative
+    const float voxa = T.sa < 0 ? -vox : vox, voxb = T.sb < 0 ? -vox : vox;
+    const int sta = T.sa < 0 ? -8 : 8, stb = T.sb < 0 ? -bx8 : bx8;
+    // v_cvt_rpi_i32_f32: floor(x + 1/2) without an intermediate rounding (checked over all floats in
+    // [0, 2^22)), which is round_away of an x >= 0 in one instruction
+    auto round_up = [](float x) {
+        int r;
+        asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+        return r;
+    };
+    // fast: the pair's voxels lie in the box and its value below 2^32; a pair that fails the cut
+    // adds 0 (nearest) or is skipped (linear).  kSigned: q keeps its sign along the first two axes;
+    // kThin: the box is one voxel deep along the third, whose voxel is then the same for all pairs.
+    auto bin_fast = [&](const float4 &a, const f4v &b, auto cut_c, auto signed_c, auto thin_c) {
+        constexpr bool kCut = decltype(cut_c)::value, kSigned = decltype(signed_c)::value;
+        constexpr bool kThin = decltype(thin_c)::value;
+        const float w = a.w * b.w, qa = a.x - b.x, qb = a.y - b.y, qc = a.z - b.z;
+        if (!LINEAR) {
+            const double x = (double)w * S.mult;
+            int o = kSigned ? __mul24(round_up(qb * voxb), stb) + (__mul24(round_up(qa * voxa), sta) + (kThin ? cab8 : c8))
+                            : __mul24(round_away(qb * vox), bx8) + (round_away(qa * vox) * 8 + (kThin ? cab8 : c8));
+            if (!kThin) o += __mul24(round_away(qc * vox), bxby8);
+            add8(o, !kCut || norm2(qa, qb, qc) < cut_sq ? x : 0.0);
+            return;
+        }
+        if (kCut && !(norm2(qa, qb, qc) < cut_sq)) return;
+        const float xa = qa * vox, xb = qb * vox, xc = qc * vox;
+        const float fa = floorf(xa), fb = floorf(xb), fc = floorf(xc);
+        const double sa = (double)(1.0f - (xa - fa)), sb = (double)(1.0f - (xb - fb)), sc = (double)(1.0f - (xc - fc));
+        const double vm = (double)w * S.mult;
+        const int o = __mul24((int)fc, bxby8) + (__mul24((int)fb, bx8) + ((int)fa * 8 + c8));
+        const double p00 = sa * sb, p10 = (1 - sa) * sb, p01 = sa * (1 - sb), p11 = (1 - sa) * (1 - sb), tc = 1 - sc;
+        add8(o, vm * (p00 * sc));
+        add8(o + 8, vm * (p10 * sc));
+        add8(o + bx8, vm * (p01 * sc));
+        add8(o + bx8 + 8, vm * (p11 * sc));
+        add8(o + bxby8, vm * (p00 * tc));
+        add8(o + bxby8 + 8, vm * (p10 * tc));
+        add8(o + bxby8 + bx8, vm * (p01 * tc));
+        add8(o + bxby8 + bx8 + 8, vm * (p11 * tc));
+    };
+    // any pair, through the checked box
+    auto bin_any = [&](const float4 &a, const f4v &b) {
+        auto as_k = [&](float x, float y, float z, float w) {  // mesh axes -> k components
+            return make_float4(S.ka == 0 ? x : (S.kb == 0 ? y : z), S.ka == 1 ? x : (S.kb == 1 ? y : z),
+                               S.ka == 2 ? x : (S.kb == 2 ? y : z), w);
+        };
+        const float4 ra = as_k(a.x, a.y, a.z, a.w), rb = as_k(b.x, b.y, b.z, b.w);
+        if (LINEAR) {
+            bin_ordered<kKindCq>(S, ra, rb, sink);
+        } else {
+            int fs, ms, ss;
+            uint64_t v;
+            if (bin_sym<kKindCq>(S, ra, rb, fs, ms, ss, v)) sink.add(fs, ms, ss, v);
+        }
+    };
+
+    for (uint32_t f = CH.f0; f < CH.f1; f++) {
+        const size_t parts = (size_t)side * side;
+        const uint32_t *csf = cs + f * (ncell * parts + 1);
+        const float4 *rec = srec + (size_t)f * npix;
+        const uint32_t a0 = csf[T.ci * parts], na = csf[(T.ci + 1) * parts] - a0;
+        const uint32_t b0 = csf[T.cj * parts], nb = csf[(T.cj + 1) * parts] - b0;
+        if (na == 0 || nb == 0) continue;
+        const scalar_rec_t brec = (scalar_rec_t)(uintptr_t)(rec + b0);
+        if constexpr (!LINEAR) {
+            if (by_parts && fast && T.allin && !tri) {
+                tile_by_parts(rec, csf, parts, a0, na, T, vox, S.mult, bx8, bxby8, c8, boxb, part_ext, share, shares);
+                continue;
+            }
+        }
+        // units: lane groups of the a records (group gr holds records gr + lane groups) times
+        // runs of kTileB b records
+        const uint32_t groups = (na + 63) / 64, runs = (nb + kTileB - 1) / kTileB;
+        const uint64_t units = (uint64_t)groups * runs;
+        const uint64_t u0 = units * share / shares, u1 = units * (share + 1) / shares;
+        uint32_t gr = (uint32_t)(u0 / runs), run = (uint32_t)(u0 - (uint64_t)gr * runs);
+        uint32_t ia = gr + lane * groups;
+        float4 ra = rec[a0 + min(ia, na - 1)];
+        auto unit = [&](auto edge_c, auto bin) {
+            constexpr bool kEdge = decltype(edge_c)::value;
+            constexpr int kTileBatch = TileBatch<LINEAR>::n;
+#pragma unroll 1
+            for (uint32_t j0 = run * kTileB; j0 < (run + 1) * kTileB; j0 += kTileBatch) {
+                f4v rb[kTileBatch];
+#pragma unroll
+                for (int k = 0; k < kTileBatch; k++) rb[k] = brec[kEdge ? min(j0 + k, nb - 1) : j0 + k];
+#pragma unroll
+                for (int k = 0; k < kTileBatch; k++) {
+                    // tri: each unordered pair of distinct records once
+                    if (kEdge && (j0 + k >= nb || (tri && j0 + k <= ia))) continue;
+                    bin(ra, rb[k]);
+                }
+            }
+        };
+        using T_ = std::true_type;
+        using F_ = std::false_type;
+        for (uint64_t u = u0; u < u1; u++) {
+            if (ia < na) {
+                const bool edge = tri || (run + 1) * kTileB > nb;
+                auto go = [&](auto edge_c, auto cut_c, auto signed_c, auto thin_c) {
+                    unit(edge_c, [&](const float4 &a, const f4v &b) { bin_fast(a, b, cut_c, signed_c, thin_c); });
+                };
+                if (!fast) {
+                    unit(T_{}, bin_any);
+                } else if (edge) {
+                    go(T_{}, T_{}, F_{}, F_{});
+                } else if (LINEAR) {
+                    if (T.allin) go(F_{}, F_{}, F_{}, F_{}); else go(F_{}, T_{}, F_{}, F_{});
+                } else if (T.allin && is_signed) {
+                    if (T.bz == 1) go(F_{}, F_{}, T_{}, T_{}); else go(F_{}, F_{}, T_{}, F_{});
+                } else if (T.allin) {
+                    go(F_{}, F_{}, F_{}, F_{});
+                } else {
+                    go(F_{}, T_{}, F_{}, F_{});
+                }
+            }
+            if (++run == runs) {
+                run = 0;
+                ia = ++gr + lane * groups;
+                ra = rec[a0 + min(ia, na - 1)];
+            }
+        }
+    }
+    __syncthreads();
+    for (int v = threadIdx.x; v < vbox; v += kBlock) {
+        const unsigned long long x = box[v];
+        if (!x) continue;
+        const int fs = T.bx0 + v % T.bx, ms = T.by0 + v / T.bx % T.by, ss = T.bz0 + v / (T.bx * T.by);
+        atomicAdd(out + (size_t)fs + (size_t)ms * S.P.sab + (size_t)ss * S.P.sab * S.P.sab, x);
+    }
+}
+
 // ---- host planning ---------------------------------------------------------------
 
 // The specialised pair path: AC_uw, symmetric (nearest-neighbour) binning, identity
@@ -1335,6 +1797,11 @@ struct iac_pair_plan {
     // product
     std::vector<iac::Task> tasks;
     iac::Task *d_tasks = nullptr;
+    // region tiles (region == kRegionTiles): their tasks, and whether nearly all have a box
+    std::vector<iac::TileTask> tiles;
+    iac::TileTask *d_tiles = nullptr;
+    bool tiles_fit = false;
+    size_t tile_box = 0;  // voxels of the largest box
     int pins = 0;  // frame queues holding this plan (never evicted while > 0)
 };
 
@@ -1462,37 +1929,106 @@ iac_pair_plan *find_plan(iac_ctx *ctx, const float *kmap, uint32_t npix, int cel
     return nullptr;
 }
 
-// Cell grid of the k-map (two host round trips for the extents) and the task
-// table, from the context's cache when the geometry matches.
-int get_plan(iac_ctx *ctx, hipStream_t st, const PairRun &R, int cell_vox, int box_cap, int region,
-             iac_pair_plan **out)
+constexpr int kRegionTiles = -1;  // iac_pair_plan::region of a region-tile plan
+
+// Tasks of the region tiles: pairs of regions (ci <= cj, or all ordered pairs of linear runs) that
+// are not wholly beyond the cut, with the box of their voxels (linear: of their corners).
+void build_tiles(iac_pair_plan &pl, bool ordered)
 {
-    const PairSpec &S = R.spec;
-    void *ext = nullptr;
-    IAC_TRY(scratch(ctx, 3, (6 + 6 * (size_t)kMaxCells) * sizeof(uint32_t), &ext));
-    uint32_t *d_ext = static_cast<uint32_t *>(ext);
+    const CellGeom &g = pl.g;
+    const PairSpec &S = pl.spec;
+    const int nc = g.ncu * g.ncv, cax[3] = {S.ka, S.kb, S.kc};
+    const int cen[3] = {S.P.c0, S.P.c1, S.P.c2}, dim[3] = {S.P.sab, S.P.sab, S.P.sc};
+    const long cap = pl.box_cap;
+    const double maxq = std::sqrt((double)S.P.cut_sq);
+    size_t boxed = 0;
+    for (int ci = 0; ci < nc; ci++) {
+        const uint32_t *ea = &pl.cell_ext[6 * (size_t)ci];
+        if (ea[0] == 0xffffffffu) continue;  // no pixel there
+        for (int cj = ordered ? 0 : ci; cj < nc; cj++) {
+            const uint32_t *eb = &pl.cell_ext[6 * (size_t)cj];
+            if (eb[0] == 0xffffffffu) continue;
+            double qlo[3], qhi[3], near2 = 0, far2 = 0;
+            for (int d = 0; d < 3; d++) {
+                qlo[d] = (double)unkey(ea[d]) - unkey(eb[3 + d]);
+                qhi[d] = (double)unkey(ea[3 + d]) - unkey(eb[d]);
+                const double m = qlo[d] > 0 ? qlo[d] : (qhi[d] < 0 ? -qhi[d] : 0.0);
+                near2 += m * m;
+                far2 += std::max(qlo[d] * qlo[d], qhi[d] * qhi[d]);
+            }
+            if (std::sqrt(near2) > maxq * (1.0 + 1e-5) + 1e-7) continue;
+            TileTask t{};
+            t.ci = ci;
+            t.cj = cj;
+            auto sign = [&](int d) { return qlo[d] >= 0.0 ? 1 : (qhi[d] <= 0.0 ? -1 : 0); };
+            t.sa = sign(S.ka);
+            t.sb = sign(S.kb);
+            t.allin = far2 * (1.0 + 1e-5) < (double)S.P.cut_sq ? 1 : 0;
+            // voxels round_away(x), or corners floor(x) and floor(x) + 1, of x within eps of
+            // [l, h] (two float roundings)
+            int lo[3], ext[3];
+            bool box = true, inside = true;
+            double vol = 1;
+            for (int m = 0; m < 3; m++) {
+                const double l = qlo[cax[m]] * S.P.vox, h = qhi[cax[m]] * S.P.vox;
+                const double eps = 1e-3 + 1e-6 * std::max(std::fabs(l), std::fabs(h));
+                const double v0 = (ordered ? std::floor(l - eps) : std::ceil(l - eps - 0.5)) + cen[m];
+                const double v1 = (ordered ? std::floor(h + eps) + 1 : std::floor(h + eps + 0.5)) + cen[m];
+                inside = inside && v0 >= 0.0 && v1 <= (double)dim[m] - 1;  // false for NaN
+                const double c0 = std::max(0.0, v0), c1 = std::min((double)dim[m] - 1, v1);
+                box = box && c1 >= c0;
+                vol *= c1 - c0 + 1;
+                lo[m] = box ? (int)c0 : 0;
+                ext[m] = box ? (int)(c1 - c0) + 1 : 0;
+            }
+            if (box && vol <= (double)cap) {
+                t.inbox = inside ? 1 : 0;
+                t.bx0 = lo[0];
+                t.by0 = lo[1];
+                t.bz0 = lo[2];
+                t.bx = ext[0];
+                t.by = ext[1];
+                t.bz = ext[2];
+                pl.tile_box = std::max(pl.tile_box, (size_t)t.bx * t.by * t.bz);
+                boxed++;
+            }
+            pl.tiles.push_back(t);
+        }
+    }
+    pl.tiles_fit = !pl.tiles.empty() && boxed >= pl.tiles.size() - pl.tiles.size() / 32;
+}
+
+// Extents of the k-map (one host round trip).
+int kmap_extents(iac_ctx *ctx, hipStream_t st, const float *d_kmap, uint32_t npix, uint32_t *d_ext, float kmin[3],
+                 float ext3[3])
+{
     hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, d_ext, 0xffffffffu, (size_t)3);
     hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, d_ext + 3, 0u, (size_t)3);
-    const unsigned eb = std::max(1u, std::min<unsigned>(1024, (R.npix + 255) / 256));
+    const unsigned eb = std::max(1u, std::min<unsigned>(64, (npix + 255) / 256));
     // few blocks: the six extent words take one atomic per wave, all on the same addresses
-    hipLaunchKernelGGL(kext_kernel, dim3(std::min(eb, 64u)), dim3(256), 0, st, R.d_kmap, R.npix, d_ext);
+    hipLaunchKernelGGL(kext_kernel, dim3(eb), dim3(256), 0, st, d_kmap, npix, d_ext);
     IAC_HIP(hipGetLastError());
     uint32_t hext[6];
     IAC_HIP(hipMemcpyAsync(hext, d_ext, sizeof(hext), hipMemcpyDeviceToHost, st));
     IAC_HIP(hipStreamSynchronize(st));
-    float kmin[3], ext3[3];
     for (int d = 0; d < 3; d++) {
         kmin[d] = unkey(hext[d]);
         ext3[d] = unkey(hext[3 + d]) - kmin[d];
     }
+    return IAC_OK;
+}
+
+// The grid of cells cell_vox % 1000 (u) by cell_vox / 1000 (v, 0: as u) voxels over the two widest
+// axes, larger where it would exceed kMaxCells.
+CellGeom cell_grid(const float kmin[3], const float ext3[3], float vox, int cell_vox)
+{
     CellGeom g{};
     int order[3] = {0, 1, 2};
     std::sort(order, order + 3, [&](int a, int b) { return ext3[a] > ext3[b]; });
     g.au = std::min(order[0], order[1]);
     g.av = std::max(order[0], order[1]);
-    // cell_vox = u side + 1000 * v side (voxels); cells may be longer along u
-    double wu = (double)(cell_vox % 1000) / (double)S.P.vox;
-    double wv = (double)(cell_vox / 1000 ? cell_vox / 1000 : cell_vox % 1000) / (double)S.P.vox;
+    double wu = (double)(cell_vox % 1000) / (double)vox;
+    double wv = (double)(cell_vox / 1000 ? cell_vox / 1000 : cell_vox % 1000) / (double)vox;
     auto ncells = [&](int a, double w) { return std::max(1, (int)std::ceil(ext3[a] / w * (1 + 1e-6))); };
     while ((long)ncells(g.au, wu) * ncells(g.av, wv) > kMaxCells) {
         wu *= 1.25;
@@ -1504,19 +2040,34 @@ int get_plan(iac_ctx *ctx, hipStream_t st, const PairRun &R, int cell_vox, int b
     g.v0 = kmin[g.av];
     g.ncu = ncells(g.au, wu);
     g.ncv = ncells(g.av, wv);
+    return g;
+}
+
+// Enqueues the per-cell extents of the k-map and their copy to cext (read it after a sync).
+int cell_extents(hipStream_t st, const float *d_kmap, uint32_t npix, const CellGeom &g, uint32_t *d_cell_ext,
+                 std::vector<uint32_t> &cext)
+{
     const int nc = g.ncu * g.ncv;
-    hipLaunchKernelGGL(init_cell_ext_kernel, dim3((nc + 255) / 256), dim3(256), 0, st, d_ext + 6, nc);
+    hipLaunchKernelGGL(init_cell_ext_kernel, dim3((nc + 255) / 256), dim3(256), 0, st, d_cell_ext, nc);
     const size_t lds = 6 * sizeof(uint32_t) * (size_t)nc;
     if (lds <= 48 * 1024) {
-        const unsigned lb = std::max(1u, std::min<unsigned>(512, (R.npix + 4095) / 4096));
-        hipLaunchKernelGGL(cell_ext_lds_kernel, dim3(lb), dim3(256), lds, st, R.d_kmap, R.npix, g, d_ext + 6);
+        const unsigned lb = std::max(1u, std::min<unsigned>(512, (npix + 4095) / 4096));
+        hipLaunchKernelGGL(cell_ext_lds_kernel, dim3(lb), dim3(256), lds, st, d_kmap, npix, g, d_cell_ext);
     } else {
-        hipLaunchKernelGGL(cell_ext_kernel, dim3(eb), dim3(256), 0, st, R.d_kmap, R.npix, g, d_ext + 6);
+        const unsigned eb = std::max(1u, std::min<unsigned>(1024, (npix + 255) / 256));
+        hipLaunchKernelGGL(cell_ext_kernel, dim3(eb), dim3(256), 0, st, d_kmap, npix, g, d_cell_ext);
     }
     IAC_HIP(hipGetLastError());
-    std::vector<uint32_t> cext(6 * (size_t)nc);
-    IAC_HIP(hipMemcpyAsync(cext.data(), d_ext + 6, cext.size() * 4, hipMemcpyDeviceToHost, st));
-    IAC_HIP(hipStreamSynchronize(st));
+    cext.resize(6 * (size_t)nc);
+    IAC_HIP(hipMemcpyAsync(cext.data(), d_cell_ext, cext.size() * 4, hipMemcpyDeviceToHost, st));
+    return IAC_OK;
+}
+
+// The plan of a grid and its cell extents, from the context's cache or made.
+int plan_of(iac_ctx *ctx, const PairRun &R, int cell_vox, int box_cap, int region, const CellGeom &g,
+            std::vector<uint32_t> &cext, iac_pair_plan **out)
+{
+    const PairSpec &S = R.spec;
     iac_pair_plan *pl = find_plan(ctx, R.d_kmap, R.npix, cell_vox, box_cap, region, S);
     if (pl && (std::memcmp(&pl->g, &g, sizeof(g)) != 0 || pl->cell_ext != cext)) pl = nullptr;
     if (!pl) {
@@ -1525,6 +2076,7 @@ int get_plan(iac_ctx *ctx, hipStream_t st, const PairRun &R, int cell_vox, int b
             for (auto it = ctx->pair_plans.begin(); it != ctx->pair_plans.end(); ++it) {
                 if ((*it)->pins > 0) continue;
                 if ((*it)->d_tasks) IAC_HIP(hipFree((*it)->d_tasks));
+                if ((*it)->d_tiles) IAC_HIP(hipFree((*it)->d_tiles));
                 delete *it;
                 ctx->pair_plans.erase(it);
                 break;
@@ -1540,18 +2092,45 @@ int get_plan(iac_ctx *ctx, hipStream_t st, const PairRun &R, int cell_vox, int b
         pl->spec = S;
         pl->g = g;
         pl->cell_ext.swap(cext);
-        build_tasks(*pl, R.ordered);
-        if (pl->tasks.size() > kMaxGridBlocks)
-            return fail(IAC_ERR_LIMIT, "pair engine: more than 2^22 tasks (raise the task region or the cell size)");
-        if (!pl->tasks.empty()) {
-            IAC_HIP(hipMalloc(&pl->d_tasks, pl->tasks.size() * sizeof(Task)));
-            IAC_HIP(hipMemcpy(pl->d_tasks, pl->tasks.data(), pl->tasks.size() * sizeof(Task),
-                              hipMemcpyHostToDevice));
+        if (region == kRegionTiles) {
+            build_tiles(*pl, R.ordered);
+            if (pl->tiles_fit) {
+                IAC_HIP(hipMalloc(&pl->d_tiles, pl->tiles.size() * sizeof(TileTask)));
+                IAC_HIP(hipMemcpy(pl->d_tiles, pl->tiles.data(), pl->tiles.size() * sizeof(TileTask),
+                                  hipMemcpyHostToDevice));
+            }
+        } else {
+            build_tasks(*pl, R.ordered);
+            if (pl->tasks.size() > kMaxGridBlocks)
+                return fail(IAC_ERR_LIMIT,
+                            "pair engine: more than 2^22 tasks (raise the task region or the cell size)");
+            if (!pl->tasks.empty()) {
+                IAC_HIP(hipMalloc(&pl->d_tasks, pl->tasks.size() * sizeof(Task)));
+                IAC_HIP(hipMemcpy(pl->d_tasks, pl->tasks.data(), pl->tasks.size() * sizeof(Task),
+                                  hipMemcpyHostToDevice));
+            }
         }
         pl->valid = true;
     }
     *out = pl;
     return IAC_OK;
+}
+
+// Cell grid of the k-map (two host round trips for the extents) and the task
+// table, from the context's cache when the geometry matches.
+int get_plan(iac_ctx *ctx, hipStream_t st, const PairRun &R, int cell_vox, int box_cap, int region,
+             iac_pair_plan **out)
+{
+    void *ext = nullptr;
+    IAC_TRY(scratch(ctx, 3, (6 + 6 * (size_t)kMaxCells) * sizeof(uint32_t), &ext));
+    uint32_t *d_ext = static_cast<uint32_t *>(ext);
+    float kmin[3], ext3[3];
+    IAC_TRY(kmap_extents(ctx, st, R.d_kmap, R.npix, d_ext, kmin, ext3));
+    const CellGeom g = cell_grid(kmin, ext3, R.spec.P.vox, cell_vox);
+    std::vector<uint32_t> cext;
+    IAC_TRY(cell_extents(st, R.d_kmap, R.npix, g, d_ext + 6, cext));
+    IAC_HIP(hipStreamSynchronize(st));
+    return plan_of(ctx, R, cell_vox, box_cap, region, g, cext, out);
 }
 
 // Frame chunks inside each group, balanced by pair work: a chunk closes once its
@@ -1779,6 +2358,7 @@ void free_pair_plans(iac_ctx *ctx)
 {
     for (auto *p : ctx->pair_plans) {
         if (p->d_tasks) (void)hipFree(p->d_tasks);
+        if (p->d_tiles) (void)hipFree(p->d_tiles);
         delete p;
     }
     ctx->pair_plans.clear();
@@ -1820,6 +2400,140 @@ int pairs_run(iac_ctx *ctx, const PairRun &R)
         IAC_HIP(hipMemcpyAsync(b.d_chunks, chunks.data(), chunks.size() * sizeof(Chunk), hipMemcpyHostToDevice, st));
     IAC_HIP(hipStreamSynchronize(st));  // the host arrays above are released on return
     return enqueue(ctx, st, R, b, true);
+}
+
+// ---- dense C(q) -----------------------------------------------------------------
+
+// Region side in voxels: the largest of these that makes kTileTasks tasks or more (smaller regions
+// flush more boxes per pair).
+constexpr int kTileSides[] = {12, 8, 6, 4};
+constexpr double kTileTasks = 2048;
+// mean records per region and frame below which most of a wave's 64 lanes idle and the engine's
+// pair ranges take the run
+constexpr double kTileRecords = 32;
+// Blocks wanted, and the least pairs per block: a 350 x 350 image into 35 x 35 x 3 has 325 tasks
+// of 2.4e7 pairs and takes 46 ms with one block each, 7 ms split (384 x 360 into 129 x 129 x 3,
+// 2,080 tasks of 5.3e6: 8.6 and 6.1 ms).
+constexpr double kTileBlocks = 16384, kTileShare = 65536;
+// Mean records per voxel-sized part from which tasks add up parts in registers, pair by pair
+// below: 12.1 against 10.5 ms at 16 records (eight 256^2 images into 129 x 129 x 3), 5.6 against
+// 6.1 ms at 33 (384 x 360), 5.1 against 7.0 ms at 306 (350 x 350 into 35 x 35 x 3).
+constexpr double kPartRecords = 24;
+
+int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *done)
+{
+    *done = false;
+    const PairSpec &S = R.spec;
+    const bool ordered = R.ordered;
+    // the engine's options select the engine
+    if (ctx->pair_mode || ctx->cell_vox || ctx->cell_vox_v || ctx->box_cap || ctx->task_region || ctx->pair_prefetch ||
+        ctx->frame_chunk)
+        return IAC_OK;
+    // round_away and the boxes' 24-bit products need |q vox| < 2^22
+    if (!(std::sqrt((double)S.P.cut_sq) * S.P.vox < 4194304.0) || R.nframes == 0) return IAC_OK;
+    hipStream_t st = ctx->stream;
+    void *ext = nullptr;
+    IAC_TRY(scratch(ctx, 3, (6 + 6 * (size_t)kMaxCells) * sizeof(uint32_t), &ext));
+    uint32_t *d_ext = static_cast<uint32_t *>(ext);
+    float kmin[3], ext3[3];
+    IAC_TRY(kmap_extents(ctx, st, R.d_kmap, R.npix, d_ext, kmin, ext3));
+    const int box_cap = ordered ? kBoxMax : kBoxSmall;
+    const size_t nvox = (size_t)S.P.sab * S.P.sab * S.P.sc;
+    const uint32_t ns = std::min<uint32_t>(256, (R.npix + kBlock - 1) / kBlock);  // sort blocks per frame
+    if ((uint64_t)ns * R.nframes > 0x7fffffffull) return IAC_OK;
+    for (size_t k = 0; k < sizeof(kTileSides) / sizeof(kTileSides[0]); k++) {
+        const int side = kTileSides[k];
+        const CellGeom g = cell_grid(kmin, ext3, S.P.vox, side);
+        const int nc = g.ncu * g.ncv;
+        const double ntask = ordered ? (double)nc * nc : 0.5 * nc * (nc + 1.0);
+        if (ntask > kMaxGridBlocks) return IAC_OK;
+        if (ntask * R.ngroups < kTileTasks && k + 1 < sizeof(kTileSides) / sizeof(kTileSides[0])) continue;
+        // chunks: a group's frames in as many blocks as fill the chip
+        const uint32_t split = (uint32_t)std::max(1.0, std::ceil(kTileTasks / (ntask * R.ngroups)));
+        std::vector<Chunk> chunks;
+        for (uint32_t gi = 0; gi < R.ngroups; gi++) {
+            const uint32_t f0 = R.h_group_off[gi], n = R.h_group_off[gi + 1] - f0, parts = std::min(split, n);
+            for (uint32_t c = 0; c < parts; c++)
+                chunks.push_back(Chunk{f0 + (uint32_t)((uint64_t)n * c / parts),
+                                       f0 + (uint32_t)((uint64_t)n * (c + 1) / parts), gi});
+        }
+        auto up = [](size_t x) { return (x + 255) / 256 * 256; };
+        // records | region starts | cursors (slot 1); half meshes | group offsets | self, kept, flag | chunks (slot 2)
+        const size_t nkey = (size_t)nc * side * side;
+        const size_t brec = up((size_t)R.npix * R.nframes * sizeof(float4)),
+                     bcs = up(R.nframes * (nkey + 1) * sizeof(uint32_t)),
+                     bcur = up(R.nframes * nkey * sizeof(uint32_t));
+        const size_t bh = ordered ? 0 : up(nvox * R.ngroups * sizeof(unsigned long long)),
+                     bg = up((R.ngroups + 1) * sizeof(uint32_t)), bs = up((R.ngroups + 2) * sizeof(unsigned long long));
+        void *s1 = nullptr, *s2 = nullptr;
+        IAC_TRY(scratch(ctx, 1, brec + bcs + bcur, &s1));
+        IAC_TRY(scratch(ctx, 2, bh + bg + bs + chunks.size() * sizeof(Chunk) + 256, &s2));
+        char *p1 = static_cast<char *>(s1), *p2 = static_cast<char *>(s2);
+        auto *srec = reinterpret_cast<float4 *>(p1);
+        auto *cs = reinterpret_cast<uint32_t *>(p1 + brec);
+        auto *cursor = reinterpret_cast<uint32_t *>(p1 + brec + bcs);
+        auto *H = reinterpret_cast<unsigned long long *>(p2);
+        auto *d_goff = reinterpret_cast<uint32_t *>(p2 + bh);
+        auto *d_self = reinterpret_cast<unsigned long long *>(p2 + bh + bg);
+        auto *d_kept = d_self + R.ngroups;
+        auto *d_plain = reinterpret_cast<uint32_t *>(d_kept + 1);
+        auto *d_chunks = reinterpret_cast<Chunk *>(p2 + bh + bg + bs);
+        IAC_HIP(hipMemcpyAsync(d_goff, R.h_group_off, (R.ngroups + 1) * sizeof(uint32_t), hipMemcpyHostToDevice, st));
+        IAC_HIP(hipMemcpyAsync(d_chunks, chunks.data(), chunks.size() * sizeof(Chunk), hipMemcpyHostToDevice, st));
+        std::vector<uint32_t> cext;
+        IAC_TRY(cell_extents(st, R.d_kmap, R.npix, g, d_ext + 6, cext));
+        auto blocks = [](size_t n) { return (unsigned)std::max<size_t>(1, std::min<size_t>(4096, (n + 255) / 256)); };
+        const size_t ncs = R.nframes * (nkey + 1);
+        hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks(ncs)), dim3(256), 0, st, cs, 0u, ncs);
+        hipLaunchKernelGGL(fill_u64_kernel, dim3(blocks(R.ngroups + 1)), dim3(256), 0, st, d_self, (size_t)R.ngroups + 1);
+        hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, d_plain, 1u, (size_t)1);
+        const unsigned sblocks = ns * R.nframes;
+        hipLaunchKernelGGL(ordered ? tile_count_kernel<true> : tile_count_kernel<false>, dim3(sblocks), dim3(kBlock), 0,
+                           st, R.d_kmap, d_frames, R.npix, ns, g, side, S, d_goff, R.ngroups, cs, d_self, d_plain,
+                           d_kept);
+        hipLaunchKernelGGL(tile_scan_kernel, dim3(R.nframes), dim3(1024), 0, st, cs, cursor, (uint32_t)nkey);
+        hipLaunchKernelGGL(tile_scatter_kernel, dim3(sblocks), dim3(kBlock), 0, st, R.d_kmap, d_frames, R.npix, ns, g,
+                           side, S.ka, S.kb, S.kc, cursor, srec);
+        if (!ordered)
+            hipLaunchKernelGGL(fill_u64_kernel, dim3(blocks(nvox * R.ngroups)), dim3(256), 0, st, H, nvox * R.ngroups);
+        IAC_HIP(hipGetLastError());
+        unsigned long long kept = 0;
+        IAC_HIP(hipMemcpyAsync(&kept, d_kept, sizeof(kept), hipMemcpyDeviceToHost, st));
+        IAC_HIP(hipStreamSynchronize(st));  // also releases the host arrays copied above
+        if ((double)kept < kTileRecords * (double)R.nframes * nc) return IAC_OK;  // sparse frames
+        iac_pair_plan *pl = nullptr;
+        IAC_TRY(plan_of(ctx, R, side, box_cap, kRegionTiles, g, cext, &pl));
+        if (!pl->tiles_fit) continue;
+        const bool by_parts = !ordered && (double)kept >= kPartRecords * (double)R.nframes * (double)nkey;
+        auto *target = ordered ? reinterpret_cast<unsigned long long *>(R.d_mesh) : H;
+        const uint32_t ntasks = (uint32_t)pl->tiles.size(), nchunks = (uint32_t)chunks.size();
+        // few tasks, or tasks of uneven work (dense regions, regions with themselves): several blocks
+        // each, of at least kTileShare pairs
+        const double recs = (double)kept / ((double)R.nframes * nc);
+        const double pairs = recs * recs * std::max(1.0, (double)R.nframes / nchunks);
+        const uint32_t splits = (uint32_t)std::max(
+            1.0, std::min({std::ceil(kTileBlocks / ((double)ntasks * nchunks)), pairs / kTileShare, 4096.0}));
+        const uint32_t per = std::max<uint32_t>(1, kMaxGridBlocks / ((uint64_t)ntasks * splits));
+        IAC_TRY(timer_begin(ctx));
+        for (uint32_t c0 = 0; c0 < nchunks; c0 += per) {
+            const dim3 grid(ntasks * splits * std::min(per, nchunks - c0));
+            hipLaunchKernelGGL(ordered ? cq_tile_kernel<true> : cq_tile_kernel<false>, grid, dim3(kBlock),
+                               pl->tile_box * sizeof(unsigned long long), st, srec,
+                               R.npix, cs, nc, side, d_chunks + c0, pl->d_tiles, ntasks, S, target, nvox, ctx->d_counters,
+                               d_plain, by_parts ? 1 : 0, splits);
+            IAC_HIP(hipGetLastError());
+        }
+        IAC_TRY(timer_end(ctx));
+        if (!ordered) {
+            const size_t centre = (size_t)S.P.c0 + (size_t)S.P.c1 * S.P.sab + (size_t)S.P.c2 * S.P.sab * S.P.sab;
+            hipLaunchKernelGGL(symmetrize_kernel, dim3(blocks(nvox * R.ngroups)), dim3(256), 0, st, H,
+                               reinterpret_cast<unsigned long long *>(R.d_mesh), nvox, R.ngroups, centre, d_self);
+            IAC_HIP(hipGetLastError());
+        }
+        *done = true;
+        return IAC_OK;
+    }
+    return IAC_OK;
 }
 
 // ---- prepared runs -----------------------------------------------------------

@@ -373,3 +373,46 @@ def test_merge_bricks_vs_oracle(ctx, dev, axes, sab, sc, nev, interp):
         call(torch.from_numpy(small if multi else small[0]).to(dev), s, to_dev(rw, dev), interp, mult, big)
         assert np.array_equal(mesh_np(big), ref)
         assert ctx.dropped() - before == drop
+
+
+@pytest.mark.parametrize("rows,cols,dist,edge", [(9, 9, 2e4, 5), (40, 31, 3e4, 17), (64, 64, 5e5, 63), (90, 33, 1e5, 31),
+                                                 (130, 120, 5e5, 31), (70, 70, 4e3, 41), (33, 140, 2e4, 127)])
+@pytest.mark.parametrize("axes", [((1, 0, 0), (0, 1, 0)), ((0, 0, 1), (0, 1, 0))])
+@pytest.mark.parametrize("interp", [0, 1])
+def test_cq_region_tiles_vs_engine(dev, rows, cols, dist, edge, axes, interp):
+    """Dense C(q) by region tiles against the cell-offset engine (which its options select), equal
+    in every voxel and in the count of dropped updates: detectors facing each axis, near (regions
+    deep along the beam) and far, meshes coarser and finer than the pixels, a zoom that cuts
+    pairs, images with zeros, with negative values and values past 2^32, several frames in groups."""
+    import torch
+
+    import incohautocorrelate_amd as iac
+
+    rng = np.random.default_rng(rows * 7 + cols)
+    centre = [0, 0, dist] if axes[0] == (1, 0, 0) else [dist, 0, 0]
+    _, (km, _, _, mq) = None, iac.calc_kmap(iac.generate_pixel_map(rows, cols, 75.0, centre, axes[0], axes[1]))
+    npix = rows * cols
+    base = rng.gamma(1.0, 0.5, (5, npix)).astype(np.float32)
+    zeros = base * (rng.random((5, npix)) > 0.3)
+    kinds = {"plain": (base, 1e6), "zeros": (zeros, 1e6), "negative": (base - np.float32(0.2), 1e6), "large": (base, 1e11)}
+    a, b = iac.Context(0), iac.Context(0)
+    try:
+        b.set_option(iac.OPT_PAIR_MODE, 2)
+        for zoom in (1.0, 1.7):
+            s = iac.mesh_shape_small_cofq(mq, edge, zoom)
+            nvox = s.size_ab ** 2 * s.size_c
+            for kind, (fr, mult) in kinds.items():
+                for goff in ([0, 1], [0, 2, 5]):
+                    d = to_dev(fr[: goff[-1]], dev)
+                    got, drop = [], []
+                    for c in (a, b):
+                        m = _zeros((len(goff) - 1) * nvox, dev)
+                        before = c.dropped()
+                        c.cq_dense_frames(to_dev(km, dev), d, goff, s, m, interp, mult)
+                        got.append(m)
+                        drop.append(c.dropped() - before)
+                    assert torch.equal(got[0], got[1]), (zoom, kind, goff)
+                    assert drop[0] == drop[1], (zoom, kind, goff)
+    finally:
+        a.close()
+        b.close()
