@@ -55,6 +55,41 @@ int scratch(iac_ctx *ctx, int slot, size_t bytes, void **out)
     return IAC_OK;
 }
 
+static constexpr size_t kPinnedPart[2] = {192 * 1024, 64 * 1024};
+
+int pinned(iac_ctx *ctx, int slot, size_t bytes, void **out)
+{
+    if (slot == 1) {
+        if (!ctx->uploaded) IAC_HIP(hipEventCreateWithFlags(&ctx->uploaded, hipEventDisableTiming));
+        else IAC_HIP(hipEventSynchronize(ctx->uploaded));
+    }
+    if (!ctx->pinned_base) {
+        IAC_HIP(hipHostMalloc(&ctx->pinned_base, kPinnedPart[0] + kPinnedPart[1], hipHostMallocDefault));
+        ctx->pinned[0] = ctx->pinned_base;
+        ctx->pinned[1] = static_cast<char *>(ctx->pinned_base) + kPinnedPart[0];
+        for (int i = 0; i < 2; i++) ctx->pinned_bytes[i] = kPinnedPart[i];
+    }
+    if (ctx->pinned_bytes[slot] < bytes) {
+        const size_t want = bytes + bytes / 2;  // grow with headroom
+        void *grown = nullptr;
+        IAC_HIP(hipHostMalloc(&grown, want, hipHostMallocDefault));
+        if (ctx->pinned_bytes[slot] > kPinnedPart[slot]) {  // an allocation of its own
+            (void)hipStreamSynchronize(ctx->stream);
+            (void)hipHostFree(ctx->pinned[slot]);
+        }
+        ctx->pinned[slot] = grown;
+        ctx->pinned_bytes[slot] = want;
+    }
+    *out = ctx->pinned[slot];
+    return IAC_OK;
+}
+
+int upload_done(iac_ctx *ctx)
+{
+    IAC_HIP(hipEventRecord(ctx->uploaded, ctx->stream));
+    return IAC_OK;
+}
+
 int timer_begin(iac_ctx *ctx)
 {
     if (!ctx->timing) return IAC_OK;
@@ -159,6 +194,14 @@ int iac_ctx_destroy(iac_ctx *ctx)
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     for (int i = 0; i < 4; i++)
         if (ctx->scratch[i]) (void)hipFree(ctx->scratch[i]);
+    if (ctx->uploaded) {
+        (void)hipEventSynchronize(ctx->uploaded);
+        (void)hipEventDestroy(ctx->uploaded);
+    }
+    for (int i = 0; i < 2; i++)
+        if (ctx->pinned_bytes[i] > iac::kPinnedPart[i])  // an allocation of its own
+            (void)hipHostFree(ctx->pinned[i]);
+    if (ctx->pinned_base) (void)hipHostFree(ctx->pinned_base);
     iac::free_pair_plans(ctx);
     iac::free_sim_resources(ctx);
     for (auto e : ctx->ev_start) (void)hipEventDestroy(e);

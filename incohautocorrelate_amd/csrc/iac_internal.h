@@ -22,6 +22,13 @@ struct iac_ctx {
     // growable scratch arenas (device); each call may reuse them
     void *scratch[4] = {nullptr, nullptr, nullptr, nullptr};
     size_t scratch_bytes[4] = {0, 0, 0, 0};
+    // page-locked staging: [0] read-backs of a call (valid until its next one), [1] its uploads,
+    // rewritten once the event behind the last of them is done
+    // (both in one allocation until one outgrows its part)
+    void *pinned_base = nullptr;
+    void *pinned[2] = {nullptr, nullptr};
+    size_t pinned_bytes[2] = {0, 0};
+    hipEvent_t uploaded = nullptr;
     // measurement: event pairs around the dominant kernel of each call
     bool timing = false;
     std::vector<hipEvent_t> ev_start, ev_stop;
@@ -60,6 +67,11 @@ int hip_fail(hipError_t e, const char *what, const char *file, int line);
 int bind(iac_ctx *ctx);
 // Ensures scratch arena `slot` holds at least `bytes`; returns its pointer in *out.
 int scratch(iac_ctx *ctx, int slot, size_t bytes, void **out);
+
+// Page-locked staging of at least `bytes`; slot 1 waits until its last uploads have been read
+// (upload_done marks them on the context's stream).
+int pinned(iac_ctx *ctx, int slot, size_t bytes, void **out);
+int upload_done(iac_ctx *ctx);
 
 // Brackets the dominant kernel of a call when timing is enabled.
 int timer_begin(iac_ctx *ctx);

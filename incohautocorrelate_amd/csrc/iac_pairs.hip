@@ -141,6 +141,15 @@ __device__ __forceinline__ int round_away(float x)
     return (int)(x + copysignf(0.49999997f, x));
 }
 
+// round_away of an x in [0, 2^22) in one instruction: v_cvt_rpi_i32_f32 is floor(x + 1/2) without an
+// intermediate rounding (checked over all floats of that range)
+__device__ __forceinline__ int round_up(float x)
+{
+    int r;
+    asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(x));
+    return r;
+}
+
 // pair_val with the integer fast path in a 24-bit multiply
 __device__ __forceinline__ uint32_t pair_val_small(float p)
 {
@@ -277,32 +286,39 @@ __global__ void init_cell_ext_kernel(uint32_t *ext, int ncell)
         }
 }
 
-// min/max of each k component: ext[0..2] min keys, ext[3..5] max keys; reduced over
-// the wave by shuffles, then one atomic per wave and component
+// min/max of each k component: ext[0..2] min keys, ext[3..5] max keys, reduced over the block: all
+// blocks' atomics fall on these six words (one per wave took 20 us for 16,384 pixels, so 2 us)
 __global__ void __launch_bounds__(256) kext_kernel(const float *__restrict__ kmap, uint32_t npix, uint32_t *ext)
 {
-    uint32_t mn[3] = {0xffffffffu, 0xffffffffu, 0xffffffffu}, mx[3] = {0u, 0u, 0u};
+    __shared__ uint32_t red[4][6];
+    uint32_t m[6] = {0xffffffffu, 0xffffffffu, 0xffffffffu, 0u, 0u, 0u};
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < npix; i += gridDim.x * blockDim.x)
         for (int d = 0; d < 3; d++) {
             const uint32_t k = fkey(kmap[3 * (size_t)i + d]);
-            mn[d] = min(mn[d], k);
-            mx[d] = max(mx[d], k);
+            m[d] = min(m[d], k);
+            m[3 + d] = max(m[3 + d], k);
         }
-    for (int d = 0; d < 3; d++)
+    for (int d = 0; d < 6; d++)
         for (int o = 32; o > 0; o >>= 1) {
-            mn[d] = min(mn[d], (uint32_t)__shfl_xor(mn[d], o, 64));
-            mx[d] = max(mx[d], (uint32_t)__shfl_xor(mx[d], o, 64));
+            const uint32_t v = (uint32_t)__shfl_xor(m[d], o, 64);
+            m[d] = d < 3 ? min(m[d], v) : max(m[d], v);
         }
     if ((threadIdx.x & 63u) == 0)
-        for (int d = 0; d < 3; d++) {
-            atomicMin(ext + d, mn[d]);
-            atomicMax(ext + 3 + d, mx[d]);
-        }
+        for (int d = 0; d < 6; d++) red[threadIdx.x >> 6][d] = m[d];
+    __syncthreads();
+    if (threadIdx.x < 6) {
+        const int d = threadIdx.x;
+        uint32_t v = red[0][d];
+        for (int w = 1; w < 4; w++) v = d < 3 ? min(v, red[w][d]) : max(v, red[w][d]);
+        if (d < 3) atomicMin(ext + d, v);
+        else atomicMax(ext + d, v);
+    }
 }
 
 // per-cell k extents: ext[6c + d] min key of component d, ext[6c + 3 + d] max key.
-// LDS: the block's extents of every cell (6 ncell keys, dynamic), merged into ext
-// with one atomic per touched cell and key.
+// LDS: the block's extents of every cell (6 ncell keys, dynamic), merged into ext with one
+// atomic per touched cell and key.  A thread takes four pixels in a row and adds the extents of
+// those in one cell together: the pixels of a wave lie in few cells, whose words its lanes share.
 __global__ void __launch_bounds__(256)
     cell_ext_lds_kernel(const float *__restrict__ kmap, uint32_t npix, CellGeom g, uint32_t *ext)
 {
@@ -314,13 +330,30 @@ __global__ void __launch_bounds__(256)
             sext[6 * c + 3 + d] = 0u;
         }
     __syncthreads();
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < npix; i += gridDim.x * blockDim.x) {
-        const float k[3] = {kmap[3 * (size_t)i], kmap[3 * (size_t)i + 1], kmap[3 * (size_t)i + 2]};
-        const int c = cell_of(g, k[g.au], k[g.av]);
-        for (int d = 0; d < 3; d++) {
-            atomicMin(sext + 6 * c + d, fkey(k[d]));
-            atomicMax(sext + 6 * c + 3 + d, fkey(k[d]));
+    const uint64_t step = 4ull * gridDim.x * blockDim.x;
+    for (uint64_t i0 = 4ull * (blockIdx.x * blockDim.x + threadIdx.x); i0 < npix; i0 += step) {
+        int cell = -1;
+        uint32_t m[6];
+        auto put = [&]() {
+            if (cell < 0) return;
+            for (int d = 0; d < 3; d++) {
+                atomicMin(sext + 6 * cell + d, m[d]);
+                atomicMax(sext + 6 * cell + 3 + d, m[3 + d]);
+            }
+        };
+        for (uint64_t i = i0; i < min(i0 + 4, (uint64_t)npix); i++) {
+            const float k[3] = {kmap[3 * i], kmap[3 * i + 1], kmap[3 * i + 2]};
+            const int c = cell_of(g, k[g.au], k[g.av]);
+            const bool same = c == cell;
+            if (!same) put();
+            for (int d = 0; d < 3; d++) {
+                const uint32_t key = fkey(k[d]);
+                m[d] = same ? min(m[d], key) : key;
+                m[3 + d] = same ? max(m[3 + d], key) : key;
+            }
+            cell = c;
         }
+        put();
     }
     __syncthreads();
     for (int c = threadIdx.x; c < ncell; c += blockDim.x)
@@ -1571,13 +1604,6 @@ __global__ void __launch_bounds__(kBlock, LINEAR ? 4 : 8)
     // signed voxel scale and byte stride of the first two axes: q times the first is not negative
     const float voxa = T.sa < 0 ? -vox : vox, voxb = T.sb < 0 ? -vox : vox;
     const int sta = T.sa < 0 ? -8 : 8, stb = T.sb < 0 ? -bx8 : bx8;
-    // v_cvt_rpi_i32_f32: floor(x + 1/2) without an intermediate rounding (checked over all floats in
-    // [0, 2^22)), which is round_away of an x >= 0 in one instruction
-    auto round_up = [](float x) {
-        int r;
-        asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(x));
-        return r;
-    };
     // fast: the pair's voxels lie in the box and its value below 2^32; a pair that fails the cut
     // adds 0 (nearest) or is skipped (linear).  kSigned: q keeps its sign along the first two axes;
     // kThin: the box is one voxel deep along the third, whose voxel is then the same for all pairs.
@@ -1998,22 +2024,34 @@ void build_tiles(iac_pair_plan &pl, bool ordered)
     pl.tiles_fit = !pl.tiles.empty() && boxed >= pl.tiles.size() - pl.tiles.size() / 32;
 }
 
-// Extents of the k-map (one host round trip).
-int kmap_extents(iac_ctx *ctx, hipStream_t st, const float *d_kmap, uint32_t npix, uint32_t *d_ext, float kmin[3],
-                 float ext3[3])
+// Page-locked read-back area of a plan: the k-map's extents, the cells', 8 bytes, then more.
+struct PlanRead {
+    uint32_t *kext, *cells;
+    uint64_t *more;
+};
+int plan_read(iac_ctx *ctx, size_t more_bytes, PlanRead *out)
 {
-    hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, d_ext, 0xffffffffu, (size_t)3);
-    hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, d_ext + 3, 0u, (size_t)3);
-    const unsigned eb = std::max(1u, std::min<unsigned>(64, (npix + 255) / 256));
-    // few blocks: the six extent words take one atomic per wave, all on the same addresses
+    void *p = nullptr;
+    IAC_TRY(pinned(ctx, 0, (8 + 6 * (size_t)kMaxCells) * sizeof(uint32_t) + more_bytes, &p));
+    out->kext = static_cast<uint32_t *>(p);
+    out->cells = out->kext + 8;
+    out->more = reinterpret_cast<uint64_t *>(out->cells + 6 * (size_t)kMaxCells);
+    return IAC_OK;
+}
+
+// Extents of the k-map (one host round trip).
+int kmap_extents(hipStream_t st, const float *d_kmap, uint32_t npix, uint32_t *d_ext, const PlanRead &read,
+                 float kmin[3], float ext3[3])
+{
+    hipLaunchKernelGGL(init_cell_ext_kernel, dim3(1), dim3(64), 0, st, d_ext, 1);
+    const unsigned eb = std::max(1u, std::min<unsigned>(64, (npix + 1023) / 1024));
     hipLaunchKernelGGL(kext_kernel, dim3(eb), dim3(256), 0, st, d_kmap, npix, d_ext);
     IAC_HIP(hipGetLastError());
-    uint32_t hext[6];
-    IAC_HIP(hipMemcpyAsync(hext, d_ext, sizeof(hext), hipMemcpyDeviceToHost, st));
+    IAC_HIP(hipMemcpyAsync(read.kext, d_ext, 6 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
     IAC_HIP(hipStreamSynchronize(st));
     for (int d = 0; d < 3; d++) {
-        kmin[d] = unkey(hext[d]);
-        ext3[d] = unkey(hext[3 + d]) - kmin[d];
+        kmin[d] = unkey(read.kext[d]);
+        ext3[d] = unkey(read.kext[3 + d]) - kmin[d];
     }
     return IAC_OK;
 }
@@ -2043,31 +2081,31 @@ CellGeom cell_grid(const float kmin[3], const float ext3[3], float vox, int cell
     return g;
 }
 
-// Enqueues the per-cell extents of the k-map and their copy to cext (read it after a sync).
+// Enqueues the per-cell extents of the k-map and their copy to read.cells (valid after a sync).
 int cell_extents(hipStream_t st, const float *d_kmap, uint32_t npix, const CellGeom &g, uint32_t *d_cell_ext,
-                 std::vector<uint32_t> &cext)
+                 const PlanRead &read)
 {
     const int nc = g.ncu * g.ncv;
     hipLaunchKernelGGL(init_cell_ext_kernel, dim3((nc + 255) / 256), dim3(256), 0, st, d_cell_ext, nc);
     const size_t lds = 6 * sizeof(uint32_t) * (size_t)nc;
     if (lds <= 48 * 1024) {
-        const unsigned lb = std::max(1u, std::min<unsigned>(512, (npix + 4095) / 4096));
+        const unsigned lb = std::max(1u, std::min<unsigned>(512, (npix + 1023) / 1024));
         hipLaunchKernelGGL(cell_ext_lds_kernel, dim3(lb), dim3(256), lds, st, d_kmap, npix, g, d_cell_ext);
     } else {
         const unsigned eb = std::max(1u, std::min<unsigned>(1024, (npix + 255) / 256));
         hipLaunchKernelGGL(cell_ext_kernel, dim3(eb), dim3(256), 0, st, d_kmap, npix, g, d_cell_ext);
     }
     IAC_HIP(hipGetLastError());
-    cext.resize(6 * (size_t)nc);
-    IAC_HIP(hipMemcpyAsync(cext.data(), d_cell_ext, cext.size() * 4, hipMemcpyDeviceToHost, st));
+    IAC_HIP(hipMemcpyAsync(read.cells, d_cell_ext, lds, hipMemcpyDeviceToHost, st));
     return IAC_OK;
 }
 
 // The plan of a grid and its cell extents, from the context's cache or made.
 int plan_of(iac_ctx *ctx, const PairRun &R, int cell_vox, int box_cap, int region, const CellGeom &g,
-            std::vector<uint32_t> &cext, iac_pair_plan **out)
+            const uint32_t *cells, iac_pair_plan **out)
 {
     const PairSpec &S = R.spec;
+    std::vector<uint32_t> cext(cells, cells + 6 * (size_t)g.ncu * g.ncv);
     iac_pair_plan *pl = find_plan(ctx, R.d_kmap, R.npix, cell_vox, box_cap, region, S);
     if (pl && (std::memcmp(&pl->g, &g, sizeof(g)) != 0 || pl->cell_ext != cext)) pl = nullptr;
     if (!pl) {
@@ -2117,20 +2155,27 @@ int plan_of(iac_ctx *ctx, const PairRun &R, int cell_vox, int box_cap, int regio
 }
 
 // Cell grid of the k-map (two host round trips for the extents) and the task
-// table, from the context's cache when the geometry matches.
+// table, from the context's cache when the geometry matches.  h_off: also the frames' offsets,
+// read back with them (valid until the context's next call).
 int get_plan(iac_ctx *ctx, hipStream_t st, const PairRun &R, int cell_vox, int box_cap, int region,
-             iac_pair_plan **out)
+             iac_pair_plan **out, const uint64_t **h_off = nullptr)
 {
     void *ext = nullptr;
     IAC_TRY(scratch(ctx, 3, (6 + 6 * (size_t)kMaxCells) * sizeof(uint32_t), &ext));
     uint32_t *d_ext = static_cast<uint32_t *>(ext);
+    const size_t off_bytes = h_off ? ((size_t)R.nframes + 1) * sizeof(uint64_t) : 0;
+    PlanRead read;
+    IAC_TRY(plan_read(ctx, off_bytes, &read));
     float kmin[3], ext3[3];
-    IAC_TRY(kmap_extents(ctx, st, R.d_kmap, R.npix, d_ext, kmin, ext3));
+    IAC_TRY(kmap_extents(st, R.d_kmap, R.npix, d_ext, read, kmin, ext3));
     const CellGeom g = cell_grid(kmin, ext3, R.spec.P.vox, cell_vox);
-    std::vector<uint32_t> cext;
-    IAC_TRY(cell_extents(st, R.d_kmap, R.npix, g, d_ext + 6, cext));
+    IAC_TRY(cell_extents(st, R.d_kmap, R.npix, g, d_ext + 6, read));
+    if (h_off) {
+        IAC_HIP(hipMemcpyAsync(read.more, R.d_frame_off, off_bytes, hipMemcpyDeviceToHost, st));
+        *h_off = read.more;
+    }
     IAC_HIP(hipStreamSynchronize(st));
-    return plan_of(ctx, R, cell_vox, box_cap, region, g, cext, out);
+    return plan_of(ctx, R, cell_vox, box_cap, region, g, read.cells, out);
 }
 
 // Frame chunks inside each group, balanced by pair work: a chunk closes once its
@@ -2364,17 +2409,35 @@ void free_pair_plans(iac_ctx *ctx)
     ctx->pair_plans.clear();
 }
 
+namespace {
+// The group offsets and the chunk table to the device, through page-locked staging: the host does
+// not wait for the copies.
+int upload_tables(iac_ctx *ctx, hipStream_t st, const PairRun &R, const std::vector<Chunk> &chunks, uint32_t *d_goff,
+                  Chunk *d_chunks)
+{
+    const size_t bg = (R.ngroups + 1) * sizeof(uint32_t), bc = chunks.size() * sizeof(Chunk);
+    void *p = nullptr;
+    IAC_TRY(pinned(ctx, 1, bg + bc, &p));
+    std::memcpy(p, R.h_group_off, bg);
+    IAC_HIP(hipMemcpyAsync(d_goff, p, bg, hipMemcpyHostToDevice, st));
+    if (bc) {
+        char *c = static_cast<char *>(p) + bg;
+        std::memcpy(c, chunks.data(), bc);
+        IAC_HIP(hipMemcpyAsync(d_chunks, c, bc, hipMemcpyHostToDevice, st));
+    }
+    return upload_done(ctx);
+}
+}  // namespace
+
 int pairs_run(iac_ctx *ctx, const PairRun &R)
 {
     hipStream_t st = ctx->stream;
     if (R.n_total >= (1ull << 32)) return fail(IAC_ERR_LIMIT, "pair engine: at most 2^32 - 1 records per call");
     iac_pair_plan *pl = nullptr;
-    IAC_TRY(get_plan(ctx, st, R, cell_vox_of(ctx, R), box_cap_of(ctx, R), region_of(ctx, R), &pl));
-    std::vector<uint64_t> off(R.nframes + 1);
-    IAC_HIP(hipMemcpyAsync(off.data(), R.d_frame_off, off.size() * 8, hipMemcpyDeviceToHost, st));
-    IAC_HIP(hipStreamSynchronize(st));
-    const std::vector<Chunk> chunks = make_chunks(off.data(), R.nframes, R.h_group_off, R.ngroups, fchunk_of(ctx), R.h_rots);
-    IAC_TRY(check_chunks(off.data(), chunks));
+    const uint64_t *off = nullptr;
+    IAC_TRY(get_plan(ctx, st, R, cell_vox_of(ctx, R), box_cap_of(ctx, R), region_of(ctx, R), &pl, &off));
+    const std::vector<Chunk> chunks = make_chunks(off, R.nframes, R.h_group_off, R.ngroups, fchunk_of(ctx), R.h_rots);
+    IAC_TRY(check_chunks(off, chunks));
     const int nc = pl->g.ncu * pl->g.ncv;
     const Sizes z = sizes_of(R, nc, chunks.size());
     // scratch: sorted records + cell offsets (slot 1), H + group offsets + self + chunks (slot 2)
@@ -2395,10 +2458,7 @@ int pairs_run(iac_ctx *ctx, const PairRun &R)
     b.ntasks = (uint32_t)pl->tasks.size();
     b.g = pl->g;
     b.box_cap = pl->box_cap;
-    IAC_HIP(hipMemcpyAsync(b.d_goff, R.h_group_off, (R.ngroups + 1) * sizeof(uint32_t), hipMemcpyHostToDevice, st));
-    if (!chunks.empty())
-        IAC_HIP(hipMemcpyAsync(b.d_chunks, chunks.data(), chunks.size() * sizeof(Chunk), hipMemcpyHostToDevice, st));
-    IAC_HIP(hipStreamSynchronize(st));  // the host arrays above are released on return
+    IAC_TRY(upload_tables(ctx, st, R, chunks, b.d_goff, b.d_chunks));
     return enqueue(ctx, st, R, b, true);
 }
 
@@ -2436,7 +2496,9 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
     IAC_TRY(scratch(ctx, 3, (6 + 6 * (size_t)kMaxCells) * sizeof(uint32_t), &ext));
     uint32_t *d_ext = static_cast<uint32_t *>(ext);
     float kmin[3], ext3[3];
-    IAC_TRY(kmap_extents(ctx, st, R.d_kmap, R.npix, d_ext, kmin, ext3));
+    PlanRead read;
+    IAC_TRY(plan_read(ctx, sizeof(uint64_t), &read));
+    IAC_TRY(kmap_extents(st, R.d_kmap, R.npix, d_ext, read, kmin, ext3));
     const int box_cap = ordered ? kBoxMax : kBoxSmall;
     const size_t nvox = (size_t)S.P.sab * S.P.sab * S.P.sc;
     const uint32_t ns = std::min<uint32_t>(256, (R.npix + kBlock - 1) / kBlock);  // sort blocks per frame
@@ -2478,10 +2540,8 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
         auto *d_kept = d_self + R.ngroups;
         auto *d_plain = reinterpret_cast<uint32_t *>(d_kept + 1);
         auto *d_chunks = reinterpret_cast<Chunk *>(p2 + bh + bg + bs);
-        IAC_HIP(hipMemcpyAsync(d_goff, R.h_group_off, (R.ngroups + 1) * sizeof(uint32_t), hipMemcpyHostToDevice, st));
-        IAC_HIP(hipMemcpyAsync(d_chunks, chunks.data(), chunks.size() * sizeof(Chunk), hipMemcpyHostToDevice, st));
-        std::vector<uint32_t> cext;
-        IAC_TRY(cell_extents(st, R.d_kmap, R.npix, g, d_ext + 6, cext));
+        IAC_TRY(upload_tables(ctx, st, R, chunks, d_goff, d_chunks));
+        IAC_TRY(cell_extents(st, R.d_kmap, R.npix, g, d_ext + 6, read));
         auto blocks = [](size_t n) { return (unsigned)std::max<size_t>(1, std::min<size_t>(4096, (n + 255) / 256)); };
         const size_t ncs = R.nframes * (nkey + 1);
         hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks(ncs)), dim3(256), 0, st, cs, 0u, ncs);
@@ -2497,12 +2557,12 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
         if (!ordered)
             hipLaunchKernelGGL(fill_u64_kernel, dim3(blocks(nvox * R.ngroups)), dim3(256), 0, st, H, nvox * R.ngroups);
         IAC_HIP(hipGetLastError());
-        unsigned long long kept = 0;
-        IAC_HIP(hipMemcpyAsync(&kept, d_kept, sizeof(kept), hipMemcpyDeviceToHost, st));
-        IAC_HIP(hipStreamSynchronize(st));  // also releases the host arrays copied above
+        IAC_HIP(hipMemcpyAsync(read.more, d_kept, sizeof(uint64_t), hipMemcpyDeviceToHost, st));
+        IAC_HIP(hipStreamSynchronize(st));
+        const uint64_t kept = read.more[0];
         if ((double)kept < kTileRecords * (double)R.nframes * nc) return IAC_OK;  // sparse frames
         iac_pair_plan *pl = nullptr;
-        IAC_TRY(plan_of(ctx, R, side, box_cap, kRegionTiles, g, cext, &pl));
+        IAC_TRY(plan_of(ctx, R, side, box_cap, kRegionTiles, g, read.cells, &pl));
         if (!pl->tiles_fit) continue;
         const bool by_parts = !ordered && (double)kept >= kPartRecords * (double)R.nframes * (double)nkey;
         auto *target = ordered ? reinterpret_cast<unsigned long long *>(R.d_mesh) : H;

@@ -178,10 +178,11 @@ int iac_sparse_hit_list(iac_ctx *ctx, const float *d_kmap, uint32_t npix, const 
                        reinterpret_cast<float4 *>(d_rec4));
     IAC_HIP(hipGetLastError());
     IAC_TRY(iac::timer_end(ctx));
-    uint64_t n = 0;
-    IAC_HIP(hipMemcpyAsync(&n, d_frame_off + nframes, sizeof(n), hipMemcpyDeviceToHost, ctx->stream));
+    void *n = nullptr;
+    IAC_TRY(iac::pinned(ctx, 0, sizeof(uint64_t), &n));
+    IAC_HIP(hipMemcpyAsync(n, d_frame_off + nframes, sizeof(uint64_t), hipMemcpyDeviceToHost, ctx->stream));
     IAC_HIP(hipStreamSynchronize(ctx->stream));
-    *n_total = n;
+    *n_total = *static_cast<const uint64_t *>(n);
     return IAC_OK;
 }
 
