@@ -558,9 +558,9 @@ struct TunePoint {
 // Candidates around the measured defaults: nearest-neighbour binning (one LDS add per pair,
 // symmetric: unordered pairs and a mirror pass) and linear binning (eight corner adds per
 // ordered pair, 4096-voxel boxes); walks 1 = lanes on consecutive pairs, 2 = a pair range
-// per thread.
+// per thread; all 0 = the defaults, which take strips where they suit the run.
 const TunePoint kTuneNearest[] = {{1, 6, 1920, 32}, {1, 5, 1920, 32}, {1, 4, 1920, 32}, {1, 6, 1920, 64},
-                                  {1, 8, 4096, 32}, {1, 4, 1024, 32}, {2, 4, 1920, 32}};
+                                  {1, 8, 4096, 32}, {1, 4, 1024, 32}, {2, 4, 1920, 32}, {0, 0, 0, 0}};
 const TunePoint kTuneLinear[] = {{1, 5, 4096, 32}, {1, 4, 4096, 32}, {1, 6, 4096, 32},
                                  {1, 4, 1920, 32}, {2, 4, 4096, 32}, {1, 5, 4096, 64}};
 

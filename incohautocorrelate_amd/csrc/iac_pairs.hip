@@ -31,6 +31,7 @@
 // on the point reflection of (a,b) with the same value, so step 4 restores
 // the ordered-pair mesh exactly.  Linear modes are not odd and run ordered.
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -388,8 +389,9 @@ __global__ void __launch_bounds__(kBlock)
                      float4 *__restrict__ srec, uint32_t *__restrict__ cs, PairSpec S,
                      const uint32_t *__restrict__ group_off, uint32_t ngroups,
                      unsigned long long *__restrict__ self, uint32_t *__restrict__ wflag,
-                     uint32_t *__restrict__ cmax)
+                     uint32_t *__restrict__ cmax, const uint32_t *__restrict__ strips)
 {
+    if (strips && strips[0]) return;  // the strips take the run
     __shared__ uint32_t cnt[kMaxCells];
     __shared__ uint32_t part[kBlock];
     __shared__ unsigned long long sred[kBlock / 64];
@@ -467,8 +469,11 @@ __global__ void __launch_bounds__(kBlock)
 // mesh[g][v] += H[g][v] + H[g][last - v]; the centre also receives self[g].
 __global__ void symmetrize_kernel(const unsigned long long *__restrict__ H, unsigned long long *__restrict__ mesh,
                                   size_t nvox, uint32_t ngroups, size_t centre,
-                                  const unsigned long long *__restrict__ self)
+                                  const unsigned long long *__restrict__ self,
+                                  const unsigned long long *__restrict__ strip_self,
+                                  const uint32_t *__restrict__ strips)
 {
+    if (strips && strips[0]) self = strip_self;
     const size_t last = nvox - 1, total = nvox * ngroups;
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
         const size_t gi = i / nvox, v = i - gi * nvox;
@@ -880,8 +885,10 @@ __global__ void __launch_bounds__(kBlock, (Occupancy<FAST, BOX>::blocks))
                  const Task *__restrict__ tasks, uint32_t ntasks, CellGeom g, PairSpec S,
                  unsigned long long *__restrict__ target, size_t nvox,
                  unsigned long long *__restrict__ dropped, const uint32_t *__restrict__ wflag,
-                 const float *__restrict__ rots, const uint32_t *__restrict__ cmax)
+                 const float *__restrict__ rots, const uint32_t *__restrict__ cmax,
+                 const uint32_t *__restrict__ strips)
 {
+    if (strips && strips[0]) return;  // the strips took the run
     constexpr int kGroup = BoxCfg<BOX>::group;
     constexpr int kItemsPerThread = BoxCfg<BOX>::ipt;
     __shared__ unsigned long long box[BOX];
@@ -1304,6 +1311,8 @@ struct TileBatch {
 
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef const __attribute__((address_space(4))) f4v *scalar_rec_t;
+typedef const __attribute__((address_space(4))) uint32_t *scalar_u32_t;
+typedef const __attribute__((address_space(4))) uint64_t *scalar_u64_t;
 
 // The sort key of a k: its region, then its voxel-sized part of the region (side x side parts,
 // so records of one region that lie far apart in its order lie on different voxels).
@@ -1727,6 +1736,309 @@ __global__ void __launch_bounds__(kBlock, LINEAR ? 4 : 8)
     }
 }
 
+// ---- AC_uw strips ---------------------------------------------------------------------
+//
+// The walk above finds a pair's records through per-cell items of about 20 pairs, which costs twice
+// what binning the pair does (58 VALU instructions and 7 LDS accesses per 64 pairs).  Where a box of
+// 32-bit words can hold it, a task is instead a distance between strips of the detector (a few
+// voxels tall, all of it wide): the records of strip j and those of the strips j + dv ..
+// j + dv + nv - 1 pair completely, so a wave takes one side's records as lanes and the other's
+// one by one from the scalar unit, with no index work: 22 VALU instructions and one LDS add per
+// 64 pairs.  The box counts w_a w_b; the flush multiplies by the fixed point's 1000.
+// 32 bits are exact: weights are integers in [1, 129] (else the walk runs), a frame adds at most
+// w_max^2 n m to a voxel (n records, m in its fullest strip), and a block flushes before
+// the frames it has added could pass 2^32.
+// 3,000 frames of 2,090 photons on a 1024^2 detector into 257^3: 9.0 ms by the walk, 6.5 by strips
+// (1.0e12 pairs/s); 800 frames with a rotation each 10.1 and 4.9 (a task of several distances
+// flushes each voxel of its mesh 1.2 times, the walk's small boxes 2 to 3 times).  Bound: VALU issue
+// at three quarters, a fifth of the lanes empty; with rotations the scattered atomics of the flush.
+// Lanes without a record are off rather than adding 0: their zeros would meet in one address, 13
+// clocks of LDS per 64 pairs instead of 6 (7.4 ms).
+
+constexpr int kMaxStrips = 512;
+
+// One block per frame, as cell_sort_kernel: records by strip, strip starts, self values; bound[f] =
+// the most a voxel can receive from the frame.  A record's w holds its integer weight and, above 8
+// bits, its reach: no record of a strip fewer than reach strips away, wherever in it, is beyond the
+// cut.  A strip's records are in order of falling reach (eight classes), so that
+// most batches of b need no cut.  `usable` starts at 1 and is cleared by a weight that is no
+// integer in [1, 129] or a frame whose bound passes 2^32.
+struct StripGeom {
+    CellGeom g;
+    float ulo, uhi, zext;  // extents of the k-map along the strips and the beam
+};
+constexpr int kReachClasses = 8;
+__device__ inline uint32_t strip_reach(const StripGeom &G, float cut_sq, float u)
+{
+    const float du = fmaxf(u - G.ulo, G.uhi - u);
+    const float left = cut_sq * (1.0f - 1e-5f) - (du * du + G.zext * G.zext) * (1.0f + 1e-5f);
+    return left > 0.0f ? (uint32_t)min((float)(2 * kMaxStrips), sqrtf(left) * G.g.inv_wv * (1.0f - 1e-5f)) : 0u;
+}
+__global__ void __launch_bounds__(kBlock)
+    strip_sort_kernel(const float4 *__restrict__ rec, const uint64_t *__restrict__ off, StripGeom G,
+                      float4 *__restrict__ srec, uint32_t *__restrict__ cs, PairSpec S,
+                      const uint32_t *__restrict__ group_off, uint32_t ngroups,
+                      unsigned long long *__restrict__ self, uint32_t *__restrict__ usable,
+                      uint32_t *__restrict__ bound)
+{
+    __shared__ uint32_t cnt[kMaxStrips * kReachClasses];
+    __shared__ unsigned long long sred[kBlock / 64];
+    __shared__ uint32_t wred[kBlock / 64], nred[kBlock / 64], sums[kBlock / 64];
+    const CellGeom &g = G.g;
+    const uint32_t f = blockIdx.x, lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
+    const int ncell = g.ncv, nbin = ncell * kReachClasses;
+    const uint64_t base = off[f];
+    const uint32_t n = (uint32_t)(off[f + 1] - base);
+    auto place = [&](const float4 &r, uint32_t reach) {
+        const int cls = max(0, kReachClasses - 1 - (int)(reach * kReachClasses / (uint32_t)ncell));
+        return cell_of(g, 0.0f, comp(r, g.av)) * kReachClasses + cls;
+    };
+    for (int c = threadIdx.x; c < kMaxStrips * kReachClasses; c += kBlock) cnt[c] = 0;
+    __syncthreads();
+    unsigned long long sv = 0;
+    uint32_t wmax = 0;
+    bool ok = true;
+    for (uint32_t i = threadIdx.x; i < n; i += kBlock) {
+        const float4 r = rec[base + i];
+        if (r.w == 0.0f) continue;
+        atomicAdd(&cnt[place(r, strip_reach(G, S.P.cut_sq, comp(r, g.au)))], 1u);
+        sv += self_value<kKindAc3d>(S, r.w);
+        const bool small = r.w >= 1.0f && r.w <= 129.0f && r.w == truncf(r.w);
+        ok = ok && small;
+        if (small) wmax = max(wmax, (uint32_t)r.w);
+    }
+    if (!ok) usable[0] = 0u;
+    __syncthreads();
+    // starts: consecutive bins per thread, whole strips each
+    const int per = (nbin / kReachClasses + kBlock - 1) / kBlock;  // strips
+    uint32_t tot = 0, most = 0;
+    for (int k = 0; k < per; k++) {
+        const int c = ((int)threadIdx.x * per + k) * kReachClasses;
+        uint32_t strip = 0;
+        if (c < nbin)
+            for (int e = 0; e < kReachClasses; e++) strip += cnt[c + e];
+        tot += strip;
+        most = max(most, strip);
+    }
+    uint32_t x = tot;
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t y = __shfl_up(x, o, 64);
+        if (lane >= (uint32_t)o) x += y;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        sv += __shfl_down(sv, o, 64);
+        wmax = max(wmax, (uint32_t)__shfl_down(wmax, o, 64));
+        most = max(most, (uint32_t)__shfl_down(most, o, 64));
+    }
+    if (lane == 63) sums[wave] = x;
+    if (lane == 0) {
+        sred[wave] = sv;
+        wred[wave] = wmax;
+        nred[wave] = most;
+    }
+    __syncthreads();
+    uint32_t run = x - tot, all = 0;
+    for (uint32_t w = 0; w < kBlock / 64; w++) {
+        if (w < wave) run += sums[w];
+        all += sums[w];
+    }
+    uint32_t *csf = cs + (size_t)f * (ncell + 1);
+    for (int k = 0; k < per; k++) {
+        const int c = ((int)threadIdx.x * per + k) * kReachClasses;
+        if (c >= nbin) break;
+        csf[c / kReachClasses] = run;
+        for (int e = 0; e < kReachClasses; e++) {
+            const uint32_t v = cnt[c + e];
+            cnt[c + e] = run;
+            run += v;
+        }
+    }
+    if (threadIdx.x == 0) {
+        csf[ncell] = all;
+        uint32_t w = 0;
+        most = 0;
+        sv = 0;
+        for (uint32_t k = 0; k < kBlock / 64; k++) {
+            w = max(w, wred[k]);
+            most = max(most, nred[k]);
+            sv += sred[k];
+        }
+        const uint64_t b = (uint64_t)w * w * n * most;
+        if (b >> 32) usable[0] = 0u;
+        bound[f] = (uint32_t)b;
+        if (sv) {
+            uint32_t lo = 0, hi = ngroups;  // group of f: largest gi with group_off[gi] <= f
+            while (hi - lo > 1) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (group_off[mid] <= f) lo = mid; else hi = mid;
+            }
+            atomicAdd(self + lo, sv);
+        }
+    }
+    __syncthreads();
+    for (uint32_t i = threadIdx.x; i < n; i += kBlock) {
+        float4 r = rec[base + i];
+        if (r.w == 0.0f) continue;
+        const uint32_t reach = strip_reach(G, S.P.cut_sq, comp(r, g.au));
+        const uint32_t pos = atomicAdd(&cnt[place(r, reach)], 1u);
+        r.w = __uint_as_float(((uint32_t)r.w & 255u) | reach << 8);
+        srec[base + pos] = r;
+    }
+}
+
+constexpr int kStripBatch = 4;  // scalar records per load batch
+
+__device__ inline int mad24(int a, int b, int c)
+{
+    int r;
+    asm("v_mad_i32_i24 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));  // else two multiplies and an add3
+    return r;
+}
+
+__device__ inline uint32_t uniform(uint32_t x) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)x); }
+
+// Grid: ntasks per chunk of frames.  AV: the k component across the strips (0 or 1); the beam is
+// the third.  A task pairs b in strip j with a in the strips j + dv .. j + dv + nv - 1.
+template <int AV, int BLOCK>
+__global__ void __launch_bounds__(BLOCK)
+    strip_kernel(const float4 *__restrict__ srec, const uint64_t *__restrict__ off, const uint32_t *__restrict__ cs,
+                 const Chunk *__restrict__ chunks, const Task *__restrict__ tasks, uint32_t ntasks, int ncell,
+                 PairSpec S, unsigned long long *__restrict__ target, size_t nvox,
+                 unsigned long long *__restrict__ dropped, const uint32_t *__restrict__ usable,
+                 const uint32_t *__restrict__ bound, const float *__restrict__ rots)
+{
+    extern __shared__ uint32_t sbox[];
+    if (!usable[0]) return;
+    const Task T = tasks[blockIdx.x % ntasks];
+    const Chunk CH = chunks[blockIdx.x / ntasks];
+    const uint32_t lane = threadIdx.x & 63u, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    constexpr uint32_t kWaves = BLOCK / 64;
+    const int vbox = T.bx * T.by * T.bz;
+    for (int v = threadIdx.x; v < vbox; v += BLOCK) sbox[v] = 0u;
+    const int bx4 = 4 * T.bx, bxby4 = 4 * T.bx * T.by;
+    const int c4 = 4 * (S.P.c0 - T.bx0) + bx4 * (S.P.c1 - T.by0) + bxby4 * (S.P.c2 - T.bz0);
+    char *const boxb = reinterpret_cast<char *>(sbox);
+    const float cut_sq = S.P.cut_sq;
+    unsigned long long *const out = target + (size_t)CH.group * nvox;
+    const float *crot = rots ? rots + 9 * (size_t)CH.f0 : nullptr;
+
+    auto flush = [&]() {
+        float rr[9];
+        int ax = 0;  // the box axis consecutive lanes walk (as the walk's flush)
+        if (crot) {
+            for (int i = 0; i < 9; i++) rr[i] = crot[i];
+            const float a0 = fabsf(rr[0]), a1 = fabsf(rr[1]), a2 = fabsf(rr[2]);
+            ax = a1 > a0 ? (a2 > a1 ? 2 : 1) : (a2 > a0 ? 2 : 0);
+        }
+        const int e0 = ax == 0 ? T.bx : (ax == 1 ? T.by : T.bz), e1 = ax == 0 ? T.by : T.bx;
+        for (int v = threadIdx.x; v < vbox; v += BLOCK) {
+            const int i0 = v % e0, rest = v / e0, i1 = rest % e1, i2 = rest / e1;
+            const int lx = ax == 0 ? i0 : i1, ly = ax == 1 ? i0 : (ax == 0 ? i1 : i2), lz = ax == 2 ? i0 : i2;
+            const uint32_t x = sbox[lx + T.bx * (ly + T.by * lz)];
+            if (!x) continue;
+            int fs = T.bx0 + lx, ms = T.by0 + ly, ss = T.bz0 + lz;
+            if (crot) {
+                rotate_voxel(rr, S.P.c0, S.P.c1, S.P.c2, fs, ms, ss);
+                if ((unsigned)fs >= (unsigned)S.P.sab || (unsigned)ms >= (unsigned)S.P.sab ||
+                    (unsigned)ss >= (unsigned)S.P.sc) {
+                    atomicAdd(dropped, 1ull);  // excluded by the caller's bound check
+                    continue;
+                }
+            }
+            atomicAdd(out + (size_t)fs + (size_t)ms * S.P.sab + (size_t)ss * S.P.sab * S.P.sab, 1000ull * x);
+        }
+    };
+
+    // lane record l with scalar record s; vox carries the sign that makes it b from a
+    auto pair = [&](const float4 &l, uint32_t lw, const f4v &s, float vox, auto within_c, auto cut_c, bool on) {
+        constexpr bool kWithin = decltype(within_c)::value;  // q across the strips has both signs
+        const float dx = l.x - s.x, dy = l.y - s.y, dz = l.z - s.z;
+        if (decltype(cut_c)::value) on = ((dx * dx + dy * dy) + dz * dz < cut_sq) && on;
+        const float x = dx * vox, y = dy * vox, z = dz * vox;
+        // a - b across strips dv > 0 apart is not negative
+        const int nx = !kWithin && AV == 0 ? round_up(x) : round_away(x);
+        const int ny = !kWithin && AV == 1 ? round_up(y) : round_away(y);
+        const uint32_t v = __umul24(lw, __float_as_uint(s.w));
+        const int o = mad24(round_away(z), bxby4, mad24(ny, bx4, nx * 4 + c4));
+        atomicAdd(reinterpret_cast<uint32_t *>(boxb + o), on ? v : 0u);
+    };
+    // n lane records by m scalar ones; within: only pairs (l, s < l)
+    auto item = [&](const float4 *lr, uint32_t n, scalar_rec_t sr, uint32_t m, float vox, auto within_c) {
+        constexpr bool kWithin = decltype(within_c)::value;
+        for (uint32_t g0 = 0; g0 < n; g0 += 64) {
+            const uint32_t il = g0 + lane, me = kWithin ? min(m, g0 + 63) : m;
+            if (il >= n) continue;  // empty lanes off: their zeros would all go to one address
+            const float4 l = lr[il];
+            const uint32_t lw = __float_as_uint(l.w) & 255u;
+            // the next batch loads under the pairs of this one
+            f4v next[kStripBatch];
+#pragma unroll
+            for (int k = 0; k < kStripBatch; k++) next[k] = sr[min((uint32_t)k, m - 1)];
+            for (uint32_t j0 = 0; j0 < me; j0 += kStripBatch) {
+                f4v s[kStripBatch];
+                uint32_t least = ~0u;
+#pragma unroll
+                for (int k = 0; k < kStripBatch; k++) {
+                    s[k] = next[k];
+                    const uint32_t w = __float_as_uint(s[k].w);
+                    least = min(least, w);
+                    s[k].w = __uint_as_float(j0 + k < m ? w & 255u : 0u);
+                }
+#pragma unroll
+                for (int k = 0; k < kStripBatch; k++) next[k] = sr[min(j0 + kStripBatch + k, m - 1)];
+                if ((least >> 8) >= (uint32_t)(T.dv + T.nv)) {  // no pair of these strips beyond the cut
+#pragma unroll
+                    for (int k = 0; k < kStripBatch; k++)
+                        pair(l, lw, s[k], vox, within_c, std::false_type{}, !kWithin || j0 + k < il);
+                } else {
+#pragma unroll
+                    for (int k = 0; k < kStripBatch; k++)
+                        pair(l, lw, s[k], vox, within_c, std::true_type{}, !kWithin || j0 + k < il);
+                }
+            }
+        }
+    };
+
+    for (uint32_t fa = CH.f0; fa < CH.f1;) {
+        // frames [fa, fb) cannot pass 2^32 in any voxel
+        uint64_t most = bound[fa];
+        uint32_t fb = fa + 1;
+        while (fb < CH.f1 && most + bound[fb] < (1ull << 32)) most += bound[fb++];
+        __syncthreads();  // the box is clear
+        // items (frame, strip j of b), the waves in turn
+        uint32_t f = uniform(fa);
+        int j = (int)wave;
+        for (;; j += (int)kWaves) {
+            while (f < fb && j >= ncell - T.dv) {
+                j -= ncell - T.dv;
+                f++;
+            }
+            if (f >= fb) break;
+            const scalar_u32_t csf = (scalar_u32_t)(uintptr_t)(cs + (size_t)f * (ncell + 1));
+            const int i = j + T.dv, ie = min(i + T.nv, ncell);
+            const uint32_t a0 = uniform(csf[i]), na = uniform(csf[ie]) - a0;
+            const uint32_t b0 = uniform(csf[j]), nb = uniform(csf[j + 1]) - b0;
+            if (na == 0 || nb == 0) continue;
+            const uint64_t base = ((scalar_u64_t)(uintptr_t)off)[f];
+            const float4 *fr = srec + (((uint64_t)uniform((uint32_t)(base >> 32)) << 32) | uniform((uint32_t)base));
+            if (T.dv == 0)  // strip j itself and its neighbours: every a behind b in the order
+                item(fr + a0, na, (scalar_rec_t)(uintptr_t)(fr + b0), nb, S.P.vox, std::true_type{});
+            else if (((nb + 63) / 64) * na < ((na + 63) / 64) * nb)
+                // the lanes take the side that leaves fewer of them empty
+                item(fr + b0, nb, (scalar_rec_t)(uintptr_t)(fr + a0), na, -S.P.vox, std::false_type{});
+            else
+                item(fr + a0, na, (scalar_rec_t)(uintptr_t)(fr + b0), nb, S.P.vox, std::false_type{});
+        }
+        __syncthreads();
+        flush();
+        fa = fb;
+        if (fa < CH.f1) {
+            __syncthreads();
+            for (int v = threadIdx.x; v < vbox; v += BLOCK) sbox[v] = 0u;
+        }
+    }
+}
+
 // ---- host planning ---------------------------------------------------------------
 
 // The specialised pair path: AC_uw, symmetric (nearest-neighbour) binning, identity
@@ -1955,7 +2267,10 @@ iac_pair_plan *find_plan(iac_ctx *ctx, const float *kmap, uint32_t npix, int cel
     return nullptr;
 }
 
-constexpr int kRegionTiles = -1;  // iac_pair_plan::region of a region-tile plan
+constexpr int kRegionTiles = -1;   // iac_pair_plan::region of a region-tile plan
+constexpr int kRegionStrips = -2;  // and less: of a strip plan, its distances per task with it
+constexpr size_t kStripBox2 = 79 * 1024;  // LDS bytes of a strip box: two blocks per CU
+constexpr size_t kStripBox1 = 158 * 1024; // one block per CU
 
 // Tasks of the region tiles: pairs of regions (ci <= cj, or all ordered pairs of linear runs) that
 // are not wholly beyond the cut, with the box of their voxels (linear: of their corners).
@@ -2024,18 +2339,48 @@ void build_tiles(iac_pair_plan &pl, bool ordered)
     pl.tiles_fit = !pl.tiles.empty() && boxed >= pl.tiles.size() - pl.tiles.size() / 32;
 }
 
+// One task per `per` strip distances, with the box of all of them.
+void merge_strips(iac_pair_plan &pl, int per)
+{
+    std::vector<Task> out;
+    for (const Task &t : pl.tasks) {  // in the order of dv
+        if (!out.empty() && out.back().dv / per == t.dv / per) {
+            Task &o = out.back();
+            const int x1 = std::max(o.bx0 + o.bx, t.bx0 + t.bx), y1 = std::max(o.by0 + o.by, t.by0 + t.by),
+                      z1 = std::max(o.bz0 + o.bz, t.bz0 + t.bz);
+            o.bx0 = std::min(o.bx0, t.bx0);
+            o.by0 = std::min(o.by0, t.by0);
+            o.bz0 = std::min(o.bz0, t.bz0);
+            o.bx = x1 - o.bx0;
+            o.by = y1 - o.by0;
+            o.bz = z1 - o.bz0;
+            o.inbox = o.inbox && t.inbox;
+            o.nv = t.dv - o.dv + 1;
+        } else {
+            out.push_back(t);
+            out.back().nv = 1;
+        }
+    }
+    for (Task &t : out) {
+        t.inbox = t.inbox && (long)t.bx * t.by * t.bz <= pl.box_cap;
+        pl.tile_box = std::max(pl.tile_box, (size_t)t.bx * t.by * t.bz * sizeof(uint32_t));
+    }
+    pl.tasks.swap(out);
+}
+
 // Page-locked read-back area of a plan: the k-map's extents, the cells', 8 bytes, then more.
 struct PlanRead {
-    uint32_t *kext, *cells;
+    uint32_t *kext, *cells, *strips;
     uint64_t *more;
 };
 int plan_read(iac_ctx *ctx, size_t more_bytes, PlanRead *out)
 {
     void *p = nullptr;
-    IAC_TRY(pinned(ctx, 0, (8 + 6 * (size_t)kMaxCells) * sizeof(uint32_t) + more_bytes, &p));
+    IAC_TRY(pinned(ctx, 0, (8 + 6 * (size_t)(kMaxCells + kMaxStrips)) * sizeof(uint32_t) + more_bytes, &p));
     out->kext = static_cast<uint32_t *>(p);
     out->cells = out->kext + 8;
-    out->more = reinterpret_cast<uint64_t *>(out->cells + 6 * (size_t)kMaxCells);
+    out->strips = out->cells + 6 * (size_t)kMaxCells;
+    out->more = reinterpret_cast<uint64_t *>(out->strips + 6 * (size_t)kMaxStrips);
     return IAC_OK;
 }
 
@@ -2081,9 +2426,71 @@ CellGeom cell_grid(const float kmin[3], const float ext3[3], float vox, int cell
     return g;
 }
 
-// Enqueues the per-cell extents of the k-map and their copy to read.cells (valid after a sync).
+// Frames per strip block: enough blocks to even out the last of them, few enough flushes (a 3,000
+// frame run: 7.0 ms with 3,072 blocks, 6.8 with 6,144, 7.4 with 12,288).
+constexpr double kStripBlocks = 6144;
+uint32_t strip_chunk(uint32_t nframes, size_t ntasks)
+{
+    return (uint32_t)std::max(1.0, std::min(64.0, (double)nframes * (double)ntasks / kStripBlocks));
+}
+
+// Strips of an AC_uw run: ncv of them (0: strips do not pay), a task per `per` distances.
+struct StripShape {
+    CellGeom g;
+    int per;
+};
+
+// Tall tasks waste little of their box (it spans per + 1 strips for per of lanes) and flush seldom;
+// records of the lanes' strips should fill 64 lanes, or 128, and those of b outweigh the cost of
+// starting an item.  The shape of least cost, in clocks of a CU per frame: 27 per 64 pairs (VALU
+// issue; 34 with one block per CU, whose flush nothing covers), 6 pairs' worth for an item's start,
+// 2.7 per voxel flushed to a rotated mesh (scattered atomics) or 1.5 to a plain one, shared
+// by a chunk's frames.  Measured: 34 picks seven-row boxes and 6.5 ms, 27 twelve-row ones and 6.8.
+StripShape strip_shape(const float kmin[3], const float ext3[3], const PairRun &R, double mean)
+{
+    StripShape best{};
+    CellGeom &g = best.g;
+    if (R.spec.kind != kKindAc3d || !fast_path(R.spec, R.ordered) || !(ext3[2] <= ext3[0] && ext3[2] <= ext3[1]))
+        return best;
+    g.av = ext3[1] >= ext3[0] ? 1 : 0;
+    g.au = 1 - g.av;
+    const double vox = R.spec.P.vox, wide = std::floor(2 * ext3[g.au] * vox + 2), deep = std::floor(2 * ext3[2] * vox + 2);
+    const double tall = ext3[g.av] * vox, per_vox = mean / std::max(1.0, tall);
+    // a second plan, sort and launch cost about 90 us, 0.3e-12 s per pair against the walk repay it
+    // (a rotated mesh's smaller flushes more)
+    const double pairs = 0.5 * mean * mean * R.nframes;
+    if (!(wide * deep * 4 * 3 <= kStripBox1) || !(pairs >= (R.h_rots ? 0x1p26 : 0x1p28))) return best;
+    double least = 1e300, h_best = 0;
+    for (int m = 1; m <= 8; m++)
+        for (double h = 1; h <= 64; h *= 1.0905) {  // eighths of an octave
+            const double rows = std::floor((m + 1) * h + 2), box = rows * wide * deep * 4, n = std::ceil(tall / h);
+            if (box > kStripBox1) break;
+            if (n > kMaxStrips || n < 2) continue;
+            const double L = m * h * per_vox, nb = h * per_vox;
+            double groups = 1;  // waves' loads of a Poisson number of lanes
+            for (int k = 1; k < 32; k++) groups += 0.5 * std::erfc((64.0 * k + 0.5 - L) / std::sqrt(2 * L));
+            const double items = n * (n + m) / (2.0 * m), tasks = std::ceil(n / m);
+            const double frames = R.h_rots ? 1 : strip_chunk(R.nframes, (size_t)tasks);
+            const double cost = items * groups * (nb + 7.5) * (box > kStripBox2 ? 34 : 27) + tasks * box / 4 * (R.h_rots ? 2.7 : 1.5) / frames;
+            if (cost < least) {
+                least = cost;
+                h_best = h;
+                best.per = m;
+                g.ncv = (int)n;
+            }
+        }
+    if (g.ncv == 0) return best;
+    g.u0 = 0.0f;
+    g.inv_wu = 0.0f;
+    g.ncu = 1;
+    g.v0 = kmin[g.av];
+    g.inv_wv = (float)(vox / h_best);
+    return best;
+}
+
+// Enqueues the per-cell extents of the k-map and their copy to h_cells (valid after a sync).
 int cell_extents(hipStream_t st, const float *d_kmap, uint32_t npix, const CellGeom &g, uint32_t *d_cell_ext,
-                 const PlanRead &read)
+                 uint32_t *h_cells)
 {
     const int nc = g.ncu * g.ncv;
     hipLaunchKernelGGL(init_cell_ext_kernel, dim3((nc + 255) / 256), dim3(256), 0, st, d_cell_ext, nc);
@@ -2096,7 +2503,7 @@ int cell_extents(hipStream_t st, const float *d_kmap, uint32_t npix, const CellG
         hipLaunchKernelGGL(cell_ext_kernel, dim3(eb), dim3(256), 0, st, d_kmap, npix, g, d_cell_ext);
     }
     IAC_HIP(hipGetLastError());
-    IAC_HIP(hipMemcpyAsync(read.cells, d_cell_ext, lds, hipMemcpyDeviceToHost, st));
+    IAC_HIP(hipMemcpyAsync(h_cells, d_cell_ext, lds, hipMemcpyDeviceToHost, st));
     return IAC_OK;
 }
 
@@ -2109,8 +2516,8 @@ int plan_of(iac_ctx *ctx, const PairRun &R, int cell_vox, int box_cap, int regio
     iac_pair_plan *pl = find_plan(ctx, R.d_kmap, R.npix, cell_vox, box_cap, region, S);
     if (pl && (std::memcmp(&pl->g, &g, sizeof(g)) != 0 || pl->cell_ext != cext)) pl = nullptr;
     if (!pl) {
-        // reuse the oldest unpinned slot beyond four cached plans
-        if (ctx->pair_plans.size() >= 4) {
+        // reuse the oldest unpinned slot beyond eight cached plans
+        if (ctx->pair_plans.size() >= 8) {
             for (auto it = ctx->pair_plans.begin(); it != ctx->pair_plans.end(); ++it) {
                 if ((*it)->pins > 0) continue;
                 if ((*it)->d_tasks) IAC_HIP(hipFree((*it)->d_tasks));
@@ -2139,6 +2546,7 @@ int plan_of(iac_ctx *ctx, const PairRun &R, int cell_vox, int box_cap, int regio
             }
         } else {
             build_tasks(*pl, R.ordered);
+            if (region <= kRegionStrips) merge_strips(*pl, kRegionStrips - region);
             if (pl->tasks.size() > kMaxGridBlocks)
                 return fail(IAC_ERR_LIMIT,
                             "pair engine: more than 2^22 tasks (raise the task region or the cell size)");
@@ -2154,14 +2562,18 @@ int plan_of(iac_ctx *ctx, const PairRun &R, int cell_vox, int box_cap, int regio
     return IAC_OK;
 }
 
+bool default_options(iac_ctx *ctx);
+
 // Cell grid of the k-map (two host round trips for the extents) and the task
 // table, from the context's cache when the geometry matches.  h_off: also the frames' offsets,
 // read back with them (valid until the context's next call).
+// strips: also the plan of the run's strips for frames of `mean` records (null where they do not
+// suit it).
 int get_plan(iac_ctx *ctx, hipStream_t st, const PairRun &R, int cell_vox, int box_cap, int region,
-             iac_pair_plan **out, const uint64_t **h_off = nullptr)
+             iac_pair_plan **out, const uint64_t **h_off = nullptr, double mean = 0, iac_pair_plan **strips = nullptr)
 {
     void *ext = nullptr;
-    IAC_TRY(scratch(ctx, 3, (6 + 6 * (size_t)kMaxCells) * sizeof(uint32_t), &ext));
+    IAC_TRY(scratch(ctx, 3, (6 + 6 * (size_t)(kMaxCells + kMaxStrips)) * sizeof(uint32_t), &ext));
     uint32_t *d_ext = static_cast<uint32_t *>(ext);
     const size_t off_bytes = h_off ? ((size_t)R.nframes + 1) * sizeof(uint64_t) : 0;
     PlanRead read;
@@ -2169,13 +2581,38 @@ int get_plan(iac_ctx *ctx, hipStream_t st, const PairRun &R, int cell_vox, int b
     float kmin[3], ext3[3];
     IAC_TRY(kmap_extents(st, R.d_kmap, R.npix, d_ext, read, kmin, ext3));
     const CellGeom g = cell_grid(kmin, ext3, R.spec.P.vox, cell_vox);
-    IAC_TRY(cell_extents(st, R.d_kmap, R.npix, g, d_ext + 6, read));
+    IAC_TRY(cell_extents(st, R.d_kmap, R.npix, g, d_ext + 6, read.cells));
     if (h_off) {
         IAC_HIP(hipMemcpyAsync(read.more, R.d_frame_off, off_bytes, hipMemcpyDeviceToHost, st));
         *h_off = read.more;
     }
+    StripShape shape{};
+    const CellGeom &sg = shape.g;
+    if (strips) {
+        *strips = nullptr;
+        if (default_options(ctx)) shape = strip_shape(kmin, ext3, R, mean);
+        if (sg.ncv > 0) IAC_TRY(cell_extents(st, R.d_kmap, R.npix, sg, d_ext + 6 + 6 * kMaxCells, read.strips));
+    }
     IAC_HIP(hipStreamSynchronize(st));
-    return plan_of(ctx, R, cell_vox, box_cap, region, g, read.cells, out);
+    IAC_TRY(plan_of(ctx, R, cell_vox, box_cap, region, g, read.cells, out));
+    if (sg.ncv > 0) {
+        (*out)->pins++;  // stays while the strips' plan takes a place in the cache
+        iac_pair_plan *sp = nullptr;
+        const int rc = plan_of(ctx, R, sg.ncv, (int)(kStripBox1 / 4), kRegionStrips - shape.per, sg, read.strips, &sp);
+        (*out)->pins--;
+        if (rc != IAC_OK) return rc;
+        bool fit = !sp->tasks.empty();
+        for (const Task &t : sp->tasks) fit = fit && t.inbox;  // every pair lands in the box, inside the mesh
+        if (fit) *strips = sp;
+    }
+    return IAC_OK;
+}
+
+// A context without engine options set: the options name the walk's settings, so they select it.
+bool default_options(iac_ctx *ctx)
+{
+    return !(ctx->pair_mode || ctx->cell_vox || ctx->cell_vox_v || ctx->box_cap || ctx->task_region ||
+             ctx->pair_prefetch || ctx->frame_chunk);
 }
 
 // Frame chunks inside each group, balanced by pair work: a chunk closes once its
@@ -2237,6 +2674,16 @@ struct Bufs {
     uint32_t ntasks;
     CellGeom g;
     int box_cap;
+    // strips (nst == 0: none)
+    float4 *st_rec;
+    uint32_t *st_cs, *st_bound, *st_usable;
+    unsigned long long *st_self;
+    Chunk *st_chunks;
+    uint32_t st_nchunks;
+    const Task *st_tasks;
+    uint32_t nst;
+    StripGeom st_g;
+    size_t st_box;  // bytes of the largest box
 };
 
 // per frame, the records of its fullest cell: after the frames' cell starts
@@ -2251,7 +2698,8 @@ void launch_pairs_box(int pf, bool fast, int walk, dim3 grid, hipStream_t st, co
 {
     auto go = [&](auto kernel) {
         hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, st, b.srec, R.d_frame_off, b.cs, b.d_chunks, b.d_tasks,
-                           b.ntasks, b.g, R.spec, target, nvox, dropped, b.d_flag, R.d_rots, cell_max(R, b));
+                           b.ntasks, b.g, R.spec, target, nvox, dropped, b.d_flag, R.d_rots, cell_max(R, b),
+                           b.nst ? b.st_usable : nullptr);
     };
     constexpr bool kFast = K == kKindAc3d && !O;
     if ((O || pf == 1) && fast) {
@@ -2296,20 +2744,31 @@ int enqueue(iac_ctx *ctx, hipStream_t st, const PairRun &R, const Bufs &b, bool 
         hipLaunchKernelGGL(fill_u64_kernel, dim3(1), dim3(256), 0, st, b.d_self, (size_t)R.ngroups);
     }
     hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, b.d_flag, 1u, (size_t)1);
+    if (b.nst) {
+        hipLaunchKernelGGL(fill_u64_kernel, dim3(1), dim3(256), 0, st, b.st_self, (size_t)R.ngroups);
+        hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, b.st_usable, 1u, (size_t)1);
+        hipLaunchKernelGGL(strip_sort_kernel, dim3(R.nframes), dim3(kBlock), 0, st, R.rec, R.d_frame_off, b.st_g,
+                           b.st_rec, b.st_cs, S, b.d_goff, R.ngroups, b.st_self, b.st_usable, b.st_bound);
+        IAC_HIP(hipGetLastError());
+    }
     if (S.kind == kKindAc3d) {
         if (ordered)
             hipLaunchKernelGGL((cell_sort_kernel<kKindAc3d, true>), dim3(R.nframes), dim3(kBlock), 0, st, R.rec,
-                               R.d_frame_off, b.g, b.srec, b.cs, S, b.d_goff, R.ngroups, b.d_self, b.d_flag, cell_max(R, b));
+                               R.d_frame_off, b.g, b.srec, b.cs, S, b.d_goff, R.ngroups, b.d_self, b.d_flag, cell_max(R, b),
+                               b.nst ? b.st_usable : nullptr);
         else
             hipLaunchKernelGGL((cell_sort_kernel<kKindAc3d, false>), dim3(R.nframes), dim3(kBlock), 0, st, R.rec,
-                               R.d_frame_off, b.g, b.srec, b.cs, S, b.d_goff, R.ngroups, b.d_self, b.d_flag, cell_max(R, b));
+                               R.d_frame_off, b.g, b.srec, b.cs, S, b.d_goff, R.ngroups, b.d_self, b.d_flag, cell_max(R, b),
+                               b.nst ? b.st_usable : nullptr);
     } else {
         if (ordered)
             hipLaunchKernelGGL((cell_sort_kernel<kKindCq, true>), dim3(R.nframes), dim3(kBlock), 0, st, R.rec,
-                               R.d_frame_off, b.g, b.srec, b.cs, S, b.d_goff, R.ngroups, b.d_self, b.d_flag, cell_max(R, b));
+                               R.d_frame_off, b.g, b.srec, b.cs, S, b.d_goff, R.ngroups, b.d_self, b.d_flag, cell_max(R, b),
+                               b.nst ? b.st_usable : nullptr);
         else
             hipLaunchKernelGGL((cell_sort_kernel<kKindCq, false>), dim3(R.nframes), dim3(kBlock), 0, st, R.rec,
-                               R.d_frame_off, b.g, b.srec, b.cs, S, b.d_goff, R.ngroups, b.d_self, b.d_flag, cell_max(R, b));
+                               R.d_frame_off, b.g, b.srec, b.cs, S, b.d_goff, R.ngroups, b.d_self, b.d_flag, cell_max(R, b),
+                               b.nst ? b.st_usable : nullptr);
     }
     IAC_HIP(hipGetLastError());
     auto *target = ordered ? reinterpret_cast<unsigned long long *>(R.d_mesh) : b.H;
@@ -2319,6 +2778,18 @@ int enqueue(iac_ctx *ctx, hipStream_t st, const PairRun &R, const Bufs &b, bool 
         const int pf = ordered || ctx->pair_prefetch == 0 || ctx->pair_prefetch == 1 ? 1 : (ctx->pair_prefetch == 4 ? 4 : 8);
         // block = chunk * ntasks + task; whole chunks per launch, the slice's chunks by pointer
         const int walk = walks(ctx, R) ? 1 : 0;
+        if (b.nst) {
+            const bool wide = b.st_box > kStripBox2;  // one block of 1,024 threads per CU, or two of 512
+            auto kern = b.st_g.g.av == 0 ? (wide ? strip_kernel<0, 1024> : strip_kernel<0, 512>)
+                                       : (wide ? strip_kernel<1, 1024> : strip_kernel<1, 512>);
+            const uint32_t sper = std::max<uint32_t>(1, kMaxGridBlocks / b.nst);
+            for (uint32_t c0 = 0; c0 < b.st_nchunks; c0 += sper) {
+                hipLaunchKernelGGL(kern, dim3(b.nst * std::min(sper, b.st_nchunks - c0)), dim3(wide ? 1024 : 512), b.st_box,
+                                   st, b.st_rec, R.d_frame_off, b.st_cs, b.st_chunks + c0, b.st_tasks, b.nst, b.st_g.g.ncv,
+                                   S, target, nvox, ctx->d_counters, b.st_usable, b.st_bound, R.d_rots);
+                IAC_HIP(hipGetLastError());
+            }
+        }
         const uint32_t per = std::max<uint32_t>(1, kMaxGridBlocks / b.ntasks);
         for (uint32_t c0 = 0; c0 < b.nchunks; c0 += per) {
             Bufs bs = b;
@@ -2338,7 +2809,8 @@ int enqueue(iac_ctx *ctx, hipStream_t st, const PairRun &R, const Bufs &b, bool 
     if (!ordered) {
         const size_t centre = (size_t)S.P.c0 + (size_t)S.P.c1 * S.P.sab + (size_t)S.P.c2 * S.P.sab * S.P.sab;
         hipLaunchKernelGGL(symmetrize_kernel, dim3(zb), dim3(256), 0, st, b.H,
-                           reinterpret_cast<unsigned long long *>(R.d_mesh), nvox, R.ngroups, centre, b.d_self);
+                           reinterpret_cast<unsigned long long *>(R.d_mesh), nvox, R.ngroups, centre, b.d_self,
+                           b.nst ? b.st_self : b.d_self, b.nst ? b.st_usable : nullptr);
         IAC_HIP(hipGetLastError());
     }
     return IAC_OK;
@@ -2397,6 +2869,45 @@ Sizes sizes_of(const PairRun &R, int nc, size_t nchunks)
                  up(std::max<size_t>(1, nchunks) * sizeof(Chunk))};
 }
 
+// Bytes of a run's strip buffers, and their places from p on.
+size_t strip_bytes(const PairRun &R, const iac_pair_plan *sp, size_t nchunks)
+{
+    if (!sp) return 0;
+    auto up = [](size_t x) { return (x + 255) / 256 * 256; };
+    return up(R.n_total * sizeof(float4)) + up((size_t)R.nframes * (sp->g.ncv + 2) * sizeof(uint32_t)) +
+           up((R.ngroups + 1) * sizeof(unsigned long long)) + up(std::max<size_t>(1, nchunks) * sizeof(Chunk));
+}
+void strip_place(Bufs &b, char *p, const PairRun &R, const iac_pair_plan *sp, size_t nchunks)
+{
+    b.nst = 0;
+    if (!sp) return;
+    auto up = [](size_t x) { return (x + 255) / 256 * 256; };
+    b.st_rec = reinterpret_cast<float4 *>(p);
+    p += up(R.n_total * sizeof(float4));
+    b.st_cs = reinterpret_cast<uint32_t *>(p);
+    b.st_bound = b.st_cs + (size_t)R.nframes * (sp->g.ncv + 1);
+    p += up((size_t)R.nframes * (sp->g.ncv + 2) * sizeof(uint32_t));
+    b.st_self = reinterpret_cast<unsigned long long *>(p);
+    b.st_usable = reinterpret_cast<uint32_t *>(b.st_self + R.ngroups);
+    p += up((R.ngroups + 1) * sizeof(unsigned long long));
+    b.st_chunks = reinterpret_cast<Chunk *>(p);
+    b.st_nchunks = (uint32_t)nchunks;
+    b.st_tasks = sp->d_tasks;
+    b.nst = (uint32_t)sp->tasks.size();
+    b.st_g = StripGeom{sp->g, FLT_MAX, -FLT_MAX, 0.0f};
+    float zlo = FLT_MAX, zhi = -FLT_MAX;
+    for (int c = 0; c < sp->g.ncv; c++) {
+        const uint32_t *e = &sp->cell_ext[6 * (size_t)c];
+        if (e[0] == 0xffffffffu) continue;  // no pixel there
+        b.st_g.ulo = std::min(b.st_g.ulo, unkey(e[sp->g.au]));
+        b.st_g.uhi = std::max(b.st_g.uhi, unkey(e[3 + sp->g.au]));
+        zlo = std::min(zlo, unkey(e[2]));
+        zhi = std::max(zhi, unkey(e[5]));
+    }
+    b.st_g.zext = zhi - zlo;
+    b.st_box = sp->tile_box;
+}
+
 }  // namespace
 
 void free_pair_plans(iac_ctx *ctx)
@@ -2410,21 +2921,26 @@ void free_pair_plans(iac_ctx *ctx)
 }
 
 namespace {
-// The group offsets and the chunk table to the device, through page-locked staging: the host does
+// The group offsets and the chunk tables to the device, through page-locked staging: the host does
 // not wait for the copies.
-int upload_tables(iac_ctx *ctx, hipStream_t st, const PairRun &R, const std::vector<Chunk> &chunks, uint32_t *d_goff,
-                  Chunk *d_chunks)
+int upload_tables(iac_ctx *ctx, hipStream_t st, const PairRun &R, const std::vector<Chunk> &chunks,
+                  const std::vector<Chunk> &schunks, uint32_t *d_goff, Chunk *d_chunks, Chunk *d_schunks)
 {
     const size_t bg = (R.ngroups + 1) * sizeof(uint32_t), bc = chunks.size() * sizeof(Chunk);
+    const size_t bs = schunks.size() * sizeof(Chunk);
     void *p = nullptr;
-    IAC_TRY(pinned(ctx, 1, bg + bc, &p));
-    std::memcpy(p, R.h_group_off, bg);
-    IAC_HIP(hipMemcpyAsync(d_goff, p, bg, hipMemcpyHostToDevice, st));
-    if (bc) {
-        char *c = static_cast<char *>(p) + bg;
-        std::memcpy(c, chunks.data(), bc);
-        IAC_HIP(hipMemcpyAsync(d_chunks, c, bc, hipMemcpyHostToDevice, st));
-    }
+    IAC_TRY(pinned(ctx, 1, bg + bc + bs, &p));
+    char *c = static_cast<char *>(p);
+    auto put = [&](void *dst, const void *src, size_t n) -> int {
+        if (!n) return IAC_OK;
+        std::memcpy(c, src, n);
+        IAC_HIP(hipMemcpyAsync(dst, c, n, hipMemcpyHostToDevice, st));
+        c += n;
+        return IAC_OK;
+    };
+    IAC_TRY(put(d_goff, R.h_group_off, bg));
+    IAC_TRY(put(d_chunks, chunks.data(), bc));
+    IAC_TRY(put(d_schunks, schunks.data(), bs));
     return upload_done(ctx);
 }
 }  // namespace
@@ -2435,16 +2951,22 @@ int pairs_run(iac_ctx *ctx, const PairRun &R)
     if (R.n_total >= (1ull << 32)) return fail(IAC_ERR_LIMIT, "pair engine: at most 2^32 - 1 records per call");
     iac_pair_plan *pl = nullptr;
     const uint64_t *off = nullptr;
-    IAC_TRY(get_plan(ctx, st, R, cell_vox_of(ctx, R), box_cap_of(ctx, R), region_of(ctx, R), &pl, &off));
+    iac_pair_plan *sp = nullptr;
+    IAC_TRY(get_plan(ctx, st, R, cell_vox_of(ctx, R), box_cap_of(ctx, R), region_of(ctx, R), &pl, &off,
+                     (double)R.n_total / std::max(1u, R.nframes), &sp));
     const std::vector<Chunk> chunks = make_chunks(off, R.nframes, R.h_group_off, R.ngroups, fchunk_of(ctx), R.h_rots);
     IAC_TRY(check_chunks(off, chunks));
+    std::vector<Chunk> schunks;
+    if (sp)
+        schunks = make_chunks(off, R.nframes, R.h_group_off, R.ngroups, strip_chunk(R.nframes, sp->tasks.size()), R.h_rots);
     const int nc = pl->g.ncu * pl->g.ncv;
     const Sizes z = sizes_of(R, nc, chunks.size());
     // scratch: sorted records + cell offsets (slot 1), H + group offsets + self + chunks (slot 2)
     void *s1 = nullptr, *s2 = nullptr;
-    IAC_TRY(scratch(ctx, 1, z.srec + z.cs, &s1));
+    IAC_TRY(scratch(ctx, 1, z.srec + z.cs + strip_bytes(R, sp, schunks.size()), &s1));
     IAC_TRY(scratch(ctx, 2, z.h + z.goff + z.self + z.chunks, &s2));
     Bufs b{};
+    strip_place(b, static_cast<char *>(s1) + z.srec + z.cs, R, sp, schunks.size());
     b.srec = static_cast<float4 *>(s1);
     b.cs = reinterpret_cast<uint32_t *>(static_cast<char *>(s1) + z.srec);
     char *p2 = static_cast<char *>(s2);
@@ -2458,7 +2980,7 @@ int pairs_run(iac_ctx *ctx, const PairRun &R)
     b.ntasks = (uint32_t)pl->tasks.size();
     b.g = pl->g;
     b.box_cap = pl->box_cap;
-    IAC_TRY(upload_tables(ctx, st, R, chunks, b.d_goff, b.d_chunks));
+    IAC_TRY(upload_tables(ctx, st, R, chunks, schunks, b.d_goff, b.d_chunks, b.st_chunks));
     return enqueue(ctx, st, R, b, true);
 }
 
@@ -2485,15 +3007,12 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
     *done = false;
     const PairSpec &S = R.spec;
     const bool ordered = R.ordered;
-    // the engine's options select the engine
-    if (ctx->pair_mode || ctx->cell_vox || ctx->cell_vox_v || ctx->box_cap || ctx->task_region || ctx->pair_prefetch ||
-        ctx->frame_chunk)
-        return IAC_OK;
+    if (!default_options(ctx)) return IAC_OK;
     // round_away and the boxes' 24-bit products need |q vox| < 2^22
     if (!(std::sqrt((double)S.P.cut_sq) * S.P.vox < 4194304.0) || R.nframes == 0) return IAC_OK;
     hipStream_t st = ctx->stream;
     void *ext = nullptr;
-    IAC_TRY(scratch(ctx, 3, (6 + 6 * (size_t)kMaxCells) * sizeof(uint32_t), &ext));
+    IAC_TRY(scratch(ctx, 3, (6 + 6 * (size_t)(kMaxCells + kMaxStrips)) * sizeof(uint32_t), &ext));
     uint32_t *d_ext = static_cast<uint32_t *>(ext);
     float kmin[3], ext3[3];
     PlanRead read;
@@ -2540,8 +3059,8 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
         auto *d_kept = d_self + R.ngroups;
         auto *d_plain = reinterpret_cast<uint32_t *>(d_kept + 1);
         auto *d_chunks = reinterpret_cast<Chunk *>(p2 + bh + bg + bs);
-        IAC_TRY(upload_tables(ctx, st, R, chunks, d_goff, d_chunks));
-        IAC_TRY(cell_extents(st, R.d_kmap, R.npix, g, d_ext + 6, read));
+        IAC_TRY(upload_tables(ctx, st, R, chunks, {}, d_goff, d_chunks, nullptr));
+        IAC_TRY(cell_extents(st, R.d_kmap, R.npix, g, d_ext + 6, read.cells));
         auto blocks = [](size_t n) { return (unsigned)std::max<size_t>(1, std::min<size_t>(4096, (n + 255) / 256)); };
         const size_t ncs = R.nframes * (nkey + 1);
         hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks(ncs)), dim3(256), 0, st, cs, 0u, ncs);
@@ -2587,7 +3106,8 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
         if (!ordered) {
             const size_t centre = (size_t)S.P.c0 + (size_t)S.P.c1 * S.P.sab + (size_t)S.P.c2 * S.P.sab * S.P.sab;
             hipLaunchKernelGGL(symmetrize_kernel, dim3(blocks(nvox * R.ngroups)), dim3(256), 0, st, H,
-                               reinterpret_cast<unsigned long long *>(R.d_mesh), nvox, R.ngroups, centre, d_self);
+                               reinterpret_cast<unsigned long long *>(R.d_mesh), nvox, R.ngroups, centre, d_self, d_self,
+                               (const uint32_t *)nullptr);
             IAC_HIP(hipGetLastError());
         }
         *done = true;
@@ -2602,7 +3122,7 @@ struct PairBatch {
     iac_ctx *ctx = nullptr;
     PairRun R{};
     std::vector<uint32_t> group_off;
-    void *mem = nullptr;     // srec | cs | H | goff | self | chunks | tasks
+    void *mem = nullptr;     // srec | cs | H | goff | self | chunks | tasks | strips' tasks and buffers
     Bufs b{};
 };
 
@@ -2612,12 +3132,17 @@ int pairs_prepare(iac_ctx *ctx, const PairRun &R0, PairBatch **out)
     hipStream_t st = ctx->stream;
     if (R0.n_total >= (1ull << 32)) return fail(IAC_ERR_LIMIT, "pair engine: at most 2^32 - 1 records per call");
     iac_pair_plan *pl = nullptr;
-    IAC_TRY(get_plan(ctx, st, R0, cell_vox_of(ctx, R0), box_cap_of(ctx, R0), region_of(ctx, R0), &pl));
+    iac_pair_plan *sp = nullptr;
+    IAC_TRY(get_plan(ctx, st, R0, cell_vox_of(ctx, R0), box_cap_of(ctx, R0), region_of(ctx, R0), &pl, nullptr,
+                     (double)R0.n_total / std::max(1u, R0.nframes), &sp));
     std::vector<uint64_t> off(R0.nframes + 1);
     IAC_HIP(hipMemcpyAsync(off.data(), R0.d_frame_off, off.size() * 8, hipMemcpyDeviceToHost, st));
     IAC_HIP(hipStreamSynchronize(st));
     const std::vector<Chunk> chunks = make_chunks(off.data(), R0.nframes, R0.h_group_off, R0.ngroups, fchunk_of(ctx));
     IAC_TRY(check_chunks(off.data(), chunks));
+    std::vector<Chunk> schunks;
+    if (sp)
+        schunks = make_chunks(off.data(), R0.nframes, R0.h_group_off, R0.ngroups, strip_chunk(R0.nframes, sp->tasks.size()));
     auto *B = new PairBatch();
     B->ctx = ctx;
     B->R = R0;
@@ -2626,7 +3151,10 @@ int pairs_prepare(iac_ctx *ctx, const PairRun &R0, PairBatch **out)
     const int nc = pl->g.ncu * pl->g.ncv;
     const Sizes z = sizes_of(B->R, nc, chunks.size());
     const size_t tbytes = std::max<size_t>(1, pl->tasks.size()) * sizeof(Task);
-    const size_t total = z.srec + z.cs + z.h + z.goff + z.self + z.chunks + tbytes;
+    auto up = [](size_t x) { return (x + 255) / 256 * 256; };
+    const size_t base = up(z.srec + z.cs + z.h + z.goff + z.self + z.chunks + tbytes);
+    const size_t stask = sp ? up(sp->tasks.size() * sizeof(Task)) : 0;
+    const size_t total = base + stask + strip_bytes(B->R, sp, schunks.size());
     hipError_t e = hipMalloc(&B->mem, total);
     if (e != hipSuccess) {
         delete B;
@@ -2652,6 +3180,14 @@ int pairs_prepare(iac_ctx *ctx, const PairRun &R0, PairBatch **out)
         e = hipMemcpyAsync(b.d_chunks, chunks.data(), chunks.size() * sizeof(Chunk), hipMemcpyHostToDevice, st);
     if (e == hipSuccess && !pl->tasks.empty())
         e = hipMemcpyAsync(tasks, pl->tasks.data(), pl->tasks.size() * sizeof(Task), hipMemcpyHostToDevice, st);
+    if (sp) {  // a copy of the strips' tasks too: the cache may drop their plan
+        strip_place(b, p + base + stask, B->R, sp, schunks.size());
+        b.st_tasks = reinterpret_cast<Task *>(p + base);
+        if (e == hipSuccess)
+            e = hipMemcpyAsync(p + base, sp->tasks.data(), sp->tasks.size() * sizeof(Task), hipMemcpyHostToDevice, st);
+        if (e == hipSuccess && !schunks.empty())
+            e = hipMemcpyAsync(b.st_chunks, schunks.data(), schunks.size() * sizeof(Chunk), hipMemcpyHostToDevice, st);
+    }
     if (e == hipSuccess) e = hipStreamSynchronize(st);
     if (e != hipSuccess) {
         (void)hipFree(B->mem);

@@ -286,3 +286,46 @@ def test_library_tuner(ctx, dev, interp1, interp2):
             assert np.array_equal(mesh_np(m), ref), x
     finally:
         c.close()
+
+
+@pytest.mark.parametrize("rows,cols,dist,edge", [(128, 128, 2e5, 63), (60, 200, 1e5, 95), (210, 70, 3e5, 127),
+                                                 (256, 256, 2e4, 61), (400, 64, 4e5, 191)])
+@pytest.mark.parametrize("kind", ["ones", "counts", "heavy", "full", "large"])
+def test_strips_vs_tiles(ctx, dev, rows, cols, dist, edge, kind):
+    """Nearest-neighbour batches of frames with enough photons for strips, against the
+    global-atomic tile kernel, equal in every voxel: wide and tall detectors, weights that fill a
+    32-bit box after a few frames ("heavy") or within one ("full"), or are too large for it
+    ("large"), frames that are empty, of one photon or of one corner, a zoom that cuts pairs, with
+    a rotation per frame and without."""
+    import incohautocorrelate_amd as iac
+    from gpu_helpers import gpu_batch
+
+    rng = np.random.default_rng(rows + 3 * edge)
+    km, _, _, mq = iac.calc_kmap(iac.generate_pixel_map(rows, cols, 75.0, [0, 0, dist], (1, 0, 0), (0, 1, 0)))
+    pix, cnt = [], []
+    nf = 120
+    for f in range(nf):
+        n = [0, 1, 900][f] if f < 3 else int(rng.integers(1200, 3600)) * (3 if kind == "full" and f % 20 == 19 else 1)
+        pix.append(np.sort(rng.integers(0, rows * cols if f != 2 else 16 * cols, n)))
+        top = {"ones": 1, "heavy": 60, "full": 129}.get(kind, 5)
+        cnt.append(np.full(n, top) if top > 5 else rng.integers(1, top + 1, n))
+    if kind == "large":
+        cnt[9][7] = 130
+    off = np.concatenate([[0], np.cumsum([p.size for p in pix])])
+    pix, cnt = np.concatenate(pix), np.concatenate(cnt)
+    rots = W.random_rotations(nf, 5).astype(np.float32)
+    rots[:60] = rots[0]
+    rots[60:75] = np.eye(3, dtype=np.float32).reshape(9)
+    for zoom, r in ((1.0, None), (1.8, None), (1.0, rots)):
+        shape = iac.mesh_shape_big(mq, edge, zoom)
+        got = []
+        for kernel in (0, 1):
+            ctx.set_option(iac.OPT_AC3D_KERNEL, kernel)
+            try:
+                before = ctx.dropped()
+                m = mesh_np(gpu_batch(ctx, dev, km, pix, cnt, off, shape, rots=r))
+                got.append((m, ctx.dropped() - before))
+            finally:
+                ctx.set_option(iac.OPT_AC3D_KERNEL, 0)
+        assert np.array_equal(got[0][0], got[1][0]), (zoom, r is None)
+        assert got[0][1] == got[1][1]
