@@ -1326,8 +1326,9 @@ __device__ __forceinline__ uint32_t tile_key(const CellGeom &g, int side, float 
 }
 
 // Counts of the frames' nonzero pixels per key (cs, zeroed by the caller), the groups' self
-// values (symmetric modes), the number of kept records, and the run's flag, cleared by any record
-// that could make a pair negative, NaN or 2^32 or more (then the pairs take the general value).
+// values (symmetric modes), the number of kept records, and the run's flags: plain[0] is cleared by
+// any record that could make a pair negative, NaN or 2^32 or more, plain[1] by one that could
+// make it negative, NaN or 2^62 or more.
 // Grid: ns blocks per frame.
 template <bool ORD>
 __global__ void __launch_bounds__(kBlock)
@@ -1341,16 +1342,19 @@ __global__ void __launch_bounds__(kBlock)
     const size_t nkey = (size_t)g.ncu * g.ncv * side * side;
     uint32_t *csf = cs + f * (nkey + 1);
     unsigned long long sv = 0, n = 0;
-    bool ok = 1e-37 * S.mult < 0.99;  // a product below 1e-37 adds nothing either way
+    bool ok = true, wide = 1e-37 * S.mult < 0.99;  // a product below 1e-37 adds nothing either way
     for (uint32_t p = (blockIdx.x - f * ns) * kBlock + threadIdx.x; p < npix; p += ns * kBlock) {
         const float I = frames[(size_t)f * npix + p];
         if (I == 0.0f) continue;
         atomicAdd(csf + tile_key(g, side, kmap[3 * (size_t)p + g.au], kmap[3 * (size_t)p + g.av]), 1u);
         n++;
         if (!ORD) sv += self_value<kKindCq>(S, I);
-        ok = ok && I > 0.0f && (double)(I * I) * S.mult < 4294967296.0;
+        const double most = (double)(I * I) * S.mult;
+        ok = ok && most < 4294967296.0;
+        wide = wide && I > 0.0f && most < 0x1p62;
     }
-    if (!ok) plain[0] = 0u;
+    if (!ok || !wide) plain[0] = 0u;
+    if (!wide) plain[1] = 0u;
     for (int o = 32; o > 0; o >>= 1) {
         sv += __shfl_down(sv, o, 64);
         n += __shfl_down(n, o, 64);
@@ -1570,12 +1574,14 @@ __device__ __forceinline__ void tile_by_parts(const float4 *__restrict__ rec, co
 
 // Grid: ntasks per chunk of frames of one group.  Symmetric (nearest) runs bin each unordered pair
 // once into the half mesh, linear ones every ordered pair, self pairs too, into the mesh.
-template <bool LINEAR>
+// WIDE: values up to 2^62, converted in two halves (five instructions for one).  24 frames of 256^2 in
+// 4 groups into 129 x 129 x 3 at a multiplicator of 1e10: 62.7 ms by the engine, 37.4 (31.4 at 1e6).
+template <bool LINEAR, bool WIDE>
 __global__ void __launch_bounds__(kBlock, LINEAR ? 4 : 8)
     cq_tile_kernel(const float4 *__restrict__ srec, uint32_t npix, const uint32_t *__restrict__ cs, int ncell, int side,
                    const Chunk *__restrict__ chunks, const TileTask *__restrict__ tasks, uint32_t ntasks, PairSpec S,
                    unsigned long long *__restrict__ target, size_t nvox, unsigned long long *__restrict__ dropped,
-                   const uint32_t *__restrict__ plain_flag, int by_parts, uint32_t splits)
+                   int by_parts, uint32_t splits)
 {
     __shared__ float part_ext[LINEAR ? 1 : 6][LINEAR ? 1 : kTileParts];  // by parts: min a b c, max a b c
     extern __shared__ unsigned long long box[];  // the plan's largest box
@@ -1589,7 +1595,7 @@ __global__ void __launch_bounds__(kBlock, LINEAR ? 4 : 8)
     const uint32_t share = split * (kBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t shares = splits * (kBlock / 64);
     const bool tri = !LINEAR && T.ci == T.cj;
-    const bool fast = T.inbox && plain_flag[0] != 0u, is_signed = T.sa != 0 && T.sb != 0;
+    const bool fast = T.inbox, is_signed = T.sa != 0 && T.sb != 0;
     unsigned long long *const out = target + (size_t)CH.group * nvox;
     BoxSink sink{box, out, dropped, T.bx0, T.by0, T.bz0, T.bx, T.by, T.bz, S.P.sab, S.P.sc, LINEAR ? 1ull : 2ull,
                  nullptr, 0, 0, 0};
@@ -1608,12 +1614,17 @@ __global__ void __launch_bounds__(kBlock, LINEAR ? 4 : 8)
         return ((S.kc == 2 ? a2 : (S.kb == 2 ? a2 : b2)) + (S.kc == 2 ? b2 : c2)) + z;
     };
     auto add8 = [&](int o, double x) {
-        atomicAdd(reinterpret_cast<unsigned long long *>(boxb + o), (unsigned long long)(uint32_t)x);
+        unsigned long long v = (uint32_t)x;
+        if (WIDE) {  // the high word by an exact scaling, the rest of x without rounding
+            const uint32_t hi = (uint32_t)(x * 0x1p-32);
+            v = (unsigned long long)hi << 32 | (uint32_t)fma((double)hi, -0x1p32, x);
+        }
+        atomicAdd(reinterpret_cast<unsigned long long *>(boxb + o), v);
     };
     // signed voxel scale and byte stride of the first two axes: q times the first is not negative
     const float voxa = T.sa < 0 ? -vox : vox, voxb = T.sb < 0 ? -vox : vox;
     const int sta = T.sa < 0 ? -8 : 8, stb = T.sb < 0 ? -bx8 : bx8;
-    // fast: the pair's voxels lie in the box and its value below 2^32; a pair that fails the cut
+    // fast: the pair's voxels lie in the box; a pair that fails the cut
     // adds 0 (nearest) or is skipped (linear).  kSigned: q keeps its sign along the first two axes;
     // kThin: the box is one voxel deep along the third, whose voxel is then the same for all pairs.
     auto bin_fast = [&](const float4 &a, const f4v &b, auto cut_c, auto signed_c, auto thin_c) {
@@ -1668,7 +1679,7 @@ __global__ void __launch_bounds__(kBlock, LINEAR ? 4 : 8)
         const uint32_t b0 = csf[T.cj * parts], nb = csf[(T.cj + 1) * parts] - b0;
         if (na == 0 || nb == 0) continue;
         const scalar_rec_t brec = (scalar_rec_t)(uintptr_t)(rec + b0);
-        if constexpr (!LINEAR) {
+        if constexpr (!LINEAR && !WIDE) {
             if (by_parts && fast && T.allin && !tri) {
                 tile_by_parts(rec, csf, parts, a0, na, T, vox, S.mult, bx8, bxby8, c8, boxb, part_ext, share, shares);
                 continue;
@@ -3016,7 +3027,7 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
     uint32_t *d_ext = static_cast<uint32_t *>(ext);
     float kmin[3], ext3[3];
     PlanRead read;
-    IAC_TRY(plan_read(ctx, sizeof(uint64_t), &read));
+    IAC_TRY(plan_read(ctx, 2 * sizeof(uint64_t), &read));
     IAC_TRY(kmap_extents(st, R.d_kmap, R.npix, d_ext, read, kmin, ext3));
     const int box_cap = ordered ? kBoxMax : kBoxSmall;
     const size_t nvox = (size_t)S.P.sab * S.P.sab * S.P.sc;
@@ -3065,7 +3076,7 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
         const size_t ncs = R.nframes * (nkey + 1);
         hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks(ncs)), dim3(256), 0, st, cs, 0u, ncs);
         hipLaunchKernelGGL(fill_u64_kernel, dim3(blocks(R.ngroups + 1)), dim3(256), 0, st, d_self, (size_t)R.ngroups + 1);
-        hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, d_plain, 1u, (size_t)1);
+        hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, d_plain, 1u, (size_t)2);
         const unsigned sblocks = ns * R.nframes;
         hipLaunchKernelGGL(ordered ? tile_count_kernel<true> : tile_count_kernel<false>, dim3(sblocks), dim3(kBlock), 0,
                            st, R.d_kmap, d_frames, R.npix, ns, g, side, S, d_goff, R.ngroups, cs, d_self, d_plain,
@@ -3076,14 +3087,17 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
         if (!ordered)
             hipLaunchKernelGGL(fill_u64_kernel, dim3(blocks(nvox * R.ngroups)), dim3(256), 0, st, H, nvox * R.ngroups);
         IAC_HIP(hipGetLastError());
-        IAC_HIP(hipMemcpyAsync(read.more, d_kept, sizeof(uint64_t), hipMemcpyDeviceToHost, st));
+        IAC_HIP(hipMemcpyAsync(read.more, d_kept, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, st));
         IAC_HIP(hipStreamSynchronize(st));
         const uint64_t kept = read.more[0];
+        const uint32_t *flags = reinterpret_cast<const uint32_t *>(read.more + 1);
+        const bool wide = !flags[0];
+        if (!flags[1]) return IAC_OK;  // negative values: the engine's pairs test each
         if ((double)kept < kTileRecords * (double)R.nframes * nc) return IAC_OK;  // sparse frames
         iac_pair_plan *pl = nullptr;
         IAC_TRY(plan_of(ctx, R, side, box_cap, kRegionTiles, g, read.cells, &pl));
         if (!pl->tiles_fit) continue;
-        const bool by_parts = !ordered && (double)kept >= kPartRecords * (double)R.nframes * (double)nkey;
+        const bool by_parts = !ordered && !wide && (double)kept >= kPartRecords * (double)R.nframes * (double)nkey;
         auto *target = ordered ? reinterpret_cast<unsigned long long *>(R.d_mesh) : H;
         const uint32_t ntasks = (uint32_t)pl->tiles.size(), nchunks = (uint32_t)chunks.size();
         // few tasks, or tasks of uneven work (dense regions, regions with themselves): several blocks
@@ -3093,13 +3107,15 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
         const uint32_t splits = (uint32_t)std::max(
             1.0, std::min({std::ceil(kTileBlocks / ((double)ntasks * nchunks)), pairs / kTileShare, 4096.0}));
         const uint32_t per = std::max<uint32_t>(1, kMaxGridBlocks / ((uint64_t)ntasks * splits));
+        auto kern = ordered ? (wide ? cq_tile_kernel<true, true> : cq_tile_kernel<true, false>)
+                            : (wide ? cq_tile_kernel<false, true> : cq_tile_kernel<false, false>);
         IAC_TRY(timer_begin(ctx));
         for (uint32_t c0 = 0; c0 < nchunks; c0 += per) {
             const dim3 grid(ntasks * splits * std::min(per, nchunks - c0));
-            hipLaunchKernelGGL(ordered ? cq_tile_kernel<true> : cq_tile_kernel<false>, grid, dim3(kBlock),
+            hipLaunchKernelGGL(kern, grid, dim3(kBlock),
                                pl->tile_box * sizeof(unsigned long long), st, srec,
                                R.npix, cs, nc, side, d_chunks + c0, pl->d_tiles, ntasks, S, target, nvox, ctx->d_counters,
-                               d_plain, by_parts ? 1 : 0, splits);
+                               by_parts ? 1 : 0, splits);
             IAC_HIP(hipGetLastError());
         }
         IAC_TRY(timer_end(ctx));
