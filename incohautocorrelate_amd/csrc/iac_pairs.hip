@@ -3,7 +3,9 @@
 // (AutoCorr_CQ_small, IAC/kernel.cl:27-184).
 //
 // Input: photon or pixel records {kx, ky, kz, value} of nframes frames; frames
-// form groups (frame range -> one output mesh each).  One call:
+// form groups (frame range -> one output mesh each).  Three ways to take the pairs, to the same
+// bits: detector strips (AC_uw nearest neighbour, runs of many pairs; "AC_uw strips" below), region
+// tiles (dense C(q) images; "Region tiles" below), and the cell-offset walk for the rest:
 //   1. plan (cached): the k-map's extents define a cell grid over its two
 //      widest k axes (cell side `cell_vox` voxels); per-cell k extents bound
 //      the voxel box reached by the pairs of every cell offset delta.
@@ -1760,7 +1762,7 @@ __global__ void __launch_bounds__(kBlock, LINEAR ? 4 : 8)
 // w_max^2 n m to a voxel (n records, m in its fullest strip), and a block flushes before
 // the frames it has added could pass 2^32.
 // 3,000 frames of 2,090 photons on a 1024^2 detector into 257^3: 9.0 ms by the walk, 6.5 by strips
-// (1.0e12 pairs/s); 800 frames with a rotation each 10.1 and 4.9 (a task of several distances
+// (1.0e12 pairs/s); 800 frames with a rotation each 10.0 and 4.7 (a task of several distances
 // flushes each voxel of its mesh 1.2 times, the walk's small boxes 2 to 3 times).  Bound: VALU issue
 // at three quarters, a fifth of the lanes empty; with rotations the scattered atomics of the flush.
 // Lanes without a record are off rather than adding 0: their zeros would meet in one address, 13
@@ -2456,7 +2458,9 @@ struct StripShape {
 // starting an item.  The shape of least cost, in clocks of a CU per frame: 27 per 64 pairs (VALU
 // issue; 34 with one block per CU, whose flush nothing covers), 6 pairs' worth for an item's start,
 // 2.7 per voxel flushed to a rotated mesh (scattered atomics) or 1.5 to a plain one, shared
-// by a chunk's frames.  Measured: 34 picks seven-row boxes and 6.5 ms, 27 twelve-row ones and 6.8.
+// by a chunk's frames.  Shapes that leave waves or CUs idle pay for it (60 frames of 21,000 photons in
+// strips of half the detector: 90 ms, the walk 18), and no shape near the walk's cost
+// is taken.  Measured: 34 picks seven-row boxes and 6.5 ms, 27 twelve-row ones and 6.8.
 StripShape strip_shape(const float kmin[3], const float ext3[3], const PairRun &R, double mean)
 {
     StripShape best{};
@@ -2471,6 +2475,7 @@ StripShape strip_shape(const float kmin[3], const float ext3[3], const PairRun &
     // (a rotated mesh's smaller flushes more)
     const double pairs = 0.5 * mean * mean * R.nframes;
     if (!(wide * deep * 4 * 3 <= kStripBox1) || !(pairs >= (R.h_rots ? 0x1p26 : 0x1p28))) return best;
+    const double walk = 0.5 * mean * mean / 64 * 55;  // what it takes for the pairs
     double least = 1e300, h_best = 0;
     for (int m = 1; m <= 8; m++)
         for (double h = 1; h <= 64; h *= 1.0905) {  // eighths of an octave
@@ -2482,7 +2487,13 @@ StripShape strip_shape(const float kmin[3], const float ext3[3], const PairRun &
             for (int k = 1; k < 32; k++) groups += 0.5 * std::erfc((64.0 * k + 0.5 - L) / std::sqrt(2 * L));
             const double items = n * (n + m) / (2.0 * m), tasks = std::ceil(n / m);
             const double frames = R.h_rots ? 1 : strip_chunk(R.nframes, (size_t)tasks);
-            const double cost = items * groups * (nb + 7.5) * (box > kStripBox2 ? 34 : 27) + tasks * box / 4 * (R.h_rots ? 2.7 : 1.5) / frames;
+            // idle waves where a block has few items, idle CUs where there are few blocks
+            const double waves = box > kStripBox2 ? 16 : 8, slots = box > kStripBox2 ? 256 : 512;
+            const double busy = std::min(1.0, frames * items / tasks / (3 * waves)) *
+                                std::min(1.0, tasks * R.nframes / frames / (6 * slots));
+            const double pair_cost = items * groups * (nb + 7.5) * (box > kStripBox2 ? 34 : 27) / busy;
+            if (pair_cost > 1.3 * walk) continue;  // (the model is a sixth too high for strips)
+            const double cost = pair_cost + tasks * box / 4 * (R.h_rots ? 2.7 : 1.5) / frames;
             if (cost < least) {
                 least = cost;
                 h_best = h;

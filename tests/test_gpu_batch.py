@@ -289,7 +289,7 @@ def test_library_tuner(ctx, dev, interp1, interp2):
 
 
 @pytest.mark.parametrize("rows,cols,dist,edge", [(128, 128, 2e5, 63), (60, 200, 1e5, 95), (210, 70, 3e5, 127),
-                                                 (256, 256, 2e4, 61), (400, 64, 4e5, 191)])
+                                                 (256, 256, 2e4, 61), (400, 64, 4e5, 191), (90, 90, 4e5, 21)])
 @pytest.mark.parametrize("kind", ["ones", "counts", "heavy", "full", "large"])
 def test_strips_vs_tiles(ctx, dev, rows, cols, dist, edge, kind):
     """Nearest-neighbour batches of frames with enough photons for strips, against the
