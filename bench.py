@@ -223,7 +223,8 @@ def main():
     sim = None if args.no_sim else sim_leg(args, iac, W, dev)
 
     traffic = None
-    if tuned and args.kernel != 1:
+    strips = args.kernel != 1 and not (tuned and (tuned.get("mode") or tuned.get("box")))  # the engine's defaults
+    if tuned and args.kernel != 1 and not strips:
         key = (tuned.get("mode") or 1, tuned.get("box") or 1920, tuned.get("cell_vox") or 6,
                tuned.get("frame_chunk") or 32)
         if (tuned.get("cell_vox_v") or key[2]) != key[2] or tuned.get("region"):
@@ -249,8 +250,8 @@ def main():
             "photons": n_total,
             "pair_updates_per_step": updates,
             "seed": args.seed,
-            "kernel": "tile (global atomics)" if args.kernel == 1 else "LDS cell boxes",
-            "step": "prepared frame batch (iac_ac3d_batch_launch): clear + gather + cell sort + pairs + mirror",
+            "kernel": "tile (global atomics)" if args.kernel == 1 else "LDS strips" if strips else "LDS cell boxes",
+            "step": "prepared frame batch (iac_ac3d_batch_launch): clear + gather + sort + pairs + mirror",
             "tuned": tuned,
         },
         # The 16 B read-modify-write of each pair-update lands in an LDS box, not in HBM
@@ -265,7 +266,8 @@ def main():
             "traffic": traffic,
             "traffic_unit": "HBM bytes per launch (rocprofv3 FETCH_SIZE + WRITE_SIZE, copy-scaled)",
             "traffic_over_algorithmic": (traffic / (updates * BYTES_PER_UPDATE)) if traffic else None,
-            "kernel": "pairs_kernel (LDS cell boxes)" if args.kernel != 1 else "ac3d_tiles_kernel<true>",
+            "kernel": ("ac3d_tiles_kernel<true>" if args.kernel == 1 else
+                       "strip_kernel (32-bit LDS boxes of strips)" if strips else "pairs_kernel (LDS cell boxes)"),
             "kernel_avg_ms": k_avg_ms,
             "bytes_per_update": BYTES_PER_UPDATE,
             "peak_basis": "LDS 128 B/clk/CU x 256 CUs x 2.4 GHz" if args.kernel != 1 else "HBM3E 8 TB/s",
@@ -276,6 +278,7 @@ def main():
             "updates_vs_uniform_u64_atomics": value / probes["atomic_u64_per_s"]["uniform"] if probes else None,
             # the kernel's LDS adds (one per distinct unordered pair: (updates - photons) / 2, the self
             # pairs go to the centre separately) against random uint64 adds into a 4096-voxel LDS box
+            # (the strips' adds are 32 bits wide)
             "lds_adds_per_s": (updates - n_total) / 2 / (k_avg_ms * 1e-3) if k_avg_ms > 0 else None,
             "frac_of_lds_atomic_probe": ((updates - n_total) / 2 / (k_avg_ms * 1e-3)
                                          / probes["atomic_u64_per_s"]["lds_box"]

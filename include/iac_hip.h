@@ -89,6 +89,9 @@ int iac_pinned_free(void *h_ptr);
 int iac_ctx_enable_timing(iac_ctx *ctx, int enable);
 int iac_ctx_timing(iac_ctx *ctx, double *ms, uint64_t *launches, int reset);
 /* Context options (tuning and kernel selection for measurement and tests). */
+/* The LDS kernel's options below name the settings of its cell-offset walk: with any of them set, that
+ * walk runs.  With none set, nearest-neighbour AC_uw batches of many pairs are binned by detector
+ * strips and dense C(q) images by region tiles, to the same mesh bits. */
 #define IAC_OPT_AC3D_KERNEL 1 /* 0 automatic, 1 global-atomic tile kernel, 2 LDS cell-box kernel */
 #define IAC_OPT_CELL_VOX 2    /* LDS kernel: cell side (along the widest k axis) in voxels, 0 = default (6 for
                                  AC_uw nearest neighbour, 5 for AC_uw linear, 3 for C(q) nearest neighbour, 4
