@@ -1758,9 +1758,12 @@ __global__ void __launch_bounds__(kBlock, LINEAR ? 4 : 8)
 // j + dv + nv - 1 pair completely, so a wave takes one side's records as lanes and the other's
 // one by one from the scalar unit, with no index work: 22 VALU instructions and one LDS add per
 // 64 pairs.  The box counts w_a w_b; the flush multiplies by the fixed point's 1000.
-// 32 bits are exact: weights are integers in [1, 129] (else the walk runs), a frame adds at most
-// w_max^2 n m to a voxel (n records, m in its fullest strip), and a block flushes before
-// the frames it has added could pass 2^32.
+// 32 bits are exact: weights are integers in [1, 129] (else the walk runs) and a block flushes before
+// the frames it has added could pass 2^32.  For one a the b of a voxel lie in a window one voxel
+// tall, which meets two strips where they are taller than a voxel (three at one voxel, where rounding
+// may reach over both edges), all of them in one task if it holds several distances; so a frame adds
+// at most W A to a voxel, W the sum of its weights and A that of its fullest two (three)
+// strips in a row.
 // 3,000 frames of 2,090 photons on a 1024^2 detector into 257^3: 9.0 ms by the walk, 6.5 by strips
 // (1.0e12 pairs/s); 800 frames with a rotation each 10.0 and 4.7 (a task of several distances
 // flushes each voxel of its mesh 1.2 times, the walk's small boxes 2 to 3 times).  Bound: VALU issue
@@ -1771,14 +1774,15 @@ __global__ void __launch_bounds__(kBlock, LINEAR ? 4 : 8)
 constexpr int kMaxStrips = 512;
 
 // One block per frame, as cell_sort_kernel: records by strip, strip starts, self values; bound[f] =
-// the most a voxel can receive from the frame.  A record's w holds its integer weight and, above 8
+// W A, the most a voxel can receive from the frame.  A record's w holds its integer weight and, above 8
 // bits, its reach: no record of a strip fewer than reach strips away, wherever in it, is beyond the
 // cut.  A strip's records are in order of falling reach (eight classes), so that
 // most batches of b need no cut.  `usable` starts at 1 and is cleared by a weight that is no
-// integer in [1, 129] or a frame whose bound passes 2^32.
+// integer in [1, 129] or a frame whose bound passes 2^32 (any of 2^24 records does: 512 strips).
 struct StripGeom {
     CellGeom g;
     float ulo, uhi, zext;  // extents of the k-map along the strips and the beam
+    int span;              // strips that the window of a voxel can meet
 };
 constexpr int kReachClasses = 8;
 __device__ inline uint32_t strip_reach(const StripGeom &G, float cut_sq, float u)
@@ -1794,7 +1798,7 @@ __global__ void __launch_bounds__(kBlock)
                       unsigned long long *__restrict__ self, uint32_t *__restrict__ usable,
                       uint32_t *__restrict__ bound)
 {
-    __shared__ uint32_t cnt[kMaxStrips * kReachClasses];
+    __shared__ uint32_t cnt[kMaxStrips * kReachClasses], wsum[kMaxStrips];
     __shared__ unsigned long long sred[kBlock / 64];
     __shared__ uint32_t wred[kBlock / 64], nred[kBlock / 64], sums[kBlock / 64];
     const CellGeom &g = G.g;
@@ -1807,31 +1811,33 @@ __global__ void __launch_bounds__(kBlock)
         return cell_of(g, 0.0f, comp(r, g.av)) * kReachClasses + cls;
     };
     for (int c = threadIdx.x; c < kMaxStrips * kReachClasses; c += kBlock) cnt[c] = 0;
+    for (int c = threadIdx.x; c < kMaxStrips; c += kBlock) wsum[c] = 0;
     __syncthreads();
     unsigned long long sv = 0;
-    uint32_t wmax = 0;
-    bool ok = true;
+    bool ok = n < (1u << 24);  // the sums of weights below fit 32 bits
     for (uint32_t i = threadIdx.x; i < n; i += kBlock) {
         const float4 r = rec[base + i];
         if (r.w == 0.0f) continue;
-        atomicAdd(&cnt[place(r, strip_reach(G, S.P.cut_sq, comp(r, g.au)))], 1u);
+        const int bin = place(r, strip_reach(G, S.P.cut_sq, comp(r, g.au)));
+        atomicAdd(&cnt[bin], 1u);
         sv += self_value<kKindAc3d>(S, r.w);
         const bool small = r.w >= 1.0f && r.w <= 129.0f && r.w == truncf(r.w);
         ok = ok && small;
-        if (small) wmax = max(wmax, (uint32_t)r.w);
+        if (small) atomicAdd(&wsum[bin / kReachClasses], (uint32_t)r.w);
     }
     if (!ok) usable[0] = 0u;
     __syncthreads();
     // starts: consecutive bins per thread, whole strips each
     const int per = (nbin / kReachClasses + kBlock - 1) / kBlock;  // strips
-    uint32_t tot = 0, most = 0;
+    uint32_t tot = 0, most = 0, weight = 0;
     for (int k = 0; k < per; k++) {
-        const int c = ((int)threadIdx.x * per + k) * kReachClasses;
-        uint32_t strip = 0;
-        if (c < nbin)
-            for (int e = 0; e < kReachClasses; e++) strip += cnt[c + e];
-        tot += strip;
-        most = max(most, strip);
+        const int c = (int)threadIdx.x * per + k;
+        if (c >= ncell) break;
+        for (int e = 0; e < kReachClasses; e++) tot += cnt[c * kReachClasses + e];
+        uint32_t window = 0;
+        for (int e = c; e < min(c + G.span, ncell); e++) window += wsum[e];
+        weight += wsum[c];
+        most = max(most, window);
     }
     uint32_t x = tot;
     for (int o = 1; o < 64; o <<= 1) {
@@ -1840,13 +1846,13 @@ __global__ void __launch_bounds__(kBlock)
     }
     for (int o = 32; o > 0; o >>= 1) {
         sv += __shfl_down(sv, o, 64);
-        wmax = max(wmax, (uint32_t)__shfl_down(wmax, o, 64));
+        weight += __shfl_down(weight, o, 64);
         most = max(most, (uint32_t)__shfl_down(most, o, 64));
     }
     if (lane == 63) sums[wave] = x;
     if (lane == 0) {
         sred[wave] = sv;
-        wred[wave] = wmax;
+        wred[wave] = weight;
         nred[wave] = most;
     }
     __syncthreads();
@@ -1868,15 +1874,14 @@ __global__ void __launch_bounds__(kBlock)
     }
     if (threadIdx.x == 0) {
         csf[ncell] = all;
-        uint32_t w = 0;
-        most = 0;
+        weight = most = 0;
         sv = 0;
         for (uint32_t k = 0; k < kBlock / 64; k++) {
-            w = max(w, wred[k]);
+            weight += wred[k];
             most = max(most, nred[k]);
             sv += sred[k];
         }
-        const uint64_t b = (uint64_t)w * w * n * most;
+        const uint64_t b = (uint64_t)weight * most;
         if (b >> 32) usable[0] = 0u;
         bound[f] = (uint32_t)b;
         if (sv) {
@@ -2916,7 +2921,8 @@ void strip_place(Bufs &b, char *p, const PairRun &R, const iac_pair_plan *sp, si
     b.st_nchunks = (uint32_t)nchunks;
     b.st_tasks = sp->d_tasks;
     b.nst = (uint32_t)sp->tasks.size();
-    b.st_g = StripGeom{sp->g, FLT_MAX, -FLT_MAX, 0.0f};
+    // (strips are one voxel tall or at least 9 % taller)
+    b.st_g = StripGeom{sp->g, FLT_MAX, -FLT_MAX, 0.0f, sp->g.inv_wv < 0.95f * R.spec.P.vox ? 2 : 3};
     float zlo = FLT_MAX, zhi = -FLT_MAX;
     for (int c = 0; c < sp->g.ncv; c++) {
         const uint32_t *e = &sp->cell_ext[6 * (size_t)c];

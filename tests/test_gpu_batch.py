@@ -329,3 +329,48 @@ def test_strips_vs_tiles(ctx, dev, rows, cols, dist, edge, kind):
                 ctx.set_option(iac.OPT_AC3D_KERNEL, 0)
         assert np.array_equal(got[0][0], got[1][0]), (zoom, r is None)
         assert got[0][1] == got[1][1]
+
+
+# Rows of bright patches on the edges of the detector's strips, as far apart as the distances that
+# one task of the strips holds: each record meets two strips' records in one voxel of that task.
+# "frames": 10,000 frames, a block adds nine of them; "frame": one fills the 32-bit box by itself.
+BRIGHT_ROWS = {"frames": (512, 41, 10_000, (12, 13), [2, 6, 10, 14], 1.18919025, 90),
+               "frame": (1024, 51, 400, (16, 16), [1, 5, 9, 13, 17, 21], 1.0, 129)}
+
+
+def bright_rows(name):
+    import incohautocorrelate_amd as iac
+
+    n, edge, nf, (tall, wide), at, height, count = BRIGHT_ROWS[name]
+    km, _, _, mq = iac.calc_kmap(iac.generate_pixel_map(n, n, 75.0, [0, 0, 5e5], (1, 0, 0), (0, 1, 0)))
+    shape = iac.mesh_shape_big(mq, edge)
+    k = km.reshape(n, n, 3)
+    across = 1 if abs(k[0, -1, 1] - k[0, 0, 1]) > abs(k[-1, 0, 1] - k[0, 0, 1]) else 0  # the index y grows along
+    line = k[n // 2, :, 1] if across else k[:, n // 2, 1]
+    strip = (line - km[:, 1].min()) * shape.voxel_per_dq / height
+    img = np.zeros((n, n), bool)
+    for edge_at in at:
+        c = int(np.argmin(abs(strip - edge_at)))
+        y = slice(c - tall // 2, c - tall // 2 + tall)
+        x = slice(n // 2 - wide // 2, n // 2 - wide // 2 + wide)
+        img[(x, y) if across else (y, x)] = True
+    pix = np.flatnonzero(img)
+    return km, shape, pix, np.full(pix.size, count), nf
+
+
+@pytest.mark.parametrize("name", list(BRIGHT_ROWS))
+def test_strips_bright_rows(ctx, dev, name):
+    """Equal frames whose fullest voxel passes 2^32 in a task of several strip distances: the mesh is
+    that of one frame, by the tile kernel, times their number."""
+    import incohautocorrelate_amd as iac
+    from gpu_helpers import gpu_batch
+
+    km, shape, pix, cnt, nf = bright_rows(name)
+    off = np.arange(nf + 1) * pix.size
+    m = mesh_np(gpu_batch(ctx, dev, km, np.tile(pix, nf), np.tile(cnt, nf), off, shape))
+    ctx.set_option(iac.OPT_AC3D_KERNEL, 1)
+    try:
+        one = mesh_np(gpu_batch(ctx, dev, km, pix, cnt, off[:2], shape))
+    finally:
+        ctx.set_option(iac.OPT_AC3D_KERNEL, 0)
+    assert np.array_equal(m, one * np.uint64(nf))
