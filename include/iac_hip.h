@@ -115,6 +115,10 @@ int iac_ctx_set_option(iac_ctx *ctx, int option, int64_t value);
 /* Updates whose voxel fell outside the mesh since the context was created.
  * The reference writes such updates out of bounds; this path drops them. */
 int iac_dropped_updates(iac_ctx *ctx, uint64_t *count);
+/* Passes of the LDS engine since the context was created, by what took their pairs: [0] the
+ * cell-offset walk, [1] detector strips, [2] region tiles (replays of a captured batch too).
+ * The strips' choice falls on the device, so this waits for the stream. */
+int iac_pair_paths(iac_ctx *ctx, uint64_t passes[3]);
 
 /* ---- host geometry (the reference computes these on the host as well) --------- */
 /* Simulator::GeneratePixelMap, IAC/Simulator.cpp:495-519; pixmap is [size_a][size_b][3]. */

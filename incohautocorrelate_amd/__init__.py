@@ -184,6 +184,12 @@ class Context:
         check(lib().iac_dropped_updates(self._h, C.byref(v)), "iac_dropped_updates")
         return int(v.value)
 
+    def pair_paths(self) -> tuple[int, int, int]:
+        """Passes of the LDS engine so far by the cell walk, by strips and by region tiles."""
+        v = (C.c_uint64 * 3)()
+        check(lib().iac_pair_paths(self._h, v), "iac_pair_paths")
+        return tuple(v)
+
     # ---- 3D AC_uw ------------------------------------------------------------
     def ac3d_sparse(self, hitlist, rot, shape: MeshShape, mesh, interp1: int = NEAREST,
                     interp2: int = NEAREST, double_map: bool = True) -> None:

@@ -80,6 +80,7 @@ SIGNATURES: dict[str, tuple] = {
     "iac_ctx_set_option": (I32, [P, I32, C.c_int64]),
     "iac_ctx_timing": (I32, [P, C.POINTER(C.c_double), C.POINTER(U64), I32]),
     "iac_dropped_updates": (I32, [P, C.POINTER(U64)]),
+    "iac_pair_paths": (I32, [P, C.POINTER(U64)]),
     "iac_generate_pixel_map": (I32, [I32, I32, C.c_float, F3, F3, F3, F3]),
     "iac_calc_kmap": (I32, [F3, U32, F3, F3, F3, F3]),
     "iac_mesh_shape_big": (I32, [F3, I32, C.c_float, C.POINTER(MeshShape)]),

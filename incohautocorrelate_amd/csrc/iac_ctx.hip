@@ -383,6 +383,19 @@ int iac_dropped_updates(iac_ctx *ctx, uint64_t *count)
     return IAC_OK;
 }
 
+int iac_pair_paths(iac_ctx *ctx, uint64_t passes[3])
+{
+    if (!passes) return fail(IAC_ERR_INVALID_ARG, "null passes");
+    IAC_TRY(iac::bind(ctx));
+    unsigned long long v[2] = {0, 0};
+    IAC_HIP(hipMemcpyAsync(v, ctx->d_counters + iac::kPathCounter, sizeof(v), hipMemcpyDeviceToHost, ctx->stream));
+    IAC_HIP(hipStreamSynchronize(ctx->stream));
+    passes[0] = v[0];
+    passes[1] = v[1];
+    passes[2] = ctx->tile_passes;
+    return IAC_OK;
+}
+
 // ---- host geometry ---------------------------------------------------------
 
 // Simulator::GeneratePixelMap, IAC/Simulator.cpp:495-519.  Each element is

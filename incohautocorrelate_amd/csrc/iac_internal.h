@@ -17,7 +17,8 @@ struct iac_ctx {
     int num_cus = 0;
     hipStream_t own_stream = nullptr;
     hipStream_t stream = nullptr;
-    // device counters: [0] dropped updates, [1..7] reserved
+    // device counters: [0] dropped updates, [1] photons with a pixel outside the k-map, from
+    // kPathCounter on the engine's passes by the walk and by strips, the rest reserved
     unsigned long long *d_counters = nullptr;
     // growable scratch arenas (device); each call may reuse them
     void *scratch[4] = {nullptr, nullptr, nullptr, nullptr};
@@ -29,6 +30,7 @@ struct iac_ctx {
     void *pinned[2] = {nullptr, nullptr};
     size_t pinned_bytes[2] = {0, 0};
     hipEvent_t uploaded = nullptr;
+    uint64_t tile_passes = 0;  // passes by region tiles
     // measurement: event pairs around the dominant kernel of each call
     bool timing = false;
     std::vector<hipEvent_t> ev_start, ev_stop;
@@ -62,6 +64,9 @@ namespace iac {
 void set_error(const std::string &msg);
 int fail(int code, const std::string &msg);
 int hip_fail(hipError_t e, const char *what, const char *file, int line);
+
+// ctx->d_counters index of the passes by the walk, then by the strips
+constexpr int kPathCounter = 2;
 
 // Makes ctx->device current on the calling thread.
 int bind(iac_ctx *ctx);

@@ -384,16 +384,19 @@ __global__ void cell_ext_kernel(const float *__restrict__ kmap, uint32_t npix, C
 // cs[f*(ncell+1) + c] = first sorted position of cell c relative to off[f];
 // cs[f*(ncell+1) + ncell] = number of kept records; cmax[f] = records of the
 // frame's fullest cell.  In symmetric mode the frame's self-pair values are added
-// to self[group of f].
+// to self[group of f].  paths: the passes taken by this walk, then by strips.
 template <int KIND, bool ORD>
 __global__ void __launch_bounds__(kBlock)
     cell_sort_kernel(const float4 *__restrict__ rec, const uint64_t *__restrict__ off, CellGeom g,
                      float4 *__restrict__ srec, uint32_t *__restrict__ cs, PairSpec S,
                      const uint32_t *__restrict__ group_off, uint32_t ngroups,
                      unsigned long long *__restrict__ self, uint32_t *__restrict__ wflag,
-                     uint32_t *__restrict__ cmax, const uint32_t *__restrict__ strips)
+                     uint32_t *__restrict__ cmax, const uint32_t *__restrict__ strips,
+                     unsigned long long *__restrict__ paths)
 {
-    if (strips && strips[0]) return;  // the strips take the run
+    const bool by_strips = strips && strips[0];
+    if (blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(paths + (by_strips ? 1 : 0), 1ull);
+    if (by_strips) return;
     __shared__ uint32_t cnt[kMaxCells];
     __shared__ uint32_t part[kBlock];
     __shared__ unsigned long long sred[kBlock / 64];
@@ -2782,20 +2785,20 @@ int enqueue(iac_ctx *ctx, hipStream_t st, const PairRun &R, const Bufs &b, bool 
         if (ordered)
             hipLaunchKernelGGL((cell_sort_kernel<kKindAc3d, true>), dim3(R.nframes), dim3(kBlock), 0, st, R.rec,
                                R.d_frame_off, b.g, b.srec, b.cs, S, b.d_goff, R.ngroups, b.d_self, b.d_flag, cell_max(R, b),
-                               b.nst ? b.st_usable : nullptr);
+                               b.nst ? b.st_usable : nullptr, ctx->d_counters + kPathCounter);
         else
             hipLaunchKernelGGL((cell_sort_kernel<kKindAc3d, false>), dim3(R.nframes), dim3(kBlock), 0, st, R.rec,
                                R.d_frame_off, b.g, b.srec, b.cs, S, b.d_goff, R.ngroups, b.d_self, b.d_flag, cell_max(R, b),
-                               b.nst ? b.st_usable : nullptr);
+                               b.nst ? b.st_usable : nullptr, ctx->d_counters + kPathCounter);
     } else {
         if (ordered)
             hipLaunchKernelGGL((cell_sort_kernel<kKindCq, true>), dim3(R.nframes), dim3(kBlock), 0, st, R.rec,
                                R.d_frame_off, b.g, b.srec, b.cs, S, b.d_goff, R.ngroups, b.d_self, b.d_flag, cell_max(R, b),
-                               b.nst ? b.st_usable : nullptr);
+                               b.nst ? b.st_usable : nullptr, ctx->d_counters + kPathCounter);
         else
             hipLaunchKernelGGL((cell_sort_kernel<kKindCq, false>), dim3(R.nframes), dim3(kBlock), 0, st, R.rec,
                                R.d_frame_off, b.g, b.srec, b.cs, S, b.d_goff, R.ngroups, b.d_self, b.d_flag, cell_max(R, b),
-                               b.nst ? b.st_usable : nullptr);
+                               b.nst ? b.st_usable : nullptr, ctx->d_counters + kPathCounter);
     }
     IAC_HIP(hipGetLastError());
     auto *target = ordered ? reinterpret_cast<unsigned long long *>(R.d_mesh) : b.H;
@@ -3143,6 +3146,7 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
                                (const uint32_t *)nullptr);
             IAC_HIP(hipGetLastError());
         }
+        ctx->tile_passes++;
         *done = true;
         return IAC_OK;
     }

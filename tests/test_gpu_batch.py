@@ -374,3 +374,87 @@ def test_strips_bright_rows(ctx, dev, name):
     finally:
         ctx.set_option(iac.OPT_AC3D_KERNEL, 0)
     assert np.array_equal(m, one * np.uint64(nf))
+
+
+def paths_of(ctx, call):
+    """call()'s result, and the engine passes it took by the walk, by strips and by region tiles."""
+    before = ctx.pair_paths()
+    out = call()
+    return out, tuple(b - a for a, b in zip(before, ctx.pair_paths()))
+
+
+def many_frames(rows, cols, dist, edge, nf=800, mean=1000, seed=1):
+    import incohautocorrelate_amd as iac
+
+    rng = np.random.default_rng(seed)
+    km, _, _, mq = iac.calc_kmap(iac.generate_pixel_map(rows, cols, 75.0, [0, 0, dist], (1, 0, 0), (0, 1, 0)))
+    n = rng.integers(mean - 200, mean + 201, nf)
+    n[3] = 0
+    off = np.concatenate([[0], np.cumsum(n)])
+    pix = rng.integers(0, rows * cols, off[-1])
+    return km, iac.mesh_shape_big(mq, edge), pix, rng.integers(1, 5, off[-1]), off
+
+
+@pytest.mark.parametrize("rows,cols,dist,edge", [(128, 128, 2e5, 63), (60, 200, 1e5, 95), (400, 64, 4e5, 191),
+                                                 (700, 300, 5e5, 255), (512, 512, 5e5, 255)])
+@pytest.mark.parametrize("rotated", [False, True])
+def test_strips_of_several_distances(ctx, dev, rows, cols, dist, edge, rotated):
+    """Runs whose tasks hold two to eight distances (one where the first detector is not rotated),
+    strips along either axis, taken by strips and equal to the tile kernel in every voxel."""
+    import incohautocorrelate_amd as iac
+    from gpu_helpers import gpu_batch
+
+    km, shape, pix, cnt, off = many_frames(rows, cols, dist, edge)
+    rots = W.random_rotations(off.size - 1, 7).astype(np.float32) if rotated else None
+    got, paths = paths_of(ctx, lambda: mesh_np(gpu_batch(ctx, dev, km, pix, cnt, off, shape, rots=rots)))
+    assert paths == (0, 1, 0)
+    ctx.set_option(iac.OPT_AC3D_KERNEL, 1)
+    try:
+        ref = mesh_np(gpu_batch(ctx, dev, km, pix, cnt, off, shape, rots=rots))
+    finally:
+        ctx.set_option(iac.OPT_AC3D_KERNEL, 0)
+    assert np.array_equal(got, ref)
+
+
+def test_strips_bright_rows_take_strips(ctx, dev):
+    """The nine frames of a block still go by strips, in two flushes; the frame that fills the box
+    alone goes by the walk."""
+    from gpu_helpers import gpu_batch
+
+    for name, want in (("frames", (0, 1, 0)), ("frame", (1, 0, 0))):
+        km, shape, pix, cnt, nf = bright_rows(name)
+        off = np.arange(nf + 1) * pix.size
+        call = lambda: gpu_batch(ctx, dev, km, np.tile(pix, nf), np.tile(cnt, nf), off, shape)  # noqa: E731
+        assert paths_of(ctx, call)[1] == want, name
+
+
+def test_captured_strips_follow_the_counts(ctx, dev):
+    """A captured batch on strips whose counts change between replays, with work in between: one
+    too large for the strips sends that replay by the walk, the next goes by strips again."""
+    import torch
+
+    import incohautocorrelate_amd as iac
+    from gpu_helpers import gpu_batch
+
+    km, shape, pix, cnt, off = many_frames(60, 200, 1e5, 95)
+    d_cnt = to_dev(cnt.astype(np.uint16), dev)
+    batch = ctx.ac3d_batch(to_dev(km, dev), to_dev(pix.astype(np.uint32), dev), d_cnt,
+                           to_dev(off.astype(np.uint64), dev), int(off[-1]), shape)
+    m = torch.zeros(shape.size_ab ** 2 * shape.size_c, dtype=torch.int64, device=dev)
+    try:
+        batch.capture(m, zero_mesh=True)
+        for top, want in ((4, (0, 1, 0)), (200, (1, 0, 0)), (4, (0, 1, 0)), (129, (0, 1, 0)), (130, (1, 0, 0))):
+            c = cnt.copy()
+            c[c.size // 3] = top
+            d_cnt.copy_(to_dev(c.astype(np.uint16), dev))
+            torch.cuda.synchronize()
+            got, paths = paths_of(ctx, lambda: batch.launch(m, zero_mesh=True) or mesh_np(m))
+            assert paths == want, top
+            ctx.set_option(iac.OPT_AC3D_KERNEL, 1)
+            try:
+                ref = mesh_np(gpu_batch(ctx, dev, km, pix, c, off, shape))
+            finally:
+                ctx.set_option(iac.OPT_AC3D_KERNEL, 0)
+            assert np.array_equal(got, ref), top
+    finally:
+        batch.destroy()
