@@ -85,15 +85,19 @@ __device__ __forceinline__ unsigned long long fixed_u64(double x)
 }
 
 // What one small voxel of value val_in at the rotated (q0, q1, q2) adds (kernel.cl:262-341):
-// add(fs, ms, ss, value) once, or per corner.
-template <bool kLinear, class Add>
+// add(fs, ms, ss, value) once, or per corner.  kFinite: no q is NaN (a NaN's voxel is index 0, what
+// its conversion to an integer gives).
+template <bool kLinear, bool kFinite, class Add>
 __device__ __forceinline__ void merge_voxel(float q0, float q1, float q2, double val_in, double w, double mult,
                                             int cab, Add add)
 {
     if (!kLinear) {
         // roundf(q) for |q| < 2^22: half away from zero is x + copysign(0.49999997f, x), truncated
-        auto round_away = [](float x) { return (int)(x + copysignf(0.49999997f, x)); };
-        add(round_away(q0) + cab, round_away(q1) + cab, round_away(q2) + cab, fixed_u64((val_in * w) * mult));
+        auto voxel = [cab](float x) {
+            const int n = (int)(x + copysignf(0.49999997f, x)) + cab;
+            return kFinite || x == x ? n : 0;
+        };
+        add(voxel(q0), voxel(q1), voxel(q2), fixed_u64((val_in * w) * mult));
         return;
     }
     const double sfs = (double)(1.0f - (q0 - floorf(q0)));
@@ -242,7 +246,7 @@ __global__ void __launch_bounds__(256)
                     const float q0 = (slope[0] * xf + u[0]) + v[0];
                     const float q1 = (slope[1] * xf + u[1]) + v[1];
                     const float q2 = (slope[2] * xf + u[2]) + v[2];
-                    merge_voxel<kLinear>(q0, q1, q2, val[j], w, mult, cab,
+                    merge_voxel<kLinear, true>(q0, q1, q2, val[j], w, mult, cab,
                                          [&](int fs, int ms, int ss, unsigned long long x) {
                                              const int lx = fs - b0, ly = ms - b1, lz = ss - b2;
                                              if ((unsigned)lx < (unsigned)e0_ && (unsigned)ly < (unsigned)e1_ &&
@@ -308,7 +312,7 @@ __global__ void __launch_bounds__(256)
         const float q0 = R[0] * qi0 + R[1] * qi1 + R[2] * qi2;
         const float q1 = R[3] * qi0 + R[4] * qi1 + R[5] * qi2;
         const float q2 = R[6] * qi0 + R[7] * qi1 + R[8] * qi2;
-        merge_voxel<kLinear>(q0, q1, q2, val_in, (double)R[9], mult, cab,
+        merge_voxel<kLinear, false>(q0, q1, q2, val_in, (double)R[9], mult, cab,
                              [&](int fs, int ms, int ss, unsigned long long v) {
                                  if ((unsigned)fs < (unsigned)sab && (unsigned)ms < (unsigned)sab &&
                                      (unsigned)ss < (unsigned)sab) {

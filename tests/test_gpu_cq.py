@@ -416,3 +416,31 @@ def test_cq_region_tiles_vs_engine(dev, rows, cols, dist, edge, axes, interp):
     finally:
         a.close()
         b.close()
+
+
+@pytest.mark.parametrize("nev", [1, 300])
+def test_merge_nan_rotation(ctx, dev, nev):
+    """A matrix with NaN entries bins a coordinate that is NaN at voxel 0, beside rotations or alone,
+    few events (scattered adds) and many (bricks for the others)."""
+    import torch
+
+    import incohautocorrelate_amd as iac
+
+    sab, sc = 33, 3
+    s = iac.MeshShape(k_a=0, k_b=1, k_c=2, size_ab=sab, size_c=sc)
+    s.voxel_per_dq, s.max_q = 1, 1.0
+    rots = W.random_rotations(nev, 3)
+    rots[0] = np.array([np.nan, np.nan, np.nan, 0, 1, 0, 0, 0, 1])
+    rw = np.concatenate([rots, np.ones((nev, 1))], 1).astype(np.float32)
+    small = np.random.default_rng(nev).random((sc, sab, sab))
+    mult = 1e4
+    ref, drop = np.zeros(sab ** 3, np.uint64), 0
+    if nev > 1:
+        ref, drop = O.merge_cq(small.ravel(), s, rw[1:], 0, mult)
+    box = ref.reshape(sab, sab, sab)
+    box[16 - 1:16 + 2, :, 0] += np.floor(small * mult).astype(np.uint64).sum(axis=2)
+    big = _zeros(sab ** 3, dev)
+    before = ctx.dropped()
+    ctx.merge_cq(torch.from_numpy(small.ravel()).to(dev), s, to_dev(rw, dev), 0, mult, big)
+    assert np.array_equal(mesh_np(big), ref)
+    assert ctx.dropped() - before == drop
