@@ -3039,6 +3039,8 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
     const PairSpec &S = R.spec;
     const bool ordered = R.ordered;
     if (!default_options(ctx)) return IAC_OK;
+    // what the walk refuses (pairs_run, check_chunks) stays refused
+    if (R.n_total >= (1ull << 32) || R.npix >= (1u << 28)) return IAC_OK;
     // round_away and the boxes' 24-bit products need |q vox| < 2^22
     if (!(std::sqrt((double)S.P.cut_sq) * S.P.vox < 4194304.0) || R.nframes == 0) return IAC_OK;
     hipStream_t st = ctx->stream;

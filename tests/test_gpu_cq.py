@@ -444,3 +444,20 @@ def test_merge_nan_rotation(ctx, dev, nev):
     ctx.merge_cq(torch.from_numpy(small.ravel()).to(dev), s, to_dev(rw, dev), 0, mult, big)
     assert np.array_equal(mesh_np(big), ref)
     assert ctx.dropped() - before == drop
+
+
+def test_cq_frame_limit(ctx, dev):
+    """A frame of 2^28 pixels is refused, whatever its pixels hold."""
+    import torch
+
+    import incohautocorrelate_amd as iac
+
+    s = iac.MeshShape(k_a=0, k_b=1, k_c=2, size_ab=5, size_c=5)
+    s.voxel_per_dq, s.max_q = 1, 1.0
+    npix = 1 << 28
+    img = torch.zeros(npix, device=dev)
+    img[:40] = 1.0
+    mesh = _zeros(125, dev)
+    with pytest.raises(iac.IACError, match="2\\^28"):
+        ctx.cq_small(torch.zeros((npix, 3), device=dev), img, s, mesh, 0, 1.0)
+    assert int(mesh.sum()) == 0
