@@ -458,3 +458,27 @@ def test_captured_strips_follow_the_counts(ctx, dev):
             assert np.array_equal(got, ref), top
     finally:
         batch.destroy()
+
+
+def test_batch_prepared_on_strips_follows_options_set_later(ctx, dev):
+    """An engine option set between a batch's creation and its launch names the walk that takes it,
+    and clearing it brings the strips back; the same mesh each time."""
+    import torch
+
+    import incohautocorrelate_amd as iac
+
+    km, shape, pix, cnt, off = many_frames(60, 200, 1e5, 95)
+    batch = ctx.ac3d_batch(to_dev(km, dev), to_dev(pix.astype(np.uint32), dev), to_dev(cnt.astype(np.uint16), dev),
+                           to_dev(off.astype(np.uint64), dev), int(off[-1]), shape)
+    m = torch.zeros(shape.size_ab ** 2 * shape.size_c, dtype=torch.int64, device=dev)
+    ref = None
+    try:
+        for mode, want in ((0, (0, 1, 0)), (1, (1, 0, 0)), (2, (1, 0, 0)), (0, (0, 1, 0))):
+            ctx.set_option(iac.OPT_PAIR_MODE, mode)
+            got, paths = paths_of(ctx, lambda: batch.launch(m, zero_mesh=True) or mesh_np(m))
+            ref = got if ref is None else ref
+            assert paths == want, mode
+            assert np.array_equal(got, ref), mode
+    finally:
+        ctx.set_option(iac.OPT_PAIR_MODE, 0)
+        batch.destroy()
