@@ -289,6 +289,14 @@ __global__ void init_cell_ext_kernel(uint32_t *ext, int ncell)
         }
 }
 
+// the k-map's extents start empty; what dense_scan_kernel counts starts at none, its flags at 1
+__global__ void cq_begin_kernel(uint32_t *ext, unsigned long long *kept, uint32_t *plain)
+{
+    if (threadIdx.x < 6) ext[threadIdx.x] = threadIdx.x < 3 ? 0xffffffffu : 0u;
+    if (threadIdx.x < 2) plain[threadIdx.x] = 1u;
+    if (threadIdx.x == 0) kept[0] = 0ull;
+}
+
 // min/max of each k component: ext[0..2] min keys, ext[3..5] max keys, reduced over the block: all
 // blocks' atomics fall on these six words (one per wave took 20 us for 16,384 pixels, so 2 us)
 __global__ void __launch_bounds__(256) kext_kernel(const float *__restrict__ kmap, uint32_t npix, uint32_t *ext)
@@ -1332,52 +1340,63 @@ __device__ __forceinline__ uint32_t tile_key(const CellGeom &g, int side, float 
     return (uint32_t)((cv * g.ncu + cu) * side + sv) * (uint32_t)side + (uint32_t)su;
 }
 
-// Counts of the frames' nonzero pixels per key (cs, zeroed by the caller), the groups' self
-// values (symmetric modes), the number of kept records, and the run's flags: plain[0] is cleared by
-// any record that could make a pair negative, NaN or 2^32 or more, plain[1] by one that could
-// make it negative, NaN or 2^62 or more.
-// Grid: ns blocks per frame.
+// The nonzero values of all frames, counted into kept, and the run's flags: plain[0] is cleared by
+// any value that could make a pair negative, NaN or 2^32 or more, plain[1] by one that could
+// make it negative, NaN or 2^62 or more.  Bound: one read of the frames.
+__global__ void __launch_bounds__(kBlock)
+    dense_scan_kernel(const float *__restrict__ frames, uint64_t n, double mult, unsigned long long *__restrict__ kept,
+                      uint32_t *__restrict__ plain)
+{
+    __shared__ unsigned long long kred[kBlock / 64];
+    unsigned long long c = 0;
+    bool ok = true, wide = 1e-37 * mult < 0.99;  // a product below 1e-37 adds nothing either way
+    const uint64_t step = (uint64_t)gridDim.x * kBlock;
+#pragma unroll 4
+    for (uint64_t p = (uint64_t)blockIdx.x * kBlock + threadIdx.x; p < n; p += step) {
+        const float I = frames[p];
+        const double most = (double)(I * I) * mult;
+        c += I != 0.0f ? 1u : 0u;
+        ok = ok && (I == 0.0f || most < 4294967296.0);
+        wide = wide && (I == 0.0f || (I > 0.0f && most < 0x1p62));
+    }
+    if (!ok || !wide) plain[0] = 0u;
+    if (!wide) plain[1] = 0u;
+    for (int o = 32; o > 0; o >>= 1) c += __shfl_down(c, o, 64);
+    if ((threadIdx.x & 63) == 0) kred[threadIdx.x >> 6] = c;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        c = 0;
+        for (int w = 0; w < kBlock / 64; w++) c += kred[w];
+        if (c) atomicAdd(kept, c);
+    }
+}
+
+// Counts of the frames' nonzero pixels per key (cs, zeroed by the caller) and the groups' self
+// values (symmetric modes).  Grid: ns blocks per frame.
 template <bool ORD>
 __global__ void __launch_bounds__(kBlock)
     tile_count_kernel(const float *__restrict__ kmap, const float *__restrict__ frames, uint32_t npix, uint32_t ns,
                       CellGeom g, int side, PairSpec S, const uint32_t *__restrict__ group_off, uint32_t ngroups,
-                      uint32_t *__restrict__ cs, unsigned long long *__restrict__ self,
-                      uint32_t *__restrict__ plain, unsigned long long *__restrict__ kept)
+                      uint32_t *__restrict__ cs, unsigned long long *__restrict__ self)
 {
-    __shared__ unsigned long long sred[kBlock / 64], kred[kBlock / 64];
+    __shared__ unsigned long long sred[kBlock / 64];
     const uint32_t f = blockIdx.x / ns;
     const size_t nkey = (size_t)g.ncu * g.ncv * side * side;
     uint32_t *csf = cs + f * (nkey + 1);
-    unsigned long long sv = 0, n = 0;
-    bool ok = true, wide = 1e-37 * S.mult < 0.99;  // a product below 1e-37 adds nothing either way
+    unsigned long long sv = 0;
     for (uint32_t p = (blockIdx.x - f * ns) * kBlock + threadIdx.x; p < npix; p += ns * kBlock) {
         const float I = frames[(size_t)f * npix + p];
         if (I == 0.0f) continue;
         atomicAdd(csf + tile_key(g, side, kmap[3 * (size_t)p + g.au], kmap[3 * (size_t)p + g.av]), 1u);
-        n++;
         if (!ORD) sv += self_value<kKindCq>(S, I);
-        const double most = (double)(I * I) * S.mult;
-        ok = ok && most < 4294967296.0;
-        wide = wide && I > 0.0f && most < 0x1p62;
     }
-    if (!ok || !wide) plain[0] = 0u;
-    if (!wide) plain[1] = 0u;
-    for (int o = 32; o > 0; o >>= 1) {
-        sv += __shfl_down(sv, o, 64);
-        n += __shfl_down(n, o, 64);
-    }
-    if ((threadIdx.x & 63) == 0) {
-        sred[threadIdx.x >> 6] = sv;
-        kred[threadIdx.x >> 6] = n;
-    }
+    if (ORD) return;
+    for (int o = 32; o > 0; o >>= 1) sv += __shfl_down(sv, o, 64);
+    if ((threadIdx.x & 63) == 0) sred[threadIdx.x >> 6] = sv;
     __syncthreads();
     if (threadIdx.x == 0) {
-        sv = n = 0;
-        for (int w = 0; w < kBlock / 64; w++) {
-            sv += sred[w];
-            n += kred[w];
-        }
-        if (n) atomicAdd(kept, n);
+        sv = 0;
+        for (int w = 0; w < kBlock / 64; w++) sv += sred[w];
         if (sv) {
             uint32_t lo = 0, hi = ngroups;  // group of f: largest gi with group_off[gi] <= f
             while (hi - lo > 1) {
@@ -2290,6 +2309,7 @@ iac_pair_plan *find_plan(iac_ctx *ctx, const float *kmap, uint32_t npix, int cel
     return nullptr;
 }
 
+constexpr size_t kMaxPlans = 20;   // cached plans of a context
 constexpr int kRegionTiles = -1;   // iac_pair_plan::region of a region-tile plan
 constexpr int kRegionStrips = -2;  // and less: of a strip plan, its distances per task with it
 constexpr size_t kStripBox2 = 79 * 1024;  // LDS bytes of a strip box: two blocks per CU
@@ -2306,7 +2326,9 @@ void build_tiles(iac_pair_plan &pl, bool ordered)
     const long cap = pl.box_cap;
     const double maxq = std::sqrt((double)S.P.cut_sq);
     size_t boxed = 0;
+    const size_t all = ordered ? (size_t)nc * nc : (size_t)nc * (nc + 1) / 2;
     for (int ci = 0; ci < nc; ci++) {
+        if (pl.tiles.size() - boxed > all / 32) break;  // no longer to be made good
         const uint32_t *ea = &pl.cell_ext[6 * (size_t)ci];
         if (ea[0] == 0xffffffffu) continue;  // no pixel there
         for (int cj = ordered ? 0 : ci; cj < nc; cj++) {
@@ -2360,6 +2382,7 @@ void build_tiles(iac_pair_plan &pl, bool ordered)
         }
     }
     pl.tiles_fit = !pl.tiles.empty() && boxed >= pl.tiles.size() - pl.tiles.size() / 32;
+    if (!pl.tiles_fit) std::vector<TileTask>().swap(pl.tiles);
 }
 
 // One task per `per` strip distances, with the box of all of them.
@@ -2407,20 +2430,31 @@ int plan_read(iac_ctx *ctx, size_t more_bytes, PlanRead *out)
     return IAC_OK;
 }
 
+// Enqueues the extents of the k-map, d_ext initialised, and their copy to read.kext.
+int kmap_extents_enqueue(hipStream_t st, const float *d_kmap, uint32_t npix, uint32_t *d_ext, const PlanRead &read)
+{
+    const unsigned eb = std::max(1u, std::min<unsigned>(64, (npix + 1023) / 1024));
+    hipLaunchKernelGGL(kext_kernel, dim3(eb), dim3(256), 0, st, d_kmap, npix, d_ext);
+    IAC_HIP(hipGetLastError());
+    IAC_HIP(hipMemcpyAsync(read.kext, d_ext, 6 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    return IAC_OK;
+}
+void kmap_extents_read(const PlanRead &read, float kmin[3], float ext3[3])
+{
+    for (int d = 0; d < 3; d++) {
+        kmin[d] = unkey(read.kext[d]);
+        ext3[d] = unkey(read.kext[3 + d]) - kmin[d];
+    }
+}
+
 // Extents of the k-map (one host round trip).
 int kmap_extents(hipStream_t st, const float *d_kmap, uint32_t npix, uint32_t *d_ext, const PlanRead &read,
                  float kmin[3], float ext3[3])
 {
     hipLaunchKernelGGL(init_cell_ext_kernel, dim3(1), dim3(64), 0, st, d_ext, 1);
-    const unsigned eb = std::max(1u, std::min<unsigned>(64, (npix + 1023) / 1024));
-    hipLaunchKernelGGL(kext_kernel, dim3(eb), dim3(256), 0, st, d_kmap, npix, d_ext);
-    IAC_HIP(hipGetLastError());
-    IAC_HIP(hipMemcpyAsync(read.kext, d_ext, 6 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    IAC_TRY(kmap_extents_enqueue(st, d_kmap, npix, d_ext, read));
     IAC_HIP(hipStreamSynchronize(st));
-    for (int d = 0; d < 3; d++) {
-        kmin[d] = unkey(read.kext[d]);
-        ext3[d] = unkey(read.kext[3 + d]) - kmin[d];
-    }
+    kmap_extents_read(read, kmin, ext3);
     return IAC_OK;
 }
 
@@ -2548,8 +2582,9 @@ int plan_of(iac_ctx *ctx, const PairRun &R, int cell_vox, int box_cap, int regio
     iac_pair_plan *pl = find_plan(ctx, R.d_kmap, R.npix, cell_vox, box_cap, region, S);
     if (pl && (std::memcmp(&pl->g, &g, sizeof(g)) != 0 || pl->cell_ext != cext)) pl = nullptr;
     if (!pl) {
-        // reuse the oldest unpinned slot beyond eight cached plans
-        if (ctx->pair_plans.size() >= 8) {
+        // reuse the oldest unpinned slot beyond the cached plans; a geometry holds at most five (the
+        // walk's and the strips', or the walk's and four region sides that do not fit)
+        if (ctx->pair_plans.size() >= kMaxPlans) {
             for (auto it = ctx->pair_plans.begin(); it != ctx->pair_plans.end(); ++it) {
                 if ((*it)->pins > 0) continue;
                 if ((*it)->d_tasks) IAC_HIP(hipFree((*it)->d_tasks));
@@ -3052,24 +3087,74 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
     // round_away and the boxes' 24-bit products need |q vox| < 2^22
     if (!(std::sqrt((double)S.P.cut_sq) * S.P.vox < 4194304.0) || R.nframes == 0) return IAC_OK;
     hipStream_t st = ctx->stream;
+    const uint32_t ns = std::min<uint32_t>(256, (R.npix + kBlock - 1) / kBlock);  // sort blocks per frame
+    if ((uint64_t)ns * R.nframes > 0x7fffffffull) return IAC_OK;
+    // the k-map's extents | kept, flags | the cells' extents, a grid for each side
+    constexpr size_t nsides = sizeof(kTileSides) / sizeof(kTileSides[0]);
     void *ext = nullptr;
-    IAC_TRY(scratch(ctx, 3, (6 + 6 * (size_t)(kMaxCells + kMaxStrips)) * sizeof(uint32_t), &ext));
+    IAC_TRY(scratch(ctx, 3, (12 + 6 * (size_t)(nsides * kMaxCells)) * sizeof(uint32_t), &ext));
     uint32_t *d_ext = static_cast<uint32_t *>(ext);
+    auto *d_kept = reinterpret_cast<unsigned long long *>(d_ext + 8);
+    auto *d_plain = reinterpret_cast<uint32_t *>(d_kept + 1);
+    uint32_t *d_cells = d_ext + 12;
     float kmin[3], ext3[3];
     PlanRead read;
     IAC_TRY(plan_read(ctx, 2 * sizeof(uint64_t), &read));
-    IAC_TRY(kmap_extents(st, R.d_kmap, R.npix, d_ext, read, kmin, ext3));
+    hipLaunchKernelGGL(cq_begin_kernel, dim3(1), dim3(64), 0, st, d_ext, d_kept, d_plain);
+    hipLaunchKernelGGL(dense_scan_kernel, dim3((unsigned)std::min<uint64_t>(2048, (R.n_total + 4 * kBlock - 1) / (4 * kBlock))),
+                       dim3(kBlock), 0, st, d_frames, R.n_total, S.mult, d_kept, d_plain);
+    IAC_TRY(kmap_extents_enqueue(st, R.d_kmap, R.npix, d_ext, read));
+    IAC_HIP(hipMemcpyAsync(read.more, d_kept, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, st));
+    IAC_HIP(hipStreamSynchronize(st));
+    kmap_extents_read(read, kmin, ext3);
+    const uint64_t kept = read.more[0];
+    const uint32_t *flags = reinterpret_cast<const uint32_t *>(read.more + 1);
+    const bool wide = !flags[0];
+    if (!flags[1]) return IAC_OK;  // negative values: the engine's pairs test each
     const int box_cap = ordered ? kBoxMax : kBoxSmall;
     const size_t nvox = (size_t)S.P.sab * S.P.sab * S.P.sc;
-    const uint32_t ns = std::min<uint32_t>(256, (R.npix + kBlock - 1) / kBlock);  // sort blocks per frame
-    if ((uint64_t)ns * R.nframes > 0x7fffffffull) return IAC_OK;
-    for (size_t k = 0; k < sizeof(kTileSides) / sizeof(kTileSides[0]); k++) {
-        const int side = kTileSides[k];
-        const CellGeom g = cell_grid(kmin, ext3, S.P.vox, side);
+    // the sides of enough tasks whose regions hold enough records
+    struct Side {
+        int side;
+        CellGeom g;
+    } sides[nsides];
+    size_t n = 0;
+    for (size_t k = 0; k < nsides; k++) {
+        const CellGeom g = cell_grid(kmin, ext3, S.P.vox, kTileSides[k]);
         const int nc = g.ncu * g.ncv;
         const double ntask = ordered ? (double)nc * nc : 0.5 * nc * (nc + 1.0);
-        if (ntask > kMaxGridBlocks) return IAC_OK;
-        if (ntask * R.ngroups < kTileTasks && k + 1 < sizeof(kTileSides) / sizeof(kTileSides[0])) continue;
+        if (ntask > kMaxGridBlocks || (double)kept < kTileRecords * (double)R.nframes * nc) break;
+        if (ntask * R.ngroups < kTileTasks && k + 1 < nsides) continue;
+        sides[n++] = Side{kTileSides[k], g};
+    }
+    if (n == 0) return IAC_OK;
+    // Boxes of regions this size fit wherever in the mesh they lie: the plan can wait for the sort's
+    // read-back.  Otherwise (a detector near or tilted) the sides' extents come first, in one go, so
+    // that nothing is sorted for a side that does not fit.
+    auto fits = [&](const CellGeom &g) {
+        const int third = 3 - g.au - g.av, more = ordered ? 3 : 2;
+        const double u = S.P.vox / (double)g.inv_wu, v = S.P.vox / (double)g.inv_wv, z = ext3[third] * (double)S.P.vox;
+        return (std::floor(2 * u) + more) * (std::floor(2 * v) + more) * (std::floor(2 * z) + more) <= box_cap;
+    };
+    size_t first = 0;
+    iac_pair_plan *pl = nullptr;
+    if (!fits(sides[0].g)) {
+        const size_t each = 6 * (size_t)kMaxCells;
+        IAC_TRY(plan_read(ctx, nsides * each * sizeof(uint32_t), &read));
+        uint32_t *h_cells = reinterpret_cast<uint32_t *>(read.more);
+        for (size_t k = 0; k < n; k++)
+            IAC_TRY(cell_extents(st, R.d_kmap, R.npix, sides[k].g, d_cells + k * each, h_cells + k * each));
+        IAC_HIP(hipStreamSynchronize(st));
+        for (first = 0; first < n; first++) {
+            IAC_TRY(plan_of(ctx, R, sides[first].side, box_cap, kRegionTiles, sides[first].g, h_cells + first * each, &pl));
+            if (pl->tiles_fit) break;
+        }
+    }
+    for (size_t k = first; k < n; k++) {
+        const int side = sides[k].side;
+        const CellGeom &g = sides[k].g;
+        const int nc = g.ncu * g.ncv;
+        const double ntask = ordered ? (double)nc * nc : 0.5 * nc * (nc + 1.0);
         // chunks: a group's frames in as many blocks as fill the chip
         const uint32_t split = (uint32_t)std::max(1.0, std::ceil(kTileTasks / (ntask * R.ngroups)));
         std::vector<Chunk> chunks;
@@ -3080,13 +3165,13 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
                                        f0 + (uint32_t)((uint64_t)n * (c + 1) / parts), gi});
         }
         auto up = [](size_t x) { return (x + 255) / 256 * 256; };
-        // records | region starts | cursors (slot 1); half meshes | group offsets | self, kept, flag | chunks (slot 2)
+        // records | region starts | cursors (slot 1); half meshes | group offsets | self | chunks (slot 2)
         const size_t nkey = (size_t)nc * side * side;
         const size_t brec = up((size_t)R.npix * R.nframes * sizeof(float4)),
                      bcs = up(R.nframes * (nkey + 1) * sizeof(uint32_t)),
                      bcur = up(R.nframes * nkey * sizeof(uint32_t));
         const size_t bh = ordered ? 0 : up(nvox * R.ngroups * sizeof(unsigned long long)),
-                     bg = up((R.ngroups + 1) * sizeof(uint32_t)), bs = up((R.ngroups + 2) * sizeof(unsigned long long));
+                     bg = up((R.ngroups + 1) * sizeof(uint32_t)), bs = up(R.ngroups * sizeof(unsigned long long));
         void *s1 = nullptr, *s2 = nullptr;
         IAC_TRY(scratch(ctx, 1, brec + bcs + bcur, &s1));
         IAC_TRY(scratch(ctx, 2, bh + bg + bs + chunks.size() * sizeof(Chunk) + 256, &s2));
@@ -3097,36 +3182,30 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
         auto *H = reinterpret_cast<unsigned long long *>(p2);
         auto *d_goff = reinterpret_cast<uint32_t *>(p2 + bh);
         auto *d_self = reinterpret_cast<unsigned long long *>(p2 + bh + bg);
-        auto *d_kept = d_self + R.ngroups;
-        auto *d_plain = reinterpret_cast<uint32_t *>(d_kept + 1);
         auto *d_chunks = reinterpret_cast<Chunk *>(p2 + bh + bg + bs);
         IAC_TRY(upload_tables(ctx, st, R, chunks, {}, d_goff, d_chunks, nullptr));
-        IAC_TRY(cell_extents(st, R.d_kmap, R.npix, g, d_ext + 6, read.cells));
+        if (!pl) IAC_TRY(cell_extents(st, R.d_kmap, R.npix, g, d_cells, read.cells));
         auto blocks = [](size_t n) { return (unsigned)std::max<size_t>(1, std::min<size_t>(4096, (n + 255) / 256)); };
         const size_t ncs = R.nframes * (nkey + 1);
         hipLaunchKernelGGL(fill_u32_kernel, dim3(blocks(ncs)), dim3(256), 0, st, cs, 0u, ncs);
-        hipLaunchKernelGGL(fill_u64_kernel, dim3(blocks(R.ngroups + 1)), dim3(256), 0, st, d_self, (size_t)R.ngroups + 1);
-        hipLaunchKernelGGL(fill_u32_kernel, dim3(1), dim3(64), 0, st, d_plain, 1u, (size_t)2);
+        hipLaunchKernelGGL(fill_u64_kernel, dim3(blocks(R.ngroups)), dim3(256), 0, st, d_self, (size_t)R.ngroups);
         const unsigned sblocks = ns * R.nframes;
         hipLaunchKernelGGL(ordered ? tile_count_kernel<true> : tile_count_kernel<false>, dim3(sblocks), dim3(kBlock), 0,
-                           st, R.d_kmap, d_frames, R.npix, ns, g, side, S, d_goff, R.ngroups, cs, d_self, d_plain,
-                           d_kept);
+                           st, R.d_kmap, d_frames, R.npix, ns, g, side, S, d_goff, R.ngroups, cs, d_self);
         hipLaunchKernelGGL(tile_scan_kernel, dim3(R.nframes), dim3(1024), 0, st, cs, cursor, (uint32_t)nkey);
         hipLaunchKernelGGL(tile_scatter_kernel, dim3(sblocks), dim3(kBlock), 0, st, R.d_kmap, d_frames, R.npix, ns, g,
                            side, S.ka, S.kb, S.kc, cursor, srec);
         if (!ordered)
             hipLaunchKernelGGL(fill_u64_kernel, dim3(blocks(nvox * R.ngroups)), dim3(256), 0, st, H, nvox * R.ngroups);
         IAC_HIP(hipGetLastError());
-        IAC_HIP(hipMemcpyAsync(read.more, d_kept, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, st));
-        IAC_HIP(hipStreamSynchronize(st));
-        const uint64_t kept = read.more[0];
-        const uint32_t *flags = reinterpret_cast<const uint32_t *>(read.more + 1);
-        const bool wide = !flags[0];
-        if (!flags[1]) return IAC_OK;  // negative values: the engine's pairs test each
-        if ((double)kept < kTileRecords * (double)R.nframes * nc) return IAC_OK;  // sparse frames
-        iac_pair_plan *pl = nullptr;
-        IAC_TRY(plan_of(ctx, R, side, box_cap, kRegionTiles, g, read.cells, &pl));
-        if (!pl->tiles_fit) continue;
+        if (!pl) {
+            IAC_HIP(hipStreamSynchronize(st));
+            IAC_TRY(plan_of(ctx, R, side, box_cap, kRegionTiles, g, read.cells, &pl));
+            if (!pl->tiles_fit) {  // boxes outside the mesh
+                pl = nullptr;
+                continue;
+            }
+        }
         const bool by_parts = !ordered && !wide && (double)kept >= kPartRecords * (double)R.nframes * (double)nkey;
         auto *target = ordered ? reinterpret_cast<unsigned long long *>(R.d_mesh) : H;
         const uint32_t ntasks = (uint32_t)pl->tiles.size(), nchunks = (uint32_t)chunks.size();

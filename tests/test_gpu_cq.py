@@ -461,3 +461,58 @@ def test_cq_frame_limit(ctx, dev):
     with pytest.raises(iac.IACError, match="2\\^28"):
         ctx.cq_small(torch.zeros((npix, 3), device=dev), img, s, mesh, 0, 1.0)
     assert int(mesh.sum()) == 0
+
+
+def test_cq_runs_the_tiles_leave_cost_no_scratch(dev):
+    """Small frames on a fine mesh hold too few records per region for the tiles: the walk's
+    buffers (about 130 MB here) are all that the call keeps, no key tables of the regions (1.1 GB)."""
+    import torch
+
+    import incohautocorrelate_amd as iac
+
+    nf = 2000
+    _, km, mq = W.detector(32)
+    s = iac.mesh_shape_small_cofq(mq, 511)
+    frames = to_dev(W.gamma_frames(32 * 32, nf, 1.0, 0.5, seed=4), dev)
+    d_km, mesh = to_dev(km, dev), _zeros(s.size_ab ** 2 * s.size_c, dev)
+    c = iac.Context(0)
+    try:
+        c.cq_small(d_km, frames[0], s, mesh, 0, 1e6)
+        torch.cuda.synchronize()
+        free = torch.cuda.mem_get_info()[0]
+        c.cq_dense_frames(d_km, frames, [0, nf], s, mesh, 0, 1e6)
+        c.sync()
+        assert free - torch.cuda.mem_get_info()[0] < 400e6
+        assert c.pair_paths() == (2, 0, 0)
+    finally:
+        c.close()
+
+
+@pytest.mark.parametrize("rows,cols,dist,edge,tiles", [(128, 128, 5e5, 63, "NL"), (110, 100, 8e3, 127, "NL"),
+                                                       (160, 150, 4e3, 191, "NL"), (100, 110, 2e3, 191, "L"),
+                                                       (64, 48, 2e3, 255, "")])
+@pytest.mark.parametrize("interp", [0, 1])
+def test_cq_near_detectors_find_a_side(dev, rows, cols, dist, edge, tiles, interp):
+    """Detectors so near that regions are deep along the beam: the tiles take a smaller side, or
+    leave the run to the walk (tiles: whether they take nearest and linear runs); equal meshes
+    either way, also on the second call (cached plans)."""
+    import torch
+
+    import incohautocorrelate_amd as iac
+
+    km, _, _, mq = iac.calc_kmap(iac.generate_pixel_map(rows, cols, 75.0, [0, 0, dist], (1, 0, 0), (0, 1, 0)))
+    s = iac.mesh_shape_small_cofq(mq, edge)
+    img = to_dev(W.gamma_frames(rows * cols, 1, 1.0, 0.5, seed=6)[0], dev)
+    a, b = iac.Context(0), iac.Context(0)
+    try:
+        b.set_option(iac.OPT_PAIR_MODE, 2)
+        got = []
+        for c in (a, a, b):
+            m = _zeros(s.size_ab ** 2 * s.size_c, dev)
+            c.cq_small(to_dev(km, dev), img, s, m, interp, 1e6)
+            got.append(m)
+        assert torch.equal(got[0], got[2]) and torch.equal(got[1], got[2])
+        assert a.pair_paths() == ((0, 0, 2) if "NL"[interp] in tiles else (2, 0, 0))
+    finally:
+        a.close()
+        b.close()
