@@ -111,6 +111,9 @@ int iac_ctx_timing(iac_ctx *ctx, double *ms, uint64_t *launches, int reset);
 #define IAC_OPT_LAP_GROUPS 10 /* LAP finder: two-frame groups a tile's waves take in a row of the block order
                                  (the XCD's L2 keeps the tile's mask, offset and gain rows for them),
                                  0 = default (16) */
+#define IAC_OPT_BUFFER_LIMIT 11 /* bytes of one work buffer (a scratch arena, a prepared batch) at most, as if the
+                                   device had no more; 0 = what it has.  The engine's faster paths need more
+                                   memory than its walk, which takes the run where theirs is short */
 int iac_ctx_set_option(iac_ctx *ctx, int option, int64_t value);
 /* Updates whose voxel fell outside the mesh since the context was created.
  * The reference writes such updates out of bounds; this path drops them. */

@@ -36,6 +36,23 @@ int bind(iac_ctx *ctx)
     return IAC_OK;
 }
 
+hipError_t alloc_buffer(iac_ctx *ctx, size_t bytes, void **out)
+{
+    *out = nullptr;
+    if (ctx->buffer_limit && bytes > ctx->buffer_limit) return hipErrorOutOfMemory;
+    const hipError_t e = hipMalloc(out, bytes);
+    if (e == hipErrorOutOfMemory) (void)hipGetLastError();
+    return e;
+}
+
+int scratch_if(iac_ctx *ctx, int slot, size_t bytes, void **out)
+{
+    const int rc = scratch(ctx, slot, bytes, out);
+    if (rc != IAC_ERR_OOM) return rc;
+    *out = nullptr;
+    return IAC_OK;
+}
+
 int scratch(iac_ctx *ctx, int slot, size_t bytes, void **out)
 {
     if (slot < 0 || slot >= 4) return fail(IAC_ERR_INVALID_ARG, "bad scratch slot");
@@ -48,7 +65,8 @@ int scratch(iac_ctx *ctx, int slot, size_t bytes, void **out)
             ctx->scratch_bytes[slot] = 0;
         }
         size_t want = bytes + bytes / 4;  // grow with headroom
-        IAC_HIP(hipMalloc(&ctx->scratch[slot], want));
+        if (ctx->buffer_limit) want = std::max(bytes, std::min(want, ctx->buffer_limit));
+        IAC_HIP(alloc_buffer(ctx, want, &ctx->scratch[slot]));
         ctx->scratch_bytes[slot] = want;
     }
     *out = ctx->scratch[slot];
@@ -358,6 +376,10 @@ int iac_ctx_set_option(iac_ctx *ctx, int option, int64_t value)
         if (value != 0 && value != 1 && value != 4 && value != 8)
             return fail(IAC_ERR_INVALID_ARG, "IAC_OPT_PAIR_PREFETCH is 0, 1, 4 or 8");
         ctx->pair_prefetch = (int)value;
+        return IAC_OK;
+    case IAC_OPT_BUFFER_LIMIT:
+        if (value < 0) return fail(IAC_ERR_INVALID_ARG, "IAC_OPT_BUFFER_LIMIT is 0 or more");
+        ctx->buffer_limit = (size_t)value;
         return IAC_OK;
     case IAC_OPT_LAP_GROUPS:
         if (value < 0 || value > 65536) return fail(IAC_ERR_INVALID_ARG, "IAC_OPT_LAP_GROUPS is 0..65536");

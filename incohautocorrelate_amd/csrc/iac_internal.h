@@ -44,6 +44,7 @@ struct iac_ctx {
     int pair_mode = 0;    // pair engine: 0/1 lanes on consecutive pairs, 2 a pair range per thread
     uint32_t frame_chunk = 0;
     uint32_t lap_groups = 0;      // LAP finder: two-frame groups per tile in a row of the block order (0: 16)
+    size_t buffer_limit = 0;      // bytes of one work buffer at most (0: no limit)
     uint64_t sim_chunk_rows = 0;  // simulator: rows (pixel x subpixel) per GEMM launch with subpixels or modes
     int box_cap = 0;        // pair engine: LDS box voxels, 1024, 1920 or 4096 (0 = per kind)
     int pair_prefetch = 0;  // pair engine: pairs per load batch (1, 4 or 8; 0 = 1)
@@ -72,6 +73,10 @@ constexpr int kPathCounter = 2;
 int bind(iac_ctx *ctx);
 // Ensures scratch arena `slot` holds at least `bytes`; returns its pointer in *out.
 int scratch(iac_ctx *ctx, int slot, size_t bytes, void **out);
+// The same, but *out is null where the memory is short: for a path that another can stand in for.
+int scratch_if(iac_ctx *ctx, int slot, size_t bytes, void **out);
+// hipMalloc within the context's buffer limit; out of memory leaves no error behind.
+hipError_t alloc_buffer(iac_ctx *ctx, size_t bytes, void **out);
 
 // Page-locked staging of at least `bytes`; slot 1 waits until its last uploads have been read
 // (upload_done marks them on the context's stream).

@@ -3037,7 +3037,14 @@ int pairs_run(iac_ctx *ctx, const PairRun &R)
     const Sizes z = sizes_of(R, nc, chunks.size());
     // scratch: sorted records + cell offsets (slot 1), H + group offsets + self + chunks (slot 2)
     void *s1 = nullptr, *s2 = nullptr;
-    IAC_TRY(scratch(ctx, 1, z.srec + z.cs + strip_bytes(R, sp, schunks.size()), &s1));
+    if (sp) {
+        IAC_TRY(scratch_if(ctx, 1, z.srec + z.cs + strip_bytes(R, sp, schunks.size()), &s1));
+        if (!s1) {  // the walk needs 16 bytes per record less
+            sp = nullptr;
+            schunks.clear();
+        }
+    }
+    if (!s1) IAC_TRY(scratch(ctx, 1, z.srec + z.cs, &s1));
     IAC_TRY(scratch(ctx, 2, z.h + z.goff + z.self + z.chunks, &s2));
     Bufs b{};
     strip_place(b, static_cast<char *>(s1) + z.srec + z.cs, R, sp, schunks.size());
@@ -3173,7 +3180,8 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
         const size_t bh = ordered ? 0 : up(nvox * R.ngroups * sizeof(unsigned long long)),
                      bg = up((R.ngroups + 1) * sizeof(uint32_t)), bs = up(R.ngroups * sizeof(unsigned long long));
         void *s1 = nullptr, *s2 = nullptr;
-        IAC_TRY(scratch(ctx, 1, brec + bcs + bcur, &s1));
+        IAC_TRY(scratch_if(ctx, 1, brec + bcs + bcur, &s1));
+        if (!s1) return IAC_OK;  // the keys take up to 36 bytes per pixel; the walk needs none
         IAC_TRY(scratch(ctx, 2, bh + bg + bs + chunks.size() * sizeof(Chunk) + 256, &s2));
         char *p1 = static_cast<char *>(s1), *p2 = static_cast<char *>(s2);
         auto *srec = reinterpret_cast<float4 *>(p1);
@@ -3280,8 +3288,12 @@ int pairs_prepare(iac_ctx *ctx, const PairRun &R0, PairBatch **out)
     auto up = [](size_t x) { return (x + 255) / 256 * 256; };
     const size_t base = up(z.srec + z.cs + z.h + z.goff + z.self + z.chunks + tbytes);
     const size_t stask = sp ? up(sp->tasks.size() * sizeof(Task)) : 0;
-    const size_t total = base + stask + strip_bytes(B->R, sp, schunks.size());
-    hipError_t e = hipMalloc(&B->mem, total);
+    hipError_t e = alloc_buffer(ctx, base + stask + strip_bytes(B->R, sp, schunks.size()), &B->mem);
+    if (e == hipErrorOutOfMemory && sp) {  // the walk needs 16 bytes per record less
+        sp = nullptr;
+        schunks.clear();
+        e = alloc_buffer(ctx, base, &B->mem);
+    }
     if (e != hipSuccess) {
         delete B;
         return hip_fail(e, "pairs_prepare allocation", __FILE__, __LINE__);

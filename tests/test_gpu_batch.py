@@ -482,3 +482,42 @@ def test_batch_prepared_on_strips_follows_options_set_later(ctx, dev):
     finally:
         ctx.set_option(iac.OPT_PAIR_MODE, 0)
         batch.destroy()
+
+
+def test_strips_leave_the_run_to_the_walk_where_memory_is_short(dev):
+    """A work buffer that holds the walk's records but not the strips' beside them: the same mesh by
+    the walk, from one call and from a prepared batch; a buffer too small for either is an error,
+    after which the context works on."""
+    import torch
+
+    import incohautocorrelate_amd as iac
+    from gpu_helpers import gpu_batch
+
+    km, shape, pix, cnt, off = many_frames(60, 200, 1e5, 95)
+    n = int(off[-1])
+    c = iac.Context(0)
+    try:
+        call = lambda: mesh_np(gpu_batch(c, dev, km, pix, cnt, off, shape))  # noqa: E731
+        ref, paths = paths_of(c, call)
+        assert paths == (0, 1, 0)
+        c.close()
+        c = iac.Context(0)
+        c.set_option(iac.OPT_BUFFER_LIMIT, 24 * n)
+        got, paths = paths_of(c, call)
+        assert paths == (1, 0, 0) and np.array_equal(got, ref)
+        m = torch.zeros(shape.size_ab ** 2 * shape.size_c, dtype=torch.int64, device=dev)
+        c.set_option(iac.OPT_BUFFER_LIMIT, 24 * n + 8 * m.numel())  # a batch keeps its half mesh beside them
+        batch = c.ac3d_batch(to_dev(km, dev), to_dev(pix.astype(np.uint32), dev), to_dev(cnt.astype(np.uint16), dev),
+                             to_dev(off.astype(np.uint64), dev), n, shape)
+        got, paths = paths_of(c, lambda: batch.launch(m) or mesh_np(m))
+        batch.destroy()
+        assert paths == (1, 0, 0) and np.array_equal(got, ref)
+        c.close()
+        c = iac.Context(0)
+        c.set_option(iac.OPT_BUFFER_LIMIT, 17 * n // 2)
+        with pytest.raises(iac.IACError):
+            call()
+        c.set_option(iac.OPT_BUFFER_LIMIT, 0)
+        assert np.array_equal(call(), ref)
+    finally:
+        c.close()

@@ -516,3 +516,26 @@ def test_cq_near_detectors_find_a_side(dev, rows, cols, dist, edge, tiles, inter
     finally:
         a.close()
         b.close()
+
+
+def test_cq_tiles_leave_the_run_to_the_walk_where_memory_is_short(dev):
+    import torch
+
+    import incohautocorrelate_amd as iac
+
+    _, km, mq = W.detector(256)
+    s = iac.mesh_shape_small_cofq(mq, 127)
+    img = to_dev(W.gamma_frames(256 * 256, 1, 1.0, 0.5, seed=9)[0], dev)
+    got = []
+    # the records of the image, with the walk's cell starts but not with the tiles' key tables
+    for limit, want in ((0, (0, 0, 1)), (16 * 256 * 256 + 16000, (1, 0, 0))):
+        c = iac.Context(0)
+        try:
+            c.set_option(iac.OPT_BUFFER_LIMIT, limit)
+            m = _zeros(s.size_ab ** 2 * s.size_c, dev)
+            c.cq_small(to_dev(km, dev), img, s, m, 0, 1e6)
+            assert c.pair_paths() == want
+            got.append(m)
+        finally:
+            c.close()
+    assert torch.equal(got[0], got[1])
