@@ -196,8 +196,9 @@ int iac_ac3d_batch_destroy(iac_ac3d_batch *batch);
  * with the given binning modes, timing the pair kernel of each with HIP events (best of two
  * runs after a planning run, into a scratch mesh the call allocates and frees), and makes
  * the fastest the context's options (IAC_OPT_PAIR_MODE, IAC_OPT_CELL_VOX(_V), IAC_OPT_BOX_CAP,
- * IAC_OPT_FRAME_CHUNK, IAC_OPT_TASK_REGION), which every later engine call of the context
- * uses.  The winner is cached in the context per (k-map, mesh shape, modes): a second call
+ * IAC_OPT_FRAME_CHUNK, IAC_OPT_TASK_REGION), which every later walk of the context
+ * uses (dense C(q) runs still go by region tiles).  The defaults stay where they come within 1 %
+ * of the fastest, and where strips take the whole batch but not so short a prefix.  The winner is cached in the context per (k-map, mesh shape, modes): a second call
  * with the same key applies it without timing (force_retune = 0).  *best gets the winner;
  * up to max_all candidate results go to all (may be NULL), their count to *n_all.  Pending
  * kernel timings of the context (iac_ctx_timing) are discarded.  No counterpart in the

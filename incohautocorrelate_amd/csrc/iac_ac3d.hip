@@ -572,7 +572,11 @@ void apply_point(iac_ctx *ctx, const iac_tune_result &r)
     ctx->box_cap = r.box_cap;
     ctx->task_region = r.task_region;
     ctx->frame_chunk = (uint32_t)r.frame_chunk;
+    ctx->tuned = true;
 }
+// A setting has to beat the defaults by this much to replace them: below it runs differ by chance, and
+// explicit settings keep strips and region tiles from runs that they would suit.
+constexpr float kTuneGain = 0.99f;
 
 bool same_shape(const iac_mesh_shape &a, const iac_mesh_shape &b) { return std::memcmp(&a, &b, sizeof(a)) == 0; }
 
@@ -597,7 +601,7 @@ int iac_ac3d_tune(iac_ctx *ctx, const float *d_kmap, uint32_t npix, const uint32
             e.interp1 == interp1 && e.interp2 == interp2 && e.double_map == (double_map ? 1 : 0)) {
             *best = e.best;
             best->ms = -1.0f;
-            apply_point(ctx, e.best);
+            apply_point(ctx, e.applied);
             return IAC_OK;
         }
     const uint32_t nf = std::min(nframes, prefix_frames ? prefix_frames : 1000u);
@@ -620,6 +624,7 @@ int iac_ac3d_tune(iac_ctx *ctx, const float *d_kmap, uint32_t npix, const uint32
     int rc = IAC_OK;
     iac_tune_result win{};
     win.ms = -1.0f;
+    float t_default = -1.0f;  // of the defaults (linear: of the first candidate, which equals them)
     uint32_t count = 0;
     for (size_t k = 0; k < npts && rc == IAC_OK; k++) {
         iac_tune_result r{pts[k].pair_mode, pts[k].cell_vox, pts[k].cell_vox, pts[k].box_cap, 0, pts[k].frame_chunk,
@@ -643,7 +648,27 @@ int iac_ac3d_tune(iac_ctx *ctx, const float *d_kmap, uint32_t npix, const uint32
         if (all && count < max_all) all[count] = r;
         count++;
         if (win.ms < 0 || r.ms < win.ms) win = r;
+        if (linear ? k == 0 : pts[k].pair_mode == 0) t_default = r.ms;
     }
+    // strips that take the batch but not so short a prefix have not been timed: the rule stands
+    bool strips = false;
+    if (rc == IAC_OK && !linear) {
+        iac::PairRun R;
+        std::memset(&R.spec, 0, sizeof(R.spec));
+        R.spec.kind = iac::kKindAc3d;
+        R.spec.P = engine_params(P);
+        R.ordered = false;
+        R.d_kmap = d_kmap;
+        R.npix = npix;
+        R.nframes = nframes;
+        bool timed = false;
+        rc = iac::pairs_strips_suit(ctx, R, (double)n / nf, &strips);
+        R.nframes = nf;
+        if (rc == IAC_OK) rc = iac::pairs_strips_suit(ctx, R, (double)n / nf, &timed);
+        strips = strips && !timed;
+    }
+    iac_tune_result applied = win;
+    if (strips || (t_default >= 0 && !(win.ms < kTuneGain * t_default))) applied = iac_tune_result{0, 0, 0, 0, 0, 0, win.ms};
     ctx->timing = timing;
     ctx->ev_used = 0;  // pending kernel timings of the caller are discarded
     ctx->ac3d_kernel = kernel;
@@ -651,9 +676,9 @@ int iac_ac3d_tune(iac_ctx *ctx, const float *d_kmap, uint32_t npix, const uint32
     (void)hipFree(mesh);
     if (rc != IAC_OK) return rc;
     if (n_all) *n_all = std::min(count, max_all);
-    apply_point(ctx, win);
+    apply_point(ctx, applied);
     *best = win;
-    iac_ctx::TuneEntry e{d_kmap, npix, *shape, interp1, interp2, double_map ? 1 : 0, win};
+    iac_ctx::TuneEntry e{d_kmap, npix, *shape, interp1, interp2, double_map ? 1 : 0, win, applied};
     ctx->tune_cache.push_back(e);
     return IAC_OK;
 }

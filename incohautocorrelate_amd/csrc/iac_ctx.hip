@@ -342,6 +342,19 @@ int iac_ctx_timing(iac_ctx *ctx, double *ms, uint64_t *launches, int reset)
 int iac_ctx_set_option(iac_ctx *ctx, int option, int64_t value)
 {
     IAC_TRY(iac::bind(ctx));
+    switch (option) {  // an engine option set by the caller is meant for every kind of run
+    case IAC_OPT_CELL_VOX:
+    case IAC_OPT_CELL_VOX_V:
+    case IAC_OPT_FRAME_CHUNK:
+    case IAC_OPT_TASK_REGION:
+    case IAC_OPT_PAIR_MODE:
+    case IAC_OPT_BOX_CAP:
+    case IAC_OPT_PAIR_PREFETCH:
+        ctx->tuned = false;
+        break;
+    default:
+        break;
+    }
     switch (option) {
     case IAC_OPT_AC3D_KERNEL:
         if (value < 0 || value > 2) return fail(IAC_ERR_INVALID_ARG, "IAC_OPT_AC3D_KERNEL is 0, 1 or 2");

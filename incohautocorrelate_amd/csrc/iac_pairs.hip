@@ -2675,7 +2675,8 @@ int get_plan(iac_ctx *ctx, hipStream_t st, const PairRun &R, int cell_vox, int b
     return IAC_OK;
 }
 
-// A context without engine options set: the options name the walk's settings, so they select it.
+// A context without engine options set: the options name the walk's settings, so they select it
+// (the autotuner's, which were measured on AC_uw, say nothing about the tiles of C(q)).
 bool default_options(iac_ctx *ctx)
 {
     return !(ctx->pair_mode || ctx->cell_vox || ctx->cell_vox_v || ctx->box_cap || ctx->task_region ||
@@ -3065,6 +3066,18 @@ int pairs_run(iac_ctx *ctx, const PairRun &R)
     return enqueue(ctx, st, R, b, true);
 }
 
+int pairs_strips_suit(iac_ctx *ctx, const PairRun &R, double mean, bool *suit)
+{
+    void *ext = nullptr;
+    IAC_TRY(scratch(ctx, 3, 6 * sizeof(uint32_t), &ext));
+    PlanRead read;
+    IAC_TRY(plan_read(ctx, 0, &read));
+    float kmin[3], ext3[3];
+    IAC_TRY(kmap_extents(ctx->stream, R.d_kmap, R.npix, static_cast<uint32_t *>(ext), read, kmin, ext3));
+    *suit = strip_shape(kmin, ext3, R, mean).g.ncv > 0;
+    return IAC_OK;
+}
+
 // ---- dense C(q) -----------------------------------------------------------------
 
 // Region side in voxels: the largest of these that makes kTileTasks tasks or more (smaller regions
@@ -3088,7 +3101,7 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
     *done = false;
     const PairSpec &S = R.spec;
     const bool ordered = R.ordered;
-    if (!default_options(ctx)) return IAC_OK;
+    if (!default_options(ctx) && !(ctx->tuned && ctx->pair_prefetch == 0)) return IAC_OK;
     // what the walk refuses (pairs_run, check_chunks) stays refused
     if (R.n_total >= (1ull << 32) || R.npix >= (1u << 28)) return IAC_OK;
     // round_away and the boxes' 24-bit products need |q vox| < 2^22

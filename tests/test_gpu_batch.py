@@ -521,3 +521,35 @@ def test_strips_leave_the_run_to_the_walk_where_memory_is_short(dev):
         assert np.array_equal(call(), ref)
     finally:
         c.close()
+
+
+def test_tuner_leaves_strips_and_tiles_reachable(dev):
+    """A prefix too short for strips does not keep them from the whole batch, and settings tuned on
+    AC_uw do not keep region tiles from C(q); an engine option set by the caller does both."""
+    import torch
+
+    import incohautocorrelate_amd as iac
+
+    km, shape, pix, cnt, off = many_frames(60, 200, 1e5, 95)
+    d_km, d_off = to_dev(km, dev), to_dev(off.astype(np.uint64), dev)
+    d_pix, d_cnt = to_dev(pix.astype(np.uint32), dev), to_dev(cnt.astype(np.uint16), dev)
+    small = iac.mesh_shape_small_cofq(iac.calc_kmap(iac.generate_pixel_map(60, 200, 75.0, [0, 0, 1e5], (1, 0, 0),
+                                                                           (0, 1, 0)))[3], 31)
+    img = to_dev(W.gamma_frames(60 * 200, 1, 1.0, 0.5, seed=2)[0], dev)
+    m = torch.zeros(shape.size_ab ** 2 * shape.size_c, dtype=torch.int64, device=dev)
+    cq = torch.zeros(small.size_ab ** 2 * small.size_c, dtype=torch.int64, device=dev)
+    c = iac.Context(0)
+    batch = lambda: c.ac3d_sparse_batch(d_km, d_pix, d_cnt, d_off, int(off[-1]), shape, m)  # noqa: E731
+    image = lambda: c.cq_small(d_km, img, small, cq, 0, 1e6)  # noqa: E731
+    try:
+        c.ac3d_tune(d_km, d_pix, d_cnt, d_off, shape, 0, 0, True, prefix_frames=20)
+        assert paths_of(c, batch)[1] == (0, 1, 0)
+        c.ac3d_tune(d_km, d_pix, d_cnt, d_off, shape, 0, 0, True, prefix_frames=20)  # from the cache
+        assert paths_of(c, batch)[1] == (0, 1, 0)
+        c.ac3d_tune(d_km, d_pix, d_cnt, d_off, shape, 1, 1, True, prefix_frames=20)  # linear settings
+        assert paths_of(c, image)[1] == (0, 0, 1)
+        c.set_option(iac.OPT_CELL_VOX, 5)
+        assert paths_of(c, batch)[1] == (1, 0, 0)
+        assert paths_of(c, image)[1] == (1, 0, 0)
+    finally:
+        c.close()
