@@ -2390,7 +2390,9 @@ void merge_strips(iac_pair_plan &pl, int per)
 {
     std::vector<Task> out;
     for (const Task &t : pl.tasks) {  // in the order of dv
-        if (!out.empty() && out.back().dv / per == t.dv / per) {
+        // (a distance between them that is beyond the cut or has no pixels starts another task: its
+        // pairs, if any, need not lie in the box)
+        if (!out.empty() && out.back().dv / per == t.dv / per && t.dv == out.back().dv + out.back().nv) {
             Task &o = out.back();
             const int x1 = std::max(o.bx0 + o.bx, t.bx0 + t.bx), y1 = std::max(o.by0 + o.by, t.by0 + t.by),
                       z1 = std::max(o.bz0 + o.bz, t.bz0 + t.bz);
@@ -2401,7 +2403,7 @@ void merge_strips(iac_pair_plan &pl, int per)
             o.by = y1 - o.by0;
             o.bz = z1 - o.bz0;
             o.inbox = o.inbox && t.inbox;
-            o.nv = t.dv - o.dv + 1;
+            o.nv++;
         } else {
             out.push_back(t);
             out.back().nv = 1;

@@ -553,3 +553,32 @@ def test_tuner_leaves_strips_and_tiles_reachable(dev):
         assert paths_of(c, image)[1] == (1, 0, 0)
     finally:
         c.close()
+
+
+def test_strips_with_a_distance_beyond_the_cut_between(ctx, dev):
+    """Four panels, each within one strip of 2.18 voxels: the first and the third pair five strips
+    apart, both with the second, three and two strips from it, only beyond Max_Q, and with the fourth
+    likewise.  A task of up to seven distances must not hold those between."""
+    import incohautocorrelate_amd as iac
+    from gpu_helpers import gpu_batch
+
+    mq = np.array([0.6, 0.8, 0.004], np.float32)
+    shape = iac.mesh_shape_big(mq, 95, 2.0)
+    vox, h, n = float(shape.voxel_per_dq), 2.1808762813, 24
+    panels = []
+    for y0, y1, x0 in ((0, 0.9 * h, 0), (3.05 * h, 3.9 * h, 60), (5.05 * h, 5.9 * h, 0), (0.8 * vox - 0.5, 0.8 * vox, 0)):
+        y, x = np.meshgrid(np.linspace(y0, y1, n), np.linspace(x0, x0 + 6, n), indexing="ij")
+        panels.append(np.stack([x.ravel(), y.ravel(), 0 * x.ravel()], 1))
+    km = (np.concatenate(panels) / vox).astype(np.float32)
+    rng = np.random.default_rng(3)
+    off = np.arange(801) * 1000
+    pix, cnt = rng.integers(0, len(km), off[-1]), rng.integers(1, 4, off[-1])
+    rots = W.random_rotations(800, 9).astype(np.float32)
+    got, paths = paths_of(ctx, lambda: mesh_np(gpu_batch(ctx, dev, km, pix, cnt, off, shape, rots=rots)))
+    assert paths == (0, 1, 0)
+    ctx.set_option(iac.OPT_AC3D_KERNEL, 1)
+    try:
+        ref = mesh_np(gpu_batch(ctx, dev, km, pix, cnt, off, shape, rots=rots))
+    finally:
+        ctx.set_option(iac.OPT_AC3D_KERNEL, 0)
+    assert np.array_equal(got, ref)
