@@ -2486,11 +2486,11 @@ CellGeom cell_grid(const float kmin[3], const float ext3[3], float vox, int cell
 }
 
 // Frames per strip block: enough blocks to even out the last of them, few enough flushes (a 3,000
-// frame run: 7.0 ms with 3,072 blocks, 6.8 with 6,144, 7.4 with 12,288).
-constexpr double kStripBlocks = 6144;
-uint32_t strip_chunk(uint32_t nframes, size_t ntasks)
+// frame run on 256 CUs: 7.0 ms with 12 blocks per CU, 6.8 with 24, 7.4 with 48).
+constexpr double kStripBlocks = 24;
+uint32_t strip_chunk(const iac_ctx *ctx, uint32_t nframes, size_t ntasks)
 {
-    return (uint32_t)std::max(1.0, std::min(64.0, (double)nframes * (double)ntasks / kStripBlocks));
+    return (uint32_t)std::max(1.0, std::min(64.0, (double)nframes * (double)ntasks / (kStripBlocks * ctx->num_cus)));
 }
 
 // Strips of an AC_uw run: ncv of them (0: strips do not pay), a task per `per` distances.
@@ -2502,12 +2502,13 @@ struct StripShape {
 // Tall tasks waste little of their box (it spans per + 1 strips for per of lanes) and flush seldom;
 // records of the lanes' strips should fill 64 lanes, or 128, and those of b outweigh the cost of
 // starting an item.  The shape of least cost, in clocks of a CU per frame: 27 per 64 pairs (VALU
-// issue; 34 with one block per CU, whose flush nothing covers), 6 pairs' worth for an item's start,
+// issue; 34 with one block per CU, whose flush nothing covers), 7.5 pairs' worth for an item's start,
 // 2.7 per voxel flushed to a rotated mesh (scattered atomics) or 1.5 to a plain one, shared
 // by a chunk's frames.  Shapes that leave waves or CUs idle pay for it (60 frames of 21,000 photons in
 // strips of half the detector: 90 ms, the walk 18), and no shape near the walk's cost
-// is taken.  Measured: 34 picks seven-row boxes and 6.5 ms, 27 twelve-row ones and 6.8.
-StripShape strip_shape(const float kmin[3], const float ext3[3], const PairRun &R, double mean)
+// is taken.  Measured: 34 picks seven-row boxes and 6.5 ms, 27 twelve-row ones and 6.8.  All frames
+// are taken to hold `mean` records (uneven ones have more pairs).
+StripShape strip_shape(const iac_ctx *ctx, const float kmin[3], const float ext3[3], const PairRun &R, double mean)
 {
     StripShape best{};
     CellGeom &g = best.g;
@@ -2532,9 +2533,9 @@ StripShape strip_shape(const float kmin[3], const float ext3[3], const PairRun &
             double groups = 1;  // waves' loads of a Poisson number of lanes
             for (int k = 1; k < 32; k++) groups += 0.5 * std::erfc((64.0 * k + 0.5 - L) / std::sqrt(2 * L));
             const double items = n * (n + m) / (2.0 * m), tasks = std::ceil(n / m);
-            const double frames = R.h_rots ? 1 : strip_chunk(R.nframes, (size_t)tasks);
+            const double frames = R.h_rots ? 1 : strip_chunk(ctx, R.nframes, (size_t)tasks);
             // idle waves where a block has few items, idle CUs where there are few blocks
-            const double waves = box > kStripBox2 ? 16 : 8, slots = box > kStripBox2 ? 256 : 512;
+            const double waves = box > kStripBox2 ? 16 : 8, slots = ctx->num_cus * (box > kStripBox2 ? 1 : 2);
             const double busy = std::min(1.0, frames * items / tasks / (3 * waves)) *
                                 std::min(1.0, tasks * R.nframes / frames / (6 * slots));
             const double pair_cost = items * groups * (nb + 7.5) * (box > kStripBox2 ? 34 : 27) / busy;
@@ -2659,7 +2660,7 @@ int get_plan(iac_ctx *ctx, hipStream_t st, const PairRun &R, int cell_vox, int b
     const CellGeom &sg = shape.g;
     if (strips) {
         *strips = nullptr;
-        if (default_options(ctx)) shape = strip_shape(kmin, ext3, R, mean);
+        if (default_options(ctx)) shape = strip_shape(ctx, kmin, ext3, R, mean);
         if (sg.ncv > 0) IAC_TRY(cell_extents(st, R.d_kmap, R.npix, sg, d_ext + 6 + 6 * kMaxCells, read.strips));
     }
     IAC_HIP(hipStreamSynchronize(st));
@@ -3035,7 +3036,7 @@ int pairs_run(iac_ctx *ctx, const PairRun &R)
     IAC_TRY(check_chunks(off, chunks));
     std::vector<Chunk> schunks;
     if (sp)
-        schunks = make_chunks(off, R.nframes, R.h_group_off, R.ngroups, strip_chunk(R.nframes, sp->tasks.size()), R.h_rots);
+        schunks = make_chunks(off, R.nframes, R.h_group_off, R.ngroups, strip_chunk(ctx, R.nframes, sp->tasks.size()), R.h_rots);
     const int nc = pl->g.ncu * pl->g.ncv;
     const Sizes z = sizes_of(R, nc, chunks.size());
     // scratch: sorted records + cell offsets (slot 1), H + group offsets + self + chunks (slot 2)
@@ -3076,7 +3077,7 @@ int pairs_strips_suit(iac_ctx *ctx, const PairRun &R, double mean, bool *suit)
     IAC_TRY(plan_read(ctx, 0, &read));
     float kmin[3], ext3[3];
     IAC_TRY(kmap_extents(ctx->stream, R.d_kmap, R.npix, static_cast<uint32_t *>(ext), read, kmin, ext3));
-    *suit = strip_shape(kmin, ext3, R, mean).g.ncv > 0;
+    *suit = strip_shape(ctx, kmin, ext3, R, mean).g.ncv > 0;
     return IAC_OK;
 }
 
@@ -3291,7 +3292,7 @@ int pairs_prepare(iac_ctx *ctx, const PairRun &R0, PairBatch **out)
     IAC_TRY(check_chunks(off.data(), chunks));
     std::vector<Chunk> schunks;
     if (sp)
-        schunks = make_chunks(off.data(), R0.nframes, R0.h_group_off, R0.ngroups, strip_chunk(R0.nframes, sp->tasks.size()));
+        schunks = make_chunks(off.data(), R0.nframes, R0.h_group_off, R0.ngroups, strip_chunk(ctx, R0.nframes, sp->tasks.size()));
     auto *B = new PairBatch();
     B->ctx = ctx;
     B->R = R0;
