@@ -89,14 +89,14 @@ __global__ void finish_kernel(uint32_t npix, uint32_t ntotal, float S, const flo
 // One block per frame: ArrayOperators::Sum<float> (IAC/ArrayOperators.h:260-268) of the frame's
 // values, a serial float sum in pixel order; MeanIntensity = sum / P and, with photon
 // discretisation, PhotonCount = (int) sum.
-template <bool kMask, bool kPhotons>
+template <bool kMask, bool kPhotons, class Index>
 __global__ void __launch_bounds__(iac::kSumThreads)
     frame_sums_kernel(const float *__restrict__ frames, uint32_t npix, const int *__restrict__ mask, float T, float S,
                       float *__restrict__ mean_intensity, int *__restrict__ photon_count)
 {
     __shared__ iac::SerialSumShared sh;
     const uint32_t f = blockIdx.x;
-    const float s = iac::serial_sum_block<kMask>(
+    const float s = iac::serial_sum_block<kMask, Index>(
         frames + (size_t)f * npix, mask, npix, sh,
         [=](float v, int m) { return frame_value(v, m, kMask, T, kPhotons ? S : 0.0f); });
     if (threadIdx.x != 0) return;
@@ -111,8 +111,12 @@ int accumulate_stack(iac_ctx *ctx, const float *d_frames, uint32_t nframes, uint
 {
     if (d_mean_intensity || d_photon_count) {
         if (nframes > 0x7fffffffu) return iac::fail(IAC_ERR_LIMIT, "too many frames in one stack");
-        auto sums = S > 0 ? (d_mask ? frame_sums_kernel<true, true> : frame_sums_kernel<false, true>)
-                          : (d_mask ? frame_sums_kernel<true, false> : frame_sums_kernel<false, false>);
+        auto pick = [&](auto index) {
+            using I = decltype(index);
+            return S > 0 ? (d_mask ? frame_sums_kernel<true, true, I> : frame_sums_kernel<false, true, I>)
+                         : (d_mask ? frame_sums_kernel<true, false, I> : frame_sums_kernel<false, false, I>);
+        };
+        auto sums = iac::sum_in_64(npix) ? pick(uint64_t{}) : pick(uint32_t{});
         hipLaunchKernelGGL(sums, dim3(nframes), dim3(iac::kSumThreads), 0, ctx->stream, d_frames, npix,
                            d_mask, T, S, d_mean_intensity, d_photon_count);
         IAC_HIP(hipGetLastError());

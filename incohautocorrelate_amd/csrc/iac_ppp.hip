@@ -369,6 +369,7 @@ __global__ void zero_acc_kernel(FrameAcc *acc, uint32_t n)
 // Pass 2: PhotonCount = (int) of the frame sum and MeanIntensity = (float)PhotonCount /
 // (float)npix (IAC/PPP.cpp:490-491); the exact integer sum where it holds, else the serial float
 // sum.  One block per frame.
+template <class Index>
 __global__ void __launch_bounds__(iac::kSumThreads)
     photon_count_kernel(const float *__restrict__ frames, uint32_t npix, const FrameAcc *__restrict__ acc,
                         int *__restrict__ count, float *__restrict__ mean)
@@ -377,7 +378,7 @@ __global__ void __launch_bounds__(iac::kSumThreads)
     const bool exact = !acc[f].bad && acc[f].mag <= (1ull << 24);
     __shared__ iac::SerialSumShared sh;
     const float s = exact ? (float)acc[f].sum
-                          : iac::serial_sum_block<false>(frames + (size_t)f * npix, nullptr, npix, sh,
+                          : iac::serial_sum_block<false, Index>(frames + (size_t)f * npix, nullptr, npix, sh,
                                                          [](float v, int) { return v; });
     if (threadIdx.x != 0) return;
     const int pc = iac::cvtt_i32(s);
@@ -491,7 +492,8 @@ int iac_ppp_lap(iac_ctx *ctx, const float *d_in, float *d_out, uint32_t nframes,
     }
     IAC_TRY(iac::timer_end(ctx));
     if (acc) {
-        hipLaunchKernelGGL(photon_count_kernel, dim3(nframes), dim3(iac::kSumThreads), 0, ctx->stream, d_out, npix, acc,
+        auto count = iac::sum_in_64(npix) ? photon_count_kernel<uint64_t> : photon_count_kernel<uint32_t>;
+        hipLaunchKernelGGL(count, dim3(nframes), dim3(iac::kSumThreads), 0, ctx->stream, d_out, npix, acc,
                            d_photon_count, d_mean_intensity);
         IAC_HIP(hipGetLastError());
     }

@@ -66,16 +66,21 @@ __device__ __forceinline__ void load_run(const T *__restrict__ p, T *v)
     }
 }
 
-// value(v, m): what a pixel of value v and mask m (1 without kMask) adds to the sum.  Called by
-// all threads of a block of kSumThreads; returns the frame's sum in every thread.
-template <bool kMask, class V>
+// Frames whose last chunk's pixel numbers may pass 2^32 count them in 64 bits (which costs 2 %:
+// 252 -> 257 us for averaging and sparsifying the frames above).
+inline bool sum_in_64(uint32_t npix) { return npix > UINT32_MAX - kSumChunk; }
+
+// value(v, m): what a pixel of value v and mask m (1 without kMask) adds to the sum.  Index: of pixels,
+// uint32_t or, where sum_in_64, uint64_t.  Called by all threads of a block of kSumThreads; returns the
+// frame's sum in every thread.
+template <bool kMask, class Index, class V>
 __device__ __forceinline__ float serial_sum_block(const float *__restrict__ fr, const int *__restrict__ mask,
-                                                  uint32_t npix, SerialSumShared &sh, V value)
+                                                  Index npix, SerialSumShared &sh, V value)
 {
     const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
     constexpr float kMid = 12582912.0f;  // 1.5 * 2^23, even: floats within 2^22 of it are 1 apart
-    auto load = [&](uint32_t j0, float *v) {
-        const uint32_t j = j0 + t * kSumPer;
+    auto load = [&](Index j0, float *v) {
+        const Index j = j0 + t * kSumPer;
         int m[kSumPer];
         if (npix - j0 >= kSumChunk) {
             load_run(fr + j, v);
@@ -95,7 +100,7 @@ __device__ __forceinline__ float serial_sum_block(const float *__restrict__ fr, 
     float s = 0.0f, v[kSumPer], next[kSumPer];
     uint32_t retries = 0;
     load(0, v);
-    for (uint32_t j0 = 0; j0 < npix; j0 += kSumChunk) {
+    for (Index j0 = 0; j0 < npix; j0 += kSumChunk) {
         if (npix - j0 > kSumChunk) load(j0 + kSumChunk, next);
         for (uint32_t first = 0; first < kSumThreads;) {  // threads below `first` are in s
             // s = m ulps; an s near zero (no such binade), infinite or NaN takes only zeros
@@ -105,7 +110,7 @@ __device__ __forceinline__ float serial_sum_block(const float *__restrict__ fr, 
             const float ulp = flat ? 0.0f : copysignf(__uint_as_float((uint32_t)(127 - 23 + ex) << 23), s);
             const int m0 = flat ? 0 : (int)((__float_as_uint(s) & 0x7fffffu) | 0x800000u);
             // the window: as many values as the frame has behind it, in whole waves
-            const uint32_t behind = (j0 / kSumPer + first) / 64 + 1;
+            const uint32_t behind = (uint32_t)((j0 / kSumPer + first) / 64) + 1;
             const uint32_t end = min(kSumThreads, (first / 64 + behind) * 64);
             UlpMap own{0, 0};
             int lo = 0, hi = 0;
@@ -181,7 +186,7 @@ __device__ __forceinline__ float serial_sum_block(const float *__restrict__ fr, 
             if (++retries > kSumRetries) {
                 // the rest value by value, fed in order into wave 0's running sum
                 if (wave == 0) {
-                    for (uint32_t j = j0 + first * kSumPer; j < npix; j += 64) {
+                    for (Index j = j0 + first * kSumPer; j < npix; j += 64) {
                         const bool in = lane < npix - j;
                         const int x = __float_as_int(in ? value(fr[j + lane], kMask ? mask[j + lane] : 1) : 0.0f);
 #pragma unroll

@@ -96,3 +96,18 @@ def test_hit_lists_at_slice_edges(ctx, dev, npix, nframes, fill):
         assert np.array_equal(off.cpu().numpy(), np.cumsum([0] + [len(r) for r in ref]))
         want = np.concatenate([np.asarray(r, np.float32).reshape(-1, 4) for r in ref])
         assert np.array_equal(rec[:n].cpu().numpy().view(np.int32), want.view(np.int32))
+
+
+def test_frame_sum_near_2_32_pixels(ctx, dev):
+    """The last chunk of a frame whose pixel positions end just below 2^32."""
+    import torch
+
+    npix = 2**32 - 300
+    fr = torch.zeros(npix, device=dev)
+    fr[0], fr[2**31 + 5], fr[-1] = 1.0, 4.0, 2.5
+    avg, mean = torch.zeros(npix, device=dev), torch.zeros(1, device=dev)
+    ctx.average_intensity(fr.reshape(1, npix), None, 0.0, 0.0, avg, mean)
+    assert float(mean[0]) == float(np.float32(7.5) / np.float32(npix))
+    assert [float(avg[i]) for i in (0, 2**31 + 5, npix - 1, 77)] == [1.0, 4.0, 2.5, 0.0]
+    del fr, avg
+    torch.cuda.empty_cache()
