@@ -533,13 +533,16 @@ uint64_t tri_units(uint64_t n)
     return nt * (nt + 1) / 2 * kUnits;
 }
 
-// A block clears and flushes a whole histogram, so small runs take fewer blocks: kShare units per
-// wave at least (linear C(q) and AC_uw of a 64 x 70 detector, 500 bins: 64.5 us with every block,
-// 53.2 us so).
+// A block clears and flushes a whole histogram, so small runs take fewer blocks: up to kShare units
+// per wave (linear C(q) and AC_uw of a 64 x 70 detector, 500 bins: 64.5 us with every block,
+// 53.2 us so), fewer where that would leave CUs without a block (C(q) of a 20 x 20 detector: 35.5 us
+// with kShare each, 23.4 so).
 constexpr uint64_t kShare = 4;
 unsigned blocks_for_units(iac_ctx *ctx, uint32_t size, uint64_t units)
 {
-    const uint64_t want = (units + kWaves * kShare - 1) / (kWaves * kShare);
+    const uint64_t cus = (uint64_t)std::max(1, ctx->num_cus);
+    const uint64_t share = std::max<uint64_t>(1, std::min(kShare, units / (kWaves * cus)));
+    const uint64_t want = (units + kWaves * share - 1) / (kWaves * share);
     return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(persistent_blocks(ctx, size), want));
 }
 
