@@ -45,7 +45,7 @@ __global__ void u64_to_f64_kernel(const unsigned long long *__restrict__ in, siz
 // 1,000 events of a 129 x 129 x 3 mesh), so the big mesh is cut into bricks held in LDS: a block
 // takes a brick and a slice of the events, finds per event the small voxels that can reach the
 // brick (the brick turned back by the transposed matrix), bins exactly those and flushes the
-// brick with contiguous adds: 284 us and 42 us for the rest.  Bound: VALU issue, most of it for
+// brick with contiguous adds: 284 us and 39 us for the rest.  Bound: VALU issue, most of it for
 // the rows of candidates, whose 54 updates per brick and event lie in about 50 rows.  Other bricks
 // and events per block measured (whole call, 315 us): 16 x 8 x 8 with 32, 128 or 256 events 340,
 // 326, 378 us; 16 x 16 x 16 with 128 events 358; 16 x 8 x 4 459; the z rows of a y row in one
@@ -57,7 +57,8 @@ __global__ void u64_to_f64_kernel(const unsigned long long *__restrict__ in, siz
 constexpr float kOrtho = 1e-4f;               // largest |(R^T R - 1)_ij| the bricks take
 constexpr int kBrX = 16, kBrY = 8, kBrZ = 8;  // 8 KB: 16 voxels are two 64-byte segments to flush
 constexpr int kBrick = kBrX * kBrY * kBrZ;
-constexpr uint32_t kBrickEvents = 64;        // events that reach a brick, per block (about)
+constexpr uint32_t kBrickEvents = 6;       // log2 of the events that reach a brick, per block (about), at most
+constexpr uint32_t kBrickEventsLeast = 2;  // and at least, where the bricks alone leave CUs idle
 
 __device__ __forceinline__ bool orthonormal(const float *R)
 {
@@ -126,7 +127,7 @@ struct BrickEvent {
 template <bool kLinear>
 __global__ void __launch_bounds__(256)
     merge_brick_kernel(const double *__restrict__ small, size_t small_stride, int sab, int sc, int ka, int kb, int kc,
-                       const float *__restrict__ rw, uint32_t nev, double mult, int nbx, int nby,
+                       const float *__restrict__ rw, uint32_t nev, uint32_t per_log2, double mult, int nbx, int nby,
                        unsigned long long *__restrict__ big)
 {
     __shared__ unsigned long long box[kBrick];
@@ -147,7 +148,7 @@ __global__ void __launch_bounds__(256)
     // (its half diagonal + cc) / r
     const float r = sqrtf(mid[0] * mid[0] + mid[1] * mid[1] + mid[2] * mid[2]);
     const float share = fminf(1.0f, (11.0f + (float)cc) / fmaxf(r, 1.0f));
-    const uint32_t slices = min(gridDim.y, (uint32_t)((float)nev * share) / kBrickEvents + 1);
+    const uint32_t slices = min(gridDim.y, ((uint32_t)((float)nev * share) >> per_log2) + 1);
     if (blockIdx.y >= slices) return;
     const uint32_t ev0 = (uint32_t)((uint64_t)nev * blockIdx.y / slices);
     const uint32_t ev1 = (uint32_t)((uint64_t)nev * (blockIdx.y + 1) / slices);
@@ -271,24 +272,24 @@ __global__ void __launch_bounds__(256)
 constexpr uint32_t kRestEvents = 16;  // at most 64
 
 // Small voxel `ind` under the events of this block row: every update of an event the bricks
-// do not take (all events where bricks is 0), of the others only the count of updates outside
+// do not take (kBricks false: all events), of the others only the count of updates outside
 // the mesh, which voxels well inside its inscribed sphere do not have.
-template <bool kLinear>
+template <bool kLinear, bool kBricks>
 __global__ void __launch_bounds__(256)
     merge_rest_kernel(const double *__restrict__ small, size_t small_stride, int sab, int sc, int ka, int kb, int kc,
-                      const float *__restrict__ rw, uint32_t nev, double mult, int bricks,
+                      const float *__restrict__ rw, uint32_t nev, double mult,
                       unsigned long long *__restrict__ big, unsigned long long *__restrict__ dropped)
 {
     __shared__ uint64_t taken;  // bit k: the bricks take event e0 + k
     const size_t nsmall = (size_t)sab * sab * sc;
     const size_t ind = blockIdx.x * (size_t)blockDim.x + threadIdx.x;
     const uint32_t e0 = blockIdx.y * kRestEvents, e1 = min(nev, e0 + kRestEvents);
-    if (threadIdx.x < 64) {
+    if (kBricks && threadIdx.x < 64) {
         const uint32_t e = e0 + threadIdx.x;
-        const uint64_t b = __ballot(bricks && e < e1 && orthonormal(rw + 10 * (size_t)e));
+        const uint64_t b = __ballot(e < e1 && orthonormal(rw + 10 * (size_t)e));
         if (threadIdx.x == 0) taken = b;
     }
-    __syncthreads();
+    if (kBricks) __syncthreads();
     if (ind >= nsmall) return;
     const int cab = (sab - 1) / 2, cc = (sc - 1) / 2;
     const int ss_in = (int)(ind / ((size_t)sab * sab));
@@ -300,28 +301,27 @@ __global__ void __launch_bounds__(256)
     // |R q| <= |q| sqrt(1 + 3 kOrtho); the farthest corner is within one voxel of it per axis
     const float inner = (float)cab - 1.5f;
     const bool inside = inner > 0.0f && (qa * qa + qb * qb + qc * qc) * (1.0f + 4.0f * kOrtho) < inner * inner;
-    const uint64_t skip = taken;
+    const uint64_t skip = kBricks ? taken : 0;
     const uint32_t n = e1 - e0;
-    if (inside && skip == (n < 64 ? (1ull << n) - 1 : ~0ull)) return;
+    if (kBricks && inside && skip == (n < 64 ? (1ull << n) - 1 : ~0ull)) return;
     for (uint32_t i = e0; i < e1; i++) {
         const float *R = rw + 10 * (size_t)i;
-        const bool in_bricks = (skip >> (i - e0)) & 1;
+        const bool in_bricks = kBricks && ((skip >> (i - e0)) & 1);
         if (in_bricks && inside) continue;
         const double val_in = small[small_stride * i + ind];  // stride 0: one mesh for all events
         if (val_in < (double)1e-37f) continue;
         const float q0 = R[0] * qi0 + R[1] * qi1 + R[2] * qi2;
         const float q1 = R[3] * qi0 + R[4] * qi1 + R[5] * qi2;
         const float q2 = R[6] * qi0 + R[7] * qi1 + R[8] * qi2;
-        merge_voxel<kLinear, false>(q0, q1, q2, val_in, (double)R[9], mult, cab,
-                             [&](int fs, int ms, int ss, unsigned long long v) {
-                                 if ((unsigned)fs < (unsigned)sab && (unsigned)ms < (unsigned)sab &&
-                                     (unsigned)ss < (unsigned)sab) {
-                                     if (v && !in_bricks)
-                                         atomicAdd(big + (size_t)fs + (size_t)ms * sab + (size_t)ss * sab * sab, v);
-                                 } else {
-                                     atomicAdd(dropped, 1ull);
-                                 }
-                             });
+        auto add = [&](int fs, int ms, int ss, unsigned long long v) {
+            if ((unsigned)fs < (unsigned)sab && (unsigned)ms < (unsigned)sab && (unsigned)ss < (unsigned)sab) {
+                if (v && !in_bricks) atomicAdd(big + (size_t)fs + (size_t)ms * sab + (size_t)ss * sab * sab, v);
+            } else {
+                atomicAdd(dropped, 1ull);
+            }
+        };
+        if (in_bricks) merge_voxel<kLinear, true>(q0, q1, q2, val_in, (double)R[9], mult, cab, add);
+        else merge_voxel<kLinear, false>(q0, q1, q2, val_in, (double)R[9], mult, cab, add);
     }
 }
 
@@ -500,27 +500,38 @@ static int merge_launch(iac_ctx *ctx, const double *d_small_cq, bool per_event, 
     const int sab = (int)small_shape->size_ab, sc = (int)small_shape->size_c;
     const int ka = (int)small_shape->k_a, kb = (int)small_shape->k_b, kc = (int)small_shape->k_c;
     auto *big = reinterpret_cast<unsigned long long *>(d_big);
-    // Bricks cost about 20 us and 3 ns each before their first candidate, a scattered add costs
-    // 0.04 ns: measured break-even (nearest / linear) at 63 / 8 events of 65 x 65 x 3 (405 bricks),
-    // 11 / 1 of 129 x 129 x 3 (2,601) and 10 / 1 of 257 x 257 x 3 (18,513).  100 linear events of
-    // those meshes take 441, 1,451 and 4,938 us scattered, 150, 214 and 603 us in bricks.  The
-    // candidate ranges are 16 bits.
+    // Bricks cost a fixed time and a little each before their first candidate, scattered adds cost by
+    // their number.  Whole calls, scattered and in bricks: 944,000 adds of 53 x 53 x 7 (196 bricks)
+    // 34 and 35 us, 1,258,000 46 and 36; 710,000 of 65 x 65 x 7 (405) 38 and 28;
+    // 1,341,000 of 193 x 193 x 3 (8,125) 44 and 42, 1,788,000 60 and 45.  96 linear events of
+    // 65 x 65 x 3, 129 x 129 x 3 and 193 x 193 x 3: 409, 1,358 and 2,521 us scattered, 74, 186 and 292
+    // in bricks.  The candidate ranges are 16 bits.
     const uint64_t nbx = (sab + kBrX - 1) / kBrX, nby = (sab + kBrY - 1) / kBrY, nbz = (sab + kBrZ - 1) / kBrZ;
     const uint64_t nbricks = nbx * nby * nbz;
-    const bool bricks = (uint64_t)nev * nsmall * (interp ? 8 : 1) >= 600000 + 75 * nbricks && sab < 32768 &&
-                        sc < 32768 && nbricks < (1u << 31);
+    const uint64_t least = 600000 + 75 * nbricks + (nbricks < (uint64_t)ctx->num_cus ? 600000 : 0);
+    const bool bricks = (uint64_t)nev * nsmall * (interp ? 8 : 1) >= least && sab < 32768 && sc < 32768 &&
+                        nbricks < (1u << 31);
     const dim3 rest((unsigned)((nsmall + 255) / 256), (nev + kRestEvents - 1) / kRestEvents);
     IAC_TRY(iac::timer_begin(ctx));
     if (bricks) {
-        const dim3 grid((unsigned)nbricks, std::min<uint32_t>(65535, nev / kBrickEvents + 1));
+        // Fewer bricks than eight per CU: blocks of fewer events, so that there are about as many (share:
+        // of the events, those that reach a brick, on average).  64 linear events of 31 x 31 x 7 (32
+        // bricks): 167 us with 64 each, 50 so (107 scattered); 96 nearest of 129 x 129 x 3 (2,601): 69 and 71.
+        const double share = std::min(1.0, 1.3 * (11 + sc / 2) / (0.5 * sab));
+        const double blocks = 8.0 * std::max(1, ctx->num_cus), per = nev * share * nbricks / blocks;
+        uint32_t per_log2 = kBrickEvents;
+        if (nbricks < blocks)
+            while (per_log2 > kBrickEventsLeast && per < (double)(1u << per_log2)) per_log2--;
+        const dim3 grid((unsigned)nbricks, std::min<uint32_t>(65535, (nev >> per_log2) + 1));
         hipLaunchKernelGGL(interp ? merge_brick_kernel<true> : merge_brick_kernel<false>, grid, dim3(256), 0,
-                           ctx->stream, d_small_cq, stride, sab, sc, ka, kb, kc, d_rw10, nev, mult, (int)nbx, (int)nby,
-                           big);
+                           ctx->stream, d_small_cq, stride, sab, sc, ka, kb, kc, d_rw10, nev, per_log2, mult, (int)nbx,
+                           (int)nby, big);
         IAC_HIP(hipGetLastError());
     }
-    hipLaunchKernelGGL(interp ? merge_rest_kernel<true> : merge_rest_kernel<false>, rest, dim3(256), 0, ctx->stream,
-                       d_small_cq, stride, sab, sc, ka, kb, kc, d_rw10, nev, mult, bricks ? 1 : 0, big,
-                       ctx->d_counters);
+    auto kern = interp ? (bricks ? merge_rest_kernel<true, true> : merge_rest_kernel<true, false>)
+                       : (bricks ? merge_rest_kernel<false, true> : merge_rest_kernel<false, false>);
+    hipLaunchKernelGGL(kern, rest, dim3(256), 0, ctx->stream, d_small_cq, stride, sab, sc, ka, kb, kc, d_rw10, nev, mult,
+                       big, ctx->d_counters);
     IAC_HIP(hipGetLastError());
     IAC_TRY(iac::timer_end(ctx));
     return IAC_OK;

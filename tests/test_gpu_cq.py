@@ -418,7 +418,7 @@ def test_cq_region_tiles_vs_engine(dev, rows, cols, dist, edge, axes, interp):
         b.close()
 
 
-@pytest.mark.parametrize("nev", [1, 300])
+@pytest.mark.parametrize("nev", [1, 400])
 def test_merge_nan_rotation(ctx, dev, nev):
     """A matrix with NaN entries bins a coordinate that is NaN at voxel 0, beside rotations or alone,
     few events (scattered adds) and many (bricks for the others)."""
@@ -539,3 +539,10 @@ def test_cq_tiles_leave_the_run_to_the_walk_where_memory_is_short(dev):
         finally:
             c.close()
     assert torch.equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("sab,sc,nev", [(17, 3, 1500), (33, 7, 200), (49, 7, 100), (65, 3, 80)])
+@pytest.mark.parametrize("interp", [0, 1])
+def test_merge_bricks_in_slices_vs_oracle(ctx, dev, sab, sc, nev, interp):
+    """Meshes of fewer bricks than the chip has room for, whose events are cut into slices of 4 to 64."""
+    test_merge_bricks_vs_oracle(ctx, dev, (0, 1, 2), sab, sc, nev, interp)
