@@ -88,17 +88,19 @@ __global__ void finish_kernel(uint32_t npix, uint32_t ntotal, float S, const flo
 
 // One block per frame: ArrayOperators::Sum<float> (IAC/ArrayOperators.h:260-268) of the frame's
 // values, a serial float sum in pixel order; MeanIntensity = sum / P and, with photon
-// discretisation, PhotonCount = (int) sum.
-template <bool kMask, bool kPhotons, class Index>
-__global__ void __launch_bounds__(iac::kSumThreads)
+// discretisation, PhotonCount = (int) sum.  kShort: one wave per frame, of at most kSumShort pixels.
+template <bool kMask, bool kPhotons, class Index, bool kShort>
+__global__ void __launch_bounds__(kShort ? 64 : iac::kSumThreads)
     frame_sums_kernel(const float *__restrict__ frames, uint32_t npix, const int *__restrict__ mask, float T, float S,
                       float *__restrict__ mean_intensity, int *__restrict__ photon_count)
 {
     __shared__ iac::SerialSumShared sh;
     const uint32_t f = blockIdx.x;
-    const float s = iac::serial_sum_block<kMask, Index>(
-        frames + (size_t)f * npix, mask, npix, sh,
-        [=](float v, int m) { return frame_value(v, m, kMask, T, kPhotons ? S : 0.0f); });
+    auto value = [=](float v, int m) { return frame_value(v, m, kMask, T, kPhotons ? S : 0.0f); };
+    const float *fr = frames + (size_t)f * npix;
+    float s;
+    if constexpr (kShort) s = iac::serial_sum_wave<kMask>(fr, mask, npix, value);
+    else s = iac::serial_sum_block<kMask, Index>(fr, mask, npix, sh, value);
     if (threadIdx.x != 0) return;
     if (mean_intensity) mean_intensity[f] = s / (float)npix;
     if (photon_count && kPhotons) photon_count[f] = iac::cvtt_i32(s);
@@ -111,13 +113,16 @@ int accumulate_stack(iac_ctx *ctx, const float *d_frames, uint32_t nframes, uint
 {
     if (d_mean_intensity || d_photon_count) {
         if (nframes > 0x7fffffffu) return iac::fail(IAC_ERR_LIMIT, "too many frames in one stack");
-        auto pick = [&](auto index) {
+        auto pick = [&](auto index, auto is_short) {
             using I = decltype(index);
-            return S > 0 ? (d_mask ? frame_sums_kernel<true, true, I> : frame_sums_kernel<false, true, I>)
-                         : (d_mask ? frame_sums_kernel<true, false, I> : frame_sums_kernel<false, false, I>);
+            constexpr bool B = decltype(is_short)::value;
+            return S > 0 ? (d_mask ? frame_sums_kernel<true, true, I, B> : frame_sums_kernel<false, true, I, B>)
+                         : (d_mask ? frame_sums_kernel<true, false, I, B> : frame_sums_kernel<false, false, I, B>);
         };
-        auto sums = iac::sum_in_64(npix) ? pick(uint64_t{}) : pick(uint32_t{});
-        hipLaunchKernelGGL(sums, dim3(nframes), dim3(iac::kSumThreads), 0, ctx->stream, d_frames, npix,
+        const bool few = npix <= iac::kSumShort;
+        auto sums = few ? pick(uint32_t{}, std::true_type{})
+                        : (iac::sum_in_64(npix) ? pick(uint64_t{}, std::false_type{}) : pick(uint32_t{}, std::false_type{}));
+        hipLaunchKernelGGL(sums, dim3(nframes), dim3(few ? 64 : iac::kSumThreads), 0, ctx->stream, d_frames, npix,
                            d_mask, T, S, d_mean_intensity, d_photon_count);
         IAC_HIP(hipGetLastError());
     }

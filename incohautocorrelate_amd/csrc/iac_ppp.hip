@@ -368,18 +368,20 @@ __global__ void zero_acc_kernel(FrameAcc *acc, uint32_t n)
 
 // Pass 2: PhotonCount = (int) of the frame sum and MeanIntensity = (float)PhotonCount /
 // (float)npix (IAC/PPP.cpp:490-491); the exact integer sum where it holds, else the serial float
-// sum.  One block per frame.
-template <class Index>
-__global__ void __launch_bounds__(iac::kSumThreads)
+// sum.  One block per frame, of one wave where kShort (frames of at most kSumShort pixels).
+template <class Index, bool kShort>
+__global__ void __launch_bounds__(kShort ? 64 : iac::kSumThreads)
     photon_count_kernel(const float *__restrict__ frames, uint32_t npix, const FrameAcc *__restrict__ acc,
                         int *__restrict__ count, float *__restrict__ mean)
 {
     const uint32_t f = blockIdx.x;
     const bool exact = !acc[f].bad && acc[f].mag <= (1ull << 24);
     __shared__ iac::SerialSumShared sh;
-    const float s = exact ? (float)acc[f].sum
-                          : iac::serial_sum_block<false, Index>(frames + (size_t)f * npix, nullptr, npix, sh,
-                                                         [](float v, int) { return v; });
+    auto value = [](float v, int) { return v; };
+    float s;
+    if (exact) s = (float)acc[f].sum;
+    else if constexpr (kShort) s = iac::serial_sum_wave<false>(frames + (size_t)f * npix, nullptr, npix, value);
+    else s = iac::serial_sum_block<false, Index>(frames + (size_t)f * npix, nullptr, npix, sh, value);
     if (threadIdx.x != 0) return;
     const int pc = iac::cvtt_i32(s);
     if (count) count[f] = pc;
@@ -492,8 +494,10 @@ int iac_ppp_lap(iac_ctx *ctx, const float *d_in, float *d_out, uint32_t nframes,
     }
     IAC_TRY(iac::timer_end(ctx));
     if (acc) {
-        auto count = iac::sum_in_64(npix) ? photon_count_kernel<uint64_t> : photon_count_kernel<uint32_t>;
-        hipLaunchKernelGGL(count, dim3(nframes), dim3(iac::kSumThreads), 0, ctx->stream, d_out, npix, acc,
+        const bool few = npix <= iac::kSumShort;
+        auto count = few ? photon_count_kernel<uint32_t, true>
+                         : (iac::sum_in_64(npix) ? photon_count_kernel<uint64_t, false> : photon_count_kernel<uint32_t, false>);
+        hipLaunchKernelGGL(count, dim3(nframes), dim3(few ? 64 : iac::kSumThreads), 0, ctx->stream, d_out, npix, acc,
                            d_photon_count, d_mean_intensity);
         IAC_HIP(hipGetLastError());
     }

@@ -111,3 +111,25 @@ def test_frame_sum_near_2_32_pixels(ctx, dev):
     assert [float(avg[i]) for i in (0, 2**31 + 5, npix - 1, 77)] == [1.0, 4.0, 2.5, 0.0]
     del fr, avg
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("npix", [63, 64, 65, 2047, 2048, 2049, 5000])
+def test_frame_sums_bit_exact_about_the_short_frames(ctx, dev, npix):
+    """One wave per frame up to 2,048 pixels, a block of partial chunks beyond."""
+    test_frame_sums_bit_exact(ctx, dev, npix)
+
+
+@pytest.mark.parametrize("rows,cols", [(8, 16), (32, 64), (33, 63), (40, 60)])
+def test_photon_counts_of_corrected_frames(ctx, dev, rows, cols):
+    """Gain-corrected frames, whose sums are no whole numbers: short frames and longer ones."""
+    import torch
+
+    npix, nf = rows * cols, 9
+    rng = np.random.default_rng(npix)
+    fr = (rng.random((nf, npix)) * 50).astype(np.float32)
+    out = torch.zeros((nf, npix), device=dev)
+    pc, mi = torch.zeros(nf, dtype=torch.int32, device=dev), torch.zeros(nf, device=dev)
+    ctx.ppp_lap(torch.from_numpy(fr).to(dev), out, [], 37.0, gain_only=True, photon_count=pc, mean_intensity=mi)
+    want = np.array([int(np.add.accumulate(f, dtype=np.float32)[-1]) for f in out.cpu().numpy()])
+    assert np.array_equal(pc.cpu().numpy(), want)
+    assert np.array_equal(mi.cpu().numpy(), want.astype(np.float32) / np.float32(npix))
