@@ -88,7 +88,7 @@ __global__ void finish_kernel(uint32_t npix, uint32_t ntotal, float S, const flo
 
 // One block per frame: ArrayOperators::Sum<float> (IAC/ArrayOperators.h:260-268) of the frame's
 // values, a serial float sum in pixel order; MeanIntensity = sum / P and, with photon
-// discretisation, PhotonCount = (int) sum.  kShort: one wave per frame, of at most kSumShort pixels.
+// discretisation, PhotonCount = (int) sum.  kShort: one wave per frame.
 template <bool kMask, bool kPhotons, class Index, bool kShort>
 __global__ void __launch_bounds__(kShort ? 64 : iac::kSumThreads)
     frame_sums_kernel(const float *__restrict__ frames, uint32_t npix, const int *__restrict__ mask, float T, float S,
@@ -119,7 +119,7 @@ int accumulate_stack(iac_ctx *ctx, const float *d_frames, uint32_t nframes, uint
             return S > 0 ? (d_mask ? frame_sums_kernel<true, true, I, B> : frame_sums_kernel<false, true, I, B>)
                          : (d_mask ? frame_sums_kernel<true, false, I, B> : frame_sums_kernel<false, false, I, B>);
         };
-        const bool few = npix <= iac::kSumShort;
+        const bool few = iac::sum_short(npix, nframes, ctx->num_cus);
         auto sums = few ? pick(uint32_t{}, std::true_type{})
                         : (iac::sum_in_64(npix) ? pick(uint64_t{}, std::false_type{}) : pick(uint32_t{}, std::false_type{}));
         hipLaunchKernelGGL(sums, dim3(nframes), dim3(few ? 64 : iac::kSumThreads), 0, ctx->stream, d_frames, npix,

@@ -368,7 +368,7 @@ __global__ void zero_acc_kernel(FrameAcc *acc, uint32_t n)
 
 // Pass 2: PhotonCount = (int) of the frame sum and MeanIntensity = (float)PhotonCount /
 // (float)npix (IAC/PPP.cpp:490-491); the exact integer sum where it holds, else the serial float
-// sum.  One block per frame, of one wave where kShort (frames of at most kSumShort pixels).
+// sum.  One block per frame, of one wave where kShort.
 template <class Index, bool kShort>
 __global__ void __launch_bounds__(kShort ? 64 : iac::kSumThreads)
     photon_count_kernel(const float *__restrict__ frames, uint32_t npix, const FrameAcc *__restrict__ acc,
@@ -494,7 +494,7 @@ int iac_ppp_lap(iac_ctx *ctx, const float *d_in, float *d_out, uint32_t nframes,
     }
     IAC_TRY(iac::timer_end(ctx));
     if (acc) {
-        const bool few = npix <= iac::kSumShort;
+        const bool few = iac::sum_short(npix, nframes, ctx->num_cus);
         auto count = few ? photon_count_kernel<uint32_t, true>
                          : (iac::sum_in_64(npix) ? photon_count_kernel<uint64_t, false> : photon_count_kernel<uint32_t, false>);
         hipLaunchKernelGGL(count, dim3(nframes), dim3(few ? 64 : iac::kSumThreads), 0, ctx->stream, d_out, npix, acc,

@@ -70,10 +70,11 @@ __device__ __forceinline__ void load_run(const T *__restrict__ p, T *v)
 // 252 -> 257 us for averaging and sparsifying the frames above).
 inline bool sum_in_64(uint32_t npix) { return npix > UINT32_MAX - kSumChunk; }
 
-// Frames up to here are added value by value by one wave: a growing sum leaves its first ten binades
-// within them, a stop each (averages of 20 frames of 1,000 pixels 31.6 us by the scan, 17.0 so;
-// of 1,600 pixels 32.4 and 21.7, growing by 0.9 us per 100).
-constexpr uint32_t kSumShort = 2048;
+// Short frames are added value by value by one wave: a growing sum leaves its first ten binades within
+// them, a stop each.  Averages of 20 frames of 1,000 pixels 31.6 us by the scan, 17.0 so; of 2,560
+// 33.7 and 30.3, growing by 0.9 us per 100; with more frames than CUs the scans' blocks queue up:
+// 300 frames of 4,096 pixels 70.7 and 55.5.
+inline bool sum_short(uint32_t npix, uint32_t nframes, int cus) { return npix <= (nframes > (uint32_t)cus ? 4096u : 2560u); }
 
 // The same sum by a one-wave block: 64 values at once, fed in order into a sum that every lane holds.
 template <bool kMask, class V>

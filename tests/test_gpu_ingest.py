@@ -113,9 +113,9 @@ def test_frame_sum_near_2_32_pixels(ctx, dev):
     torch.cuda.empty_cache()
 
 
-@pytest.mark.parametrize("npix", [63, 64, 65, 2047, 2048, 2049, 5000])
+@pytest.mark.parametrize("npix", [63, 64, 65, 2559, 2560, 2561, 5000])
 def test_frame_sums_bit_exact_about_the_short_frames(ctx, dev, npix):
-    """One wave per frame up to 2,048 pixels, a block of partial chunks beyond."""
+    """One wave per frame up to 2,560 pixels, a block of partial chunks beyond."""
     test_frame_sums_bit_exact(ctx, dev, npix)
 
 
