@@ -44,6 +44,8 @@ BYTES_PER_UPDATE = 16  # one 8 B bin read + one 8 B bin write per pair-update
 # (pair mode, box, cell_vox, frame_chunk): FETCH_SIZE x2.0 + WRITE_SIZE x1.0 KiB from two
 # rocprofv3 --pmc passes, scaled by a 2 GiB copy kernel (profiles/pairs_lds_sparse1024_10k.md).
 MEASURED_TRAFFIC = {(1, 1920, 6, 32): (2 * 1511764 + 3118483) * 1024}
+# strip_kernel's, of the 10,000 frames (profiles/strips_sparse1024_10k.md)
+STRIP_TRAFFIC = (2 * 7521047 + 794909) * 1024
 # The same for sim_gemm_kernel per launch of 1,000 frames (profiles/sim_gemm_mfma_512_10k_1000.md)
 SIM_TRAFFIC = {"bf16x3": (2 * 70271911 + 1025181) * 1024}
 
@@ -165,6 +167,7 @@ def main():
 
     ctx.enable_timing(True)
     ctx.kernel_time(reset=True)
+    before = ctx.pair_paths()
     torch.cuda.synchronize()
     t1 = time.perf_counter()
     for _ in range(args.steps):
@@ -173,6 +176,7 @@ def main():
     t2 = time.perf_counter()
     kms, klaunch = ctx.kernel_time(reset=True)
     ctx.enable_timing(False)
+    path = path_since(ctx, before)  # what took the timed steps' pairs
     ms_per_step = (t2 - t1) * 1e3 / args.steps
     value = updates / ((t2 - t1) / args.steps)
     k_avg_ms = kms / max(klaunch, 1)
@@ -183,7 +187,7 @@ def main():
     if ctx.dropped():
         log(f"[bench] WARNING: {ctx.dropped()} updates fell outside the mesh")
 
-    parity = check_headline(ctx, iac, kmap, data, shape, dev, d_mesh)
+    parity = check_headline(ctx, iac, kmap, data, shape, dev, d_mesh, path, (d_kmap, d_pix, d_cnt, d_off))
     batch.destroy()
     # the one-call entry point (plans the chunks on every call) for comparison
     torch.cuda.synchronize()
@@ -223,8 +227,10 @@ def main():
     sim = None if args.no_sim else sim_leg(args, iac, W, dev)
 
     traffic = None
-    strips = args.kernel != 1 and not (tuned and (tuned.get("mode") or tuned.get("box")))  # the engine's defaults
-    if tuned and args.kernel != 1 and not strips:
+    strips = path == "strips"
+    if strips:
+        traffic = STRIP_TRAFFIC if args.frames == 10000 and args.seed == 2 else None
+    elif tuned and args.kernel != 1:
         key = (tuned.get("mode") or 1, tuned.get("box") or 1920, tuned.get("cell_vox") or 6,
                tuned.get("frame_chunk") or 32)
         if (tuned.get("cell_vox_v") or key[2]) != key[2] or tuned.get("region"):
@@ -253,6 +259,7 @@ def main():
             "kernel": "tile (global atomics)" if args.kernel == 1 else "LDS strips" if strips else "LDS cell boxes",
             "step": "prepared frame batch (iac_ac3d_batch_launch): clear + gather + sort + pairs + mirror",
             "tuned": tuned,
+            "path": path,
         },
         # The 16 B read-modify-write of each pair-update lands in an LDS box, not in HBM
         # (measured HBM traffic is under 1 % of it): the bound is the LDS, against its
@@ -306,10 +313,17 @@ def main():
 TUNE_KEYS = ("box", "cell_vox", "cell_vox_v", "region", "frame_chunk", "mode")
 
 
+def path_since(ctx, before):
+    """What took the pairs of the engine's passes since `before` (pair_paths): one name, or both."""
+    names = [n for n, a, b in zip(("walk", "strips", "region tiles"), before, ctx.pair_paths()) if b > a]
+    return " and ".join(names) if names else "tile kernel"
+
+
 def apply_lds_config(ctx, iac, cfg):
-    """Set the LDS kernel options of one tuning point (0 = library default)."""
+    """Set the LDS kernel options of one tuning point (0 = library default; all 0 leaves the engine its
+    strips and region tiles)."""
     ctx.set_option(iac.OPT_BOX_CAP, cfg.get("box", 0))
-    ctx.set_option(iac.OPT_PAIR_PREFETCH, 1)
+    ctx.set_option(iac.OPT_PAIR_PREFETCH, 0)
     ctx.set_option(iac.OPT_CELL_VOX, cfg.get("cell_vox", 0))
     ctx.set_option(iac.OPT_CELL_VOX_V, cfg.get("cell_vox_v", 0))
     ctx.set_option(iac.OPT_TASK_REGION, cfg.get("region", 0))
@@ -321,9 +335,9 @@ def cfg_str(cfg):
     return " ".join(f"{k}={cfg.get(k, 0)}" for k in TUNE_KEYS)
 
 
-# around the defaults (mode 2, 3-voxel cells, 1920-voxel boxes, 2x2-cell regions); frames per
-# block do not matter here (a dense frame is one chunk)
-CQ_GRID = [dict(mode=m, box=b, cell_vox=c, cell_vox_v=c, frame_chunk=32, region=r)
+# the engine's own choice, then the walk around its defaults (mode 2, 3-voxel cells, 1920-voxel boxes,
+# 2x2-cell regions); frames per block do not matter here (a dense frame is one chunk)
+CQ_GRID = [{}] + [dict(mode=m, box=b, cell_vox=c, cell_vox_v=c, frame_chunk=32, region=r)
            for m in (1, 2) for b, c in ((1920, 3), (1024, 3), (1920, 4), (4096, 4), (1920, 5)) for r in (2, 4)]
 
 
@@ -341,10 +355,11 @@ def autotune(ctx, iac, d_kmap, d_pix, d_cnt, d_off, shape, label="tune"):
             "by": "iac_ac3d_tune (library)", "candidates": cands}
 
 
-def check_headline(ctx, iac, kmap, data, shape, dev, d_mesh):
+def check_headline(ctx, iac, kmap, data, shape, dev, d_mesh, path, d_in):
     """Parity of the headline pass: the first 20 frames through the same prepared-batch
-    code path and tuned settings, bit for bit against the oracle; the full timed mesh
-    (all frames, identity rotation, nearest-neighbour levels) for point symmetry,
+    code path and tuned settings (so few frames go by the walk), bit for bit against the
+    oracle; the full timed mesh (all frames, identity rotation, nearest-neighbour levels) bit for
+    bit against the walk's where another path took the timed steps, for point symmetry,
     mesh[C + d] == mesh[C - d], and a centre voxel of at least 1000 sum c^2 (every self
     pair lands there; so do neighbours closer than half a voxel)."""
     import torch
@@ -364,19 +379,32 @@ def check_headline(ctx, iac, kmap, data, shape, dev, d_mesh):
     torch.cuda.synchronize()
     sub.destroy()
     ok = bool((m.cpu().numpy().view(np.uint64) == ref).all())
+    same = None
+    if path != "walk":
+        with iac.Context(0) as walk:
+            walk.set_option(iac.OPT_AC3D_KERNEL, 2)
+            walk.set_option(iac.OPT_PAIR_MODE, 1)
+            mw = torch.zeros_like(d_mesh)
+            walk.ac3d_sparse_batch(*d_in, int(data["frame_off"][-1]), shape, mw)
+            walk.sync()
+            if walk.pair_paths() != (1, 0, 0):
+                raise SystemExit("headline check: the reference pass was not the walk's")
+            same = bool(torch.equal(mw, d_mesh))
+            del mw
     # the full timed mesh (the last replay)
     full = d_mesh.cpu().numpy().view(np.uint64).reshape(shape.size_c, shape.size_ab, shape.size_ab)
     sym = bool(np.array_equal(full, full[::-1, ::-1, ::-1]))
     cnt = data["cnt"].astype(np.uint64)
     centre = int(full[shape.center[2], shape.center[1], shape.center[0]])
     centre_ok = centre >= 1000 * int((cnt * cnt).sum())
-    log(f"[bench] bit-exact check on {nf} frames: {'OK' if ok else 'MISMATCH'} (oracle {dt:.1f}s); full mesh "
-        f"point symmetric: {sym}; centre voxel >= 1000 sum c^2: {centre_ok}")
-    if not (ok and sym and centre_ok):
+    log(f"[bench] bit-exact check on {nf} frames: {'OK' if ok else 'MISMATCH'} (oracle {dt:.1f}s); full mesh by {path} "
+        f"equals the walk's: {same}; point symmetric: {sym}; centre voxel >= 1000 sum c^2: {centre_ok}")
+    if not (ok and sym and centre_ok and same is not False):
         raise SystemExit("headline parity check failed")
-    return {"oracle_frames": nf, "bit_exact_vs_oracle": ok, "full_mesh_point_symmetric": sym,
+    return {"oracle_frames": nf, "bit_exact_vs_oracle": ok, "timed_path": path, "full_mesh_equals_walk": same,
+            "full_mesh_point_symmetric": sym,
             "full_mesh_centre_at_least_1000_sum_c2": centre_ok,
-            "path": "the timed prepared-batch path with the tuned settings"}
+            "path": "oracle: the prepared-batch path with the tuned settings; the walk: the timed full mesh"}
 
 
 def queue_leg(args, iac, dev, kmap, d_kmap, data, shape, d_ref, updates, batch_ms):
@@ -912,8 +940,10 @@ def cq_dense_leg(args, iac, W, dev):
         ctx.enable_timing(False)
         apply_lds_config(ctx, iac, best[1])
         tuned = dict(best[1])
+    before = ctx.pair_paths()
     run()
     torch.cuda.synchronize()
+    path = path_since(ctx, before)
     steps = max(1, min(args.steps, 3))
     t = time.perf_counter()
     for _ in range(steps):
@@ -932,7 +962,7 @@ def cq_dense_leg(args, iac, W, dev):
     return {"workload": f"dense C(q) small (AutoCorr_CQ_small): {n}x{n} detector, {nf} FP32 Gamma(1, 0.5) frames, "
                         f"{s.size_ab}x{s.size_ab}x{s.size_c} uint64 mesh, nearest neighbour",
             "value": pairs / (ms * 1e-3), "unit": "ordered pixel pairs/s", "ms_per_step": ms, "steps": steps,
-            "pairs_per_step": pairs, "tuned": tuned, "cpu_baseline": cpu}
+            "pairs_per_step": pairs, "path": path, "tuned": tuned, "cpu_baseline": cpu}
 
 
 def ppp_leg(args, iac, dev, probes):
