@@ -2530,16 +2530,24 @@ StripShape strip_shape(const iac_ctx *ctx, const float kmin[3], const float ext3
             if (box > kStripBox1) break;
             if (n > kMaxStrips || n < 2) continue;
             const double L = m * h * per_vox, nb = h * per_vox;
-            double groups = 1;  // waves' loads of a Poisson number of lanes
-            for (int k = 1; k < 32; k++) groups += 0.5 * std::erfc((64.0 * k + 0.5 - L) / std::sqrt(2 * L));
             const double items = n * (n + m) / (2.0 * m), tasks = std::ceil(n / m);
             const double frames = R.h_rots ? 1 : strip_chunk(ctx, R.nframes, (size_t)tasks);
             // idle waves where a block has few items, idle CUs where there are few blocks
             const double waves = box > kStripBox2 ? 16 : 8, slots = ctx->num_cus * (box > kStripBox2 ? 1 : 2);
             const double busy = std::min(1.0, frames * items / tasks / (3 * waves)) *
                                 std::min(1.0, tasks * R.nframes / frames / (6 * slots));
-            const double pair_cost = items * groups * (nb + 7.5) * (box > kStripBox2 ? 34 : 27) / busy;
-            if (pair_cost > 1.3 * walk) continue;  // (the model is a sixth too high for strips)
+            const double per_group = items * (nb + 7.5) * (box > kStripBox2 ? 34 : 27) / busy;
+            // (the model is a sixth too high for strips)
+            if (per_group * 0.9 * std::max(1.0, std::min(L / 64, 30.0)) > std::min(1.3 * walk, least)) continue;
+            double groups = 1;  // waves' loads of a Poisson number of lanes; erfc(6) is 2e-17
+            const double sd = std::sqrt(2 * L);
+            for (int k = 1; k < 32; k++) {
+                const double z = (64.0 * k + 0.5 - L) / sd;
+                if (z > 6) break;
+                groups += z < -6 ? 1.0 : 0.5 * std::erfc(z);
+            }
+            const double pair_cost = per_group * groups;
+            if (pair_cost > 1.3 * walk) continue;
             const double cost = pair_cost + tasks * box / 4 * (R.h_rots ? 2.7 : 1.5) / frames;
             if (cost < least) {
                 least = cost;
