@@ -2416,7 +2416,9 @@ void merge_strips(iac_pair_plan &pl, int per)
     pl.tasks.swap(out);
 }
 
-// Page-locked read-back area of a plan: the k-map's extents, the cells', 8 bytes, then more.
+// Page-locked read-back area of a plan: the k-map's extents (and a dense run's counts: kHead words),
+// the cells', the strips', then more.
+constexpr size_t kHead = 12;
 struct PlanRead {
     uint32_t *kext, *cells, *strips;
     uint64_t *more;
@@ -2424,21 +2426,22 @@ struct PlanRead {
 int plan_read(iac_ctx *ctx, size_t more_bytes, PlanRead *out)
 {
     void *p = nullptr;
-    IAC_TRY(pinned(ctx, 0, (8 + 6 * (size_t)(kMaxCells + kMaxStrips)) * sizeof(uint32_t) + more_bytes, &p));
+    IAC_TRY(pinned(ctx, 0, (kHead + 6 * (size_t)(kMaxCells + kMaxStrips)) * sizeof(uint32_t) + more_bytes, &p));
     out->kext = static_cast<uint32_t *>(p);
-    out->cells = out->kext + 8;
+    out->cells = out->kext + kHead;
     out->strips = out->cells + 6 * (size_t)kMaxCells;
     out->more = reinterpret_cast<uint64_t *>(out->strips + 6 * (size_t)kMaxStrips);
     return IAC_OK;
 }
 
-// Enqueues the extents of the k-map, d_ext initialised, and their copy to read.kext.
-int kmap_extents_enqueue(hipStream_t st, const float *d_kmap, uint32_t npix, uint32_t *d_ext, const PlanRead &read)
+// Enqueues the extents of the k-map, d_ext initialised, and the copy of `words` words there to read.kext.
+int kmap_extents_enqueue(hipStream_t st, const float *d_kmap, uint32_t npix, uint32_t *d_ext, const PlanRead &read,
+                         size_t words = 6)
 {
     const unsigned eb = std::max(1u, std::min<unsigned>(64, (npix + 1023) / 1024));
     hipLaunchKernelGGL(kext_kernel, dim3(eb), dim3(256), 0, st, d_kmap, npix, d_ext);
     IAC_HIP(hipGetLastError());
-    IAC_HIP(hipMemcpyAsync(read.kext, d_ext, 6 * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    IAC_HIP(hipMemcpyAsync(read.kext, d_ext, words * sizeof(uint32_t), hipMemcpyDeviceToHost, st));
     return IAC_OK;
 }
 void kmap_extents_read(const PlanRead &read, float kmin[3], float ext3[3])
@@ -3123,23 +3126,23 @@ int cq_tiles_run(iac_ctx *ctx, const PairRun &R, const float *d_frames, bool *do
     // the k-map's extents | kept, flags | the cells' extents, a grid for each side
     constexpr size_t nsides = sizeof(kTileSides) / sizeof(kTileSides[0]);
     void *ext = nullptr;
-    IAC_TRY(scratch(ctx, 3, (12 + 6 * (size_t)(nsides * kMaxCells)) * sizeof(uint32_t), &ext));
+    IAC_TRY(scratch(ctx, 3, (kHead + 6 * (size_t)(nsides * kMaxCells)) * sizeof(uint32_t), &ext));
     uint32_t *d_ext = static_cast<uint32_t *>(ext);
     auto *d_kept = reinterpret_cast<unsigned long long *>(d_ext + 8);
     auto *d_plain = reinterpret_cast<uint32_t *>(d_kept + 1);
-    uint32_t *d_cells = d_ext + 12;
+    uint32_t *d_cells = d_ext + kHead;
     float kmin[3], ext3[3];
     PlanRead read;
-    IAC_TRY(plan_read(ctx, 2 * sizeof(uint64_t), &read));
+    IAC_TRY(plan_read(ctx, 0, &read));
     hipLaunchKernelGGL(cq_begin_kernel, dim3(1), dim3(64), 0, st, d_ext, d_kept, d_plain);
     hipLaunchKernelGGL(dense_scan_kernel, dim3((unsigned)std::min<uint64_t>(2048, (R.n_total + 4 * kBlock - 1) / (4 * kBlock))),
                        dim3(kBlock), 0, st, d_frames, R.n_total, S.mult, d_kept, d_plain);
-    IAC_TRY(kmap_extents_enqueue(st, R.d_kmap, R.npix, d_ext, read));
-    IAC_HIP(hipMemcpyAsync(read.more, d_kept, 2 * sizeof(uint64_t), hipMemcpyDeviceToHost, st));
+    IAC_TRY(kmap_extents_enqueue(st, R.d_kmap, R.npix, d_ext, read, kHead));
     IAC_HIP(hipStreamSynchronize(st));
     kmap_extents_read(read, kmin, ext3);
-    const uint64_t kept = read.more[0];
-    const uint32_t *flags = reinterpret_cast<const uint32_t *>(read.more + 1);
+    uint64_t kept = 0;
+    std::memcpy(&kept, read.kext + 8, sizeof(kept));
+    const uint32_t *flags = read.kext + 10;
     const bool wide = !flags[0];
     if (!flags[1]) return IAC_OK;  // negative values: the engine's pairs test each
     const int box_cap = ordered ? kBoxMax : kBoxSmall;
