@@ -662,9 +662,12 @@ int iac_ac3d_tune(iac_ctx *ctx, const float *d_kmap, uint32_t npix, const uint32
         R.npix = npix;
         R.nframes = nframes;
         bool timed = false;
-        rc = iac::pairs_strips_suit(ctx, R, (double)n / nf, &strips);
+        std::vector<uint64_t> off((size_t)nframes + 1);
+        const hipError_t e = hipMemcpy(off.data(), d_frame_off, off.size() * sizeof(uint64_t), hipMemcpyDeviceToHost);
+        rc = e == hipSuccess ? IAC_OK : iac::hip_fail(e, "tuner offsets", __FILE__, __LINE__);
+        if (rc == IAC_OK) rc = iac::pairs_strips_suit(ctx, R, off.data(), &strips);
         R.nframes = nf;
-        if (rc == IAC_OK) rc = iac::pairs_strips_suit(ctx, R, (double)n / nf, &timed);
+        if (rc == IAC_OK) rc = iac::pairs_strips_suit(ctx, R, off.data(), &timed);
         strips = strips && !timed;
     }
     iac_tune_result applied = win;

@@ -43,8 +43,9 @@ struct PairRun {
     const float *h_rots = nullptr;
 };
 
-// Whether strips suit an AC_uw run of R's k-map, modes and frames of `mean` records (synchronises).
-int pairs_strips_suit(iac_ctx *ctx, const PairRun &R, double mean, bool *suit);
+// Whether strips suit an AC_uw run of R's k-map, modes and frames at the offsets h_off, on the host
+// (synchronises).
+int pairs_strips_suit(iac_ctx *ctx, const PairRun &R, const uint64_t *h_off, bool *suit);
 int pairs_run(iac_ctx *ctx, const PairRun &run);
 
 // C(q) of dense frames d_frames ([nframes][npix]) by region tiles (run.rec and run.d_frame_off are

@@ -2502,6 +2502,35 @@ struct StripShape {
     int per;
 };
 
+// The records of a run's frames: their root mean square, and the most of one frame.
+struct FrameLoad {
+    double rms, most;
+};
+FrameLoad frame_load(const uint64_t *off, uint32_t nframes)
+{
+    double sum = 0, most = 0;
+    for (uint32_t f = 0; f < nframes; f++) {
+        const double n = (double)(off[f + 1] - off[f]);
+        sum += n * n;
+        most = std::max(most, n);
+    }
+    return FrameLoad{std::sqrt(sum / std::max(1u, nframes)), most};
+}
+
+// Waves' loads of a Poisson number of lanes, L on average (erfc(6) is 2e-17).
+double wave_loads(double L)
+{
+    if (L > 64.0 * 30) return L / 64 + 0.5;
+    double groups = 1;
+    const double sd = std::sqrt(2 * L);
+    for (int k = 1; k < 32; k++) {
+        const double z = (64.0 * k + 0.5 - L) / sd;
+        if (z > 6) break;
+        groups += z < -6 ? 1.0 : 0.5 * std::erfc(z);
+    }
+    return groups;
+}
+
 // Tall tasks waste little of their box (it spans per + 1 strips for per of lanes) and flush seldom;
 // records of the lanes' strips should fill 64 lanes, or 128, and those of b outweigh the cost of
 // starting an item.  The shape of least cost, in clocks of a CU per frame: 27 per 64 pairs (VALU
@@ -2509,9 +2538,13 @@ struct StripShape {
 // 2.7 per voxel flushed to a rotated mesh (scattered atomics) or 1.5 to a plain one, shared
 // by a chunk's frames.  Shapes that leave waves or CUs idle pay for it (60 frames of 21,000 photons in
 // strips of half the detector: 90 ms, the walk 18), and no shape near the walk's cost
-// is taken.  Measured: 34 picks seven-row boxes and 6.5 ms, 27 twelve-row ones and 6.8.  All frames
-// are taken to hold `mean` records (uneven ones have more pairs).
-StripShape strip_shape(const iac_ctx *ctx, const float kmin[3], const float ext3[3], const PairRun &R, double mean)
+// is taken.  Measured: 34 picks seven-row boxes and 6.5 ms, 27 twelve-row ones and 6.8.  The frames
+// count as if each held the root mean square of their records, and a frame of more than twice that
+// as the time of its block, which takes a whole task of it (250 lognormal frames of up to 20,000
+// photons, four draws: 4.4 to 7.1 ms in few tall strips by the mean alone, 1.6 to 2.3 so; the walk
+// 3.2 to 4.2).
+StripShape strip_shape(const iac_ctx *ctx, const float kmin[3], const float ext3[3], const PairRun &R,
+                       const FrameLoad &load)
 {
     StripShape best{};
     CellGeom &g = best.g;
@@ -2520,36 +2553,43 @@ StripShape strip_shape(const iac_ctx *ctx, const float kmin[3], const float ext3
     g.av = ext3[1] >= ext3[0] ? 1 : 0;
     g.au = 1 - g.av;
     const double vox = R.spec.P.vox, wide = std::floor(2 * ext3[g.au] * vox + 2), deep = std::floor(2 * ext3[2] * vox + 2);
-    const double tall = ext3[g.av] * vox, per_vox = mean / std::max(1.0, tall);
+    const double tall = ext3[g.av] * vox, rms2 = load.rms * load.rms;
     // a second plan, sort and launch cost about 90 us, 0.3e-12 s per pair against the walk repay it
     // (a rotated mesh's smaller flushes more)
-    const double pairs = 0.5 * mean * mean * R.nframes;
+    const double pairs = 0.5 * rms2 * R.nframes;
     if (!(wide * deep * 4 * 3 <= kStripBox1) || !(pairs >= (R.h_rots ? 0x1p26 : 0x1p28))) return best;
-    const double walk = 0.5 * mean * mean / 64 * 55;  // what it takes for the pairs
+    // What the walk takes for the pairs, and at its end for a task of the largest frame (its cells are six
+    // voxels; the offset of most pairs holds 2 / cells of them).
+    double walk = 0.5 * rms2 / 64 * 55;
+    const bool uneven = load.most > 2 * load.rms;
+    if (uneven) {
+        const double cells = std::ceil(ext3[0] * vox / 6) * std::ceil(ext3[1] * vox / 6);
+        walk += 0.5 * load.most * load.most / 64 * 55 * 2 / std::max(2.0, cells) * 3 * ctx->num_cus / R.nframes;
+    }
     double least = 1e300, h_best = 0;
     for (int m = 1; m <= 8; m++)
         for (double h = 1; h <= 64; h *= 1.0905) {  // eighths of an octave
             const double rows = std::floor((m + 1) * h + 2), box = rows * wide * deep * 4, n = std::ceil(tall / h);
             if (box > kStripBox1) break;
             if (n > kMaxStrips || n < 2) continue;
-            const double L = m * h * per_vox, nb = h * per_vox;
+            const double L = m * h * load.rms / std::max(1.0, tall), nb = L / m;
             const double items = n * (n + m) / (2.0 * m), tasks = std::ceil(n / m);
             const double frames = R.h_rots ? 1 : strip_chunk(ctx, R.nframes, (size_t)tasks);
             // idle waves where a block has few items, idle CUs where there are few blocks
             const double waves = box > kStripBox2 ? 16 : 8, slots = ctx->num_cus * (box > kStripBox2 ? 1 : 2);
             const double busy = std::min(1.0, frames * items / tasks / (3 * waves)) *
                                 std::min(1.0, tasks * R.nframes / frames / (6 * slots));
-            const double per_group = items * (nb + 7.5) * (box > kStripBox2 ? 34 : 27) / busy;
+            const double per_step = items * (box > kStripBox2 ? 34 : 27);
             // (the model is a sixth too high for strips)
-            if (per_group * 0.9 * std::max(1.0, std::min(L / 64, 30.0)) > std::min(1.3 * walk, least)) continue;
-            double groups = 1;  // waves' loads of a Poisson number of lanes; erfc(6) is 2e-17
-            const double sd = std::sqrt(2 * L);
-            for (int k = 1; k < 32; k++) {
-                const double z = (64.0 * k + 0.5 - L) / sd;
-                if (z > 6) break;
-                groups += z < -6 ? 1.0 : 0.5 * std::erfc(z);
+            if (per_step * (nb + 7.5) / busy * 0.9 * std::max(1.0, std::min(L / 64, 30.0)) > std::min(1.3 * walk, least))
+                continue;
+            double pair_cost = per_step * (nb + 7.5) / busy * wave_loads(L);
+            if (uneven) {
+                // its block has a CU to itself in the end, half of one (of whose SIMDs it fills half) before
+                const double x = load.most / load.rms;
+                const double late = per_step / tasks * (x * nb + 7.5) * wave_loads(x * L) * (box > kStripBox2 ? 1.5 : 3);
+                pair_cost += late * ctx->num_cus / R.nframes;
             }
-            const double pair_cost = per_group * groups;
             if (pair_cost > 1.3 * walk) continue;
             const double cost = pair_cost + tasks * box / 4 * (R.h_rots ? 2.7 : 1.5) / frames;
             if (cost < least) {
@@ -2648,10 +2688,9 @@ bool default_options(iac_ctx *ctx);
 // Cell grid of the k-map (two host round trips for the extents) and the task
 // table, from the context's cache when the geometry matches.  h_off: also the frames' offsets,
 // read back with them (valid until the context's next call).
-// strips: also the plan of the run's strips for frames of `mean` records (null where they do not
-// suit it).
+// strips (with h_off): also the plan of the run's strips (null where they do not suit it).
 int get_plan(iac_ctx *ctx, hipStream_t st, const PairRun &R, int cell_vox, int box_cap, int region,
-             iac_pair_plan **out, const uint64_t **h_off = nullptr, double mean = 0, iac_pair_plan **strips = nullptr)
+             iac_pair_plan **out, const uint64_t **h_off = nullptr, iac_pair_plan **strips = nullptr)
 {
     void *ext = nullptr;
     IAC_TRY(scratch(ctx, 3, (6 + 6 * (size_t)(kMaxCells + kMaxStrips)) * sizeof(uint32_t), &ext));
@@ -2659,19 +2698,19 @@ int get_plan(iac_ctx *ctx, hipStream_t st, const PairRun &R, int cell_vox, int b
     const size_t off_bytes = h_off ? ((size_t)R.nframes + 1) * sizeof(uint64_t) : 0;
     PlanRead read;
     IAC_TRY(plan_read(ctx, off_bytes, &read));
-    float kmin[3], ext3[3];
-    IAC_TRY(kmap_extents(st, R.d_kmap, R.npix, d_ext, read, kmin, ext3));
-    const CellGeom g = cell_grid(kmin, ext3, R.spec.P.vox, cell_vox);
-    IAC_TRY(cell_extents(st, R.d_kmap, R.npix, g, d_ext + 6, read.cells));
     if (h_off) {
         IAC_HIP(hipMemcpyAsync(read.more, R.d_frame_off, off_bytes, hipMemcpyDeviceToHost, st));
         *h_off = read.more;
     }
+    float kmin[3], ext3[3];
+    IAC_TRY(kmap_extents(st, R.d_kmap, R.npix, d_ext, read, kmin, ext3));
+    const CellGeom g = cell_grid(kmin, ext3, R.spec.P.vox, cell_vox);
+    IAC_TRY(cell_extents(st, R.d_kmap, R.npix, g, d_ext + 6, read.cells));
     StripShape shape{};
     const CellGeom &sg = shape.g;
     if (strips) {
         *strips = nullptr;
-        if (default_options(ctx)) shape = strip_shape(ctx, kmin, ext3, R, mean);
+        if (default_options(ctx)) shape = strip_shape(ctx, kmin, ext3, R, frame_load(*h_off, R.nframes));
         if (sg.ncv > 0) IAC_TRY(cell_extents(st, R.d_kmap, R.npix, sg, d_ext + 6 + 6 * kMaxCells, read.strips));
     }
     IAC_HIP(hipStreamSynchronize(st));
@@ -3041,8 +3080,7 @@ int pairs_run(iac_ctx *ctx, const PairRun &R)
     iac_pair_plan *pl = nullptr;
     const uint64_t *off = nullptr;
     iac_pair_plan *sp = nullptr;
-    IAC_TRY(get_plan(ctx, st, R, cell_vox_of(ctx, R), box_cap_of(ctx, R), region_of(ctx, R), &pl, &off,
-                     (double)R.n_total / std::max(1u, R.nframes), &sp));
+    IAC_TRY(get_plan(ctx, st, R, cell_vox_of(ctx, R), box_cap_of(ctx, R), region_of(ctx, R), &pl, &off, &sp));
     const std::vector<Chunk> chunks = make_chunks(off, R.nframes, R.h_group_off, R.ngroups, fchunk_of(ctx), R.h_rots);
     IAC_TRY(check_chunks(off, chunks));
     std::vector<Chunk> schunks;
@@ -3080,7 +3118,7 @@ int pairs_run(iac_ctx *ctx, const PairRun &R)
     return enqueue(ctx, st, R, b, true);
 }
 
-int pairs_strips_suit(iac_ctx *ctx, const PairRun &R, double mean, bool *suit)
+int pairs_strips_suit(iac_ctx *ctx, const PairRun &R, const uint64_t *h_off, bool *suit)
 {
     void *ext = nullptr;
     IAC_TRY(scratch(ctx, 3, 6 * sizeof(uint32_t), &ext));
@@ -3088,7 +3126,7 @@ int pairs_strips_suit(iac_ctx *ctx, const PairRun &R, double mean, bool *suit)
     IAC_TRY(plan_read(ctx, 0, &read));
     float kmin[3], ext3[3];
     IAC_TRY(kmap_extents(ctx->stream, R.d_kmap, R.npix, static_cast<uint32_t *>(ext), read, kmin, ext3));
-    *suit = strip_shape(ctx, kmin, ext3, R, mean).g.ncv > 0;
+    *suit = strip_shape(ctx, kmin, ext3, R, frame_load(h_off, R.nframes)).g.ncv > 0;
     return IAC_OK;
 }
 
@@ -3294,16 +3332,13 @@ int pairs_prepare(iac_ctx *ctx, const PairRun &R0, PairBatch **out)
     if (R0.n_total >= (1ull << 32)) return fail(IAC_ERR_LIMIT, "pair engine: at most 2^32 - 1 records per call");
     iac_pair_plan *pl = nullptr;
     iac_pair_plan *sp = nullptr;
-    IAC_TRY(get_plan(ctx, st, R0, cell_vox_of(ctx, R0), box_cap_of(ctx, R0), region_of(ctx, R0), &pl, nullptr,
-                     (double)R0.n_total / std::max(1u, R0.nframes), &sp));
-    std::vector<uint64_t> off(R0.nframes + 1);
-    IAC_HIP(hipMemcpyAsync(off.data(), R0.d_frame_off, off.size() * 8, hipMemcpyDeviceToHost, st));
-    IAC_HIP(hipStreamSynchronize(st));
-    const std::vector<Chunk> chunks = make_chunks(off.data(), R0.nframes, R0.h_group_off, R0.ngroups, fchunk_of(ctx));
-    IAC_TRY(check_chunks(off.data(), chunks));
+    const uint64_t *off = nullptr;
+    IAC_TRY(get_plan(ctx, st, R0, cell_vox_of(ctx, R0), box_cap_of(ctx, R0), region_of(ctx, R0), &pl, &off, &sp));
+    const std::vector<Chunk> chunks = make_chunks(off, R0.nframes, R0.h_group_off, R0.ngroups, fchunk_of(ctx));
+    IAC_TRY(check_chunks(off, chunks));
     std::vector<Chunk> schunks;
     if (sp)
-        schunks = make_chunks(off.data(), R0.nframes, R0.h_group_off, R0.ngroups, strip_chunk(ctx, R0.nframes, sp->tasks.size()));
+        schunks = make_chunks(off, R0.nframes, R0.h_group_off, R0.ngroups, strip_chunk(ctx, R0.nframes, sp->tasks.size()));
     auto *B = new PairBatch();
     B->ctx = ctx;
     B->R = R0;
