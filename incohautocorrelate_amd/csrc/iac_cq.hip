@@ -502,13 +502,14 @@ static int merge_launch(iac_ctx *ctx, const double *d_small_cq, bool per_event, 
     auto *big = reinterpret_cast<unsigned long long *>(d_big);
     // Bricks cost a fixed time and a little each before their first candidate, scattered adds cost by
     // their number.  Whole calls, scattered and in bricks: 944,000 adds of 53 x 53 x 7 (196 bricks)
-    // 34 and 35 us, 1,258,000 46 and 36; 710,000 of 65 x 65 x 7 (405) 38 and 28;
+    // 34 and 35 us, 1,258,000 46 and 36; 855,000 of 89 x 89 x 3 (864) 33 and 35, 1,140,000 42 and 40;
     // 1,341,000 of 193 x 193 x 3 (8,125) 44 and 42, 1,788,000 60 and 45.  96 linear events of
     // 65 x 65 x 3, 129 x 129 x 3 and 193 x 193 x 3: 409, 1,358 and 2,521 us scattered, 74, 186 and 292
     // in bricks.  The candidate ranges are 16 bits.
     const uint64_t nbx = (sab + kBrX - 1) / kBrX, nby = (sab + kBrY - 1) / kBrY, nbz = (sab + kBrZ - 1) / kBrZ;
     const uint64_t nbricks = nbx * nby * nbz;
-    const uint64_t least = 600000 + 75 * nbricks + (nbricks < (uint64_t)ctx->num_cus ? 600000 : 0);
+    const uint64_t cus = (uint64_t)std::max(1, ctx->num_cus);
+    const uint64_t least = nbricks >= 8 * cus ? 600000 + 75 * nbricks : (nbricks >= cus ? 850000 : 1200000);
     const bool bricks = (uint64_t)nev * nsmall * (interp ? 8 : 1) >= least && sab < 32768 && sc < 32768 &&
                         nbricks < (1u << 31);
     const dim3 rest((unsigned)((nsmall + 255) / 256), (nev + kRestEvents - 1) / kRestEvents);
@@ -518,10 +519,11 @@ static int merge_launch(iac_ctx *ctx, const double *d_small_cq, bool per_event, 
         // of the events, those that reach a brick, on average).  64 linear events of 31 x 31 x 7 (32
         // bricks): 167 us with 64 each, 50 so (107 scattered); 96 nearest of 129 x 129 x 3 (2,601): 69 and 71.
         const double share = std::min(1.0, 1.3 * (11 + sc / 2) / (0.5 * sab));
-        const double blocks = 8.0 * std::max(1, ctx->num_cus), per = nev * share * nbricks / blocks;
+        const double per = nev * share * nbricks / (8.0 * cus);
+        const uint32_t least_log2 = nbricks >= 4 * cus ? kBrickEventsLeast + 2 : kBrickEventsLeast;
         uint32_t per_log2 = kBrickEvents;
-        if (nbricks < blocks)
-            while (per_log2 > kBrickEventsLeast && per < (double)(1u << per_log2)) per_log2--;
+        if (nbricks < 8 * cus)
+            while (per_log2 > least_log2 && per < (double)(1u << per_log2)) per_log2--;
         const dim3 grid((unsigned)nbricks, std::min<uint32_t>(65535, (nev >> per_log2) + 1));
         hipLaunchKernelGGL(interp ? merge_brick_kernel<true> : merge_brick_kernel<false>, grid, dim3(256), 0,
                            ctx->stream, d_small_cq, stride, sab, sc, ka, kb, kc, d_rw10, nev, per_log2, mult, (int)nbx,
