@@ -71,22 +71,35 @@ __device__ __forceinline__ void load_run(const T *__restrict__ p, T *v)
 inline bool sum_in_64(uint32_t npix) { return npix > UINT32_MAX - kSumChunk; }
 
 // Short frames are added value by value by one wave: a growing sum leaves its first ten binades within
-// them, a stop each.  Averages of 20 frames of 1,000 pixels 31.6 us by the scan, 17.0 so; of 2,560
-// 33.7 and 30.3, growing by 0.9 us per 100; with more frames than CUs the scans' blocks queue up:
-// 300 frames of 4,096 pixels 70.7 and 55.5.
-inline bool sum_short(uint32_t npix, uint32_t nframes, int cus) { return npix <= (nframes > (uint32_t)cus ? 4096u : 2560u); }
+// them, a stop each.  Averages of 20 frames of 1,000 pixels 31.6 us by the scan, 15.6 so; of 2,560
+// 33.7 and 21.0, of 4,096 32.5 and 29.1; with more frames than CUs the scans' blocks queue up:
+// 300 frames of 4,096 pixels 70.9 and 41.6, of 8,192 76.0 and 64.4.
+inline bool sum_short(uint32_t npix, uint32_t nframes, int cus) { return npix <= (nframes > (uint32_t)cus ? 8192u : 4096u); }
 
 // The same sum by a one-wave block: 64 values at once, fed in order into a sum that every lane holds.
+// Bound: the chain of adds, an add and a lane read per value.
 template <bool kMask, class V>
 __device__ __forceinline__ float serial_sum_wave(const float *__restrict__ fr, const int *__restrict__ mask,
                                                  uint32_t npix, V value)
 {
     float s = 0.0f;
+    int m = 1;
+    float v = fr[min(threadIdx.x, npix - 1)];
+    if (kMask) m = mask[min(threadIdx.x, npix - 1)];
     for (uint32_t j0 = 0; j0 < npix; j0 += 64) {
-        const uint32_t j = j0 + threadIdx.x;
-        const int x = __float_as_int(j < npix ? value(fr[j], kMask ? mask[j] : 1) : 0.0f);
+        const int x = __float_as_int(j0 + threadIdx.x < npix ? value(v, m) : 0.0f);
+        const uint32_t next = min(j0 + 64 + threadIdx.x, npix - 1);  // loads under the adds
+        v = fr[next];
+        if (kMask) m = mask[next];
+        // a lane is read one add ahead: its scalar is ready when the chain of adds gets there
+        int a = __builtin_amdgcn_readlane(x, 0);
 #pragma unroll
-        for (int i = 0; i < 64; i++) s += __int_as_float(__builtin_amdgcn_readlane(x, i));
+        for (int i = 1; i < 64; i++) {
+            const int b = __builtin_amdgcn_readlane(x, i);
+            s += __int_as_float(a);
+            a = b;
+        }
+        s += __int_as_float(a);
     }
     return s;
 }

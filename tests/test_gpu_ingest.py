@@ -113,13 +113,13 @@ def test_frame_sum_near_2_32_pixels(ctx, dev):
     torch.cuda.empty_cache()
 
 
-@pytest.mark.parametrize("npix", [63, 64, 65, 2559, 2560, 2561, 5000])
+@pytest.mark.parametrize("npix", [63, 64, 65, 2560, 4095, 4096, 4097, 9000])
 def test_frame_sums_bit_exact_about_the_short_frames(ctx, dev, npix):
-    """One wave per frame up to 2,560 pixels, a block of partial chunks beyond."""
+    """One wave per frame up to 4,096 pixels, a block of partial chunks beyond."""
     test_frame_sums_bit_exact(ctx, dev, npix)
 
 
-@pytest.mark.parametrize("rows,cols", [(8, 16), (32, 64), (33, 63), (40, 60)])
+@pytest.mark.parametrize("rows,cols", [(8, 16), (32, 64), (33, 63), (80, 60)])
 def test_photon_counts_of_corrected_frames(ctx, dev, rows, cols):
     """Gain-corrected frames, whose sums are no whole numbers: short frames and longer ones."""
     import torch
