@@ -179,7 +179,9 @@ int iac_ac3d_records_batch(iac_ctx *ctx, const float *d_kmap, uint32_t npix, con
  * sequence into a HIP graph for (d_mesh, zero_mesh); later launches with the same pair
  * replay the graph.  d_kmap / d_pix / d_cnt / d_frame_off are kept by pointer and must
  * outlive the batch; the photon lists may change between launches with the frame count
- * and n_total unchanged.  zero_mesh
+ * and n_total unchanged.  The batch holds 32 bytes per photon (gathered and sorted records),
+ * 16 more where strips may take it (their sort beside the walk's, chosen per launch), and
+ * its half mesh, for its life.  zero_mesh
  * clears d_mesh first (by kernel).  No counterpart in the reference: it is the
  * frame loop of IAC/RunIAC.cpp:524-550 as one replayable unit. */
 typedef struct iac_ac3d_batch iac_ac3d_batch;

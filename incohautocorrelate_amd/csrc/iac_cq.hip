@@ -2,9 +2,10 @@
 // the final AC/C(q) division, on gfx950.
 //
 //   iac_cq_small / iac_cq_dense_frames: AutoCorr_CQ_small (IAC/kernel.cl:27-184)
-//     through the LDS cell-box pair engine (one record per pixel).
-//   iac_merge_cq: Merge_CQ (IAC/kernel.cl:189-344), one thread per small-mesh
-//     voxel and event slice.
+//     by region tiles where they suit the images, else through the LDS cell-box pair
+//     engine's walk (one record per pixel).
+//   iac_merge_cq: Merge_CQ (IAC/kernel.cl:189-344), bricks of the big mesh in LDS, or
+//     scattered adds where the updates are few.
 //   iac_merge_ac_cq: RunIAC::Merge_ACandCQ (IAC/RunIAC.cpp:120-158).
 #include <algorithm>
 #include <cmath>
